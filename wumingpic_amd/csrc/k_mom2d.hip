@@ -32,15 +32,6 @@ struct MomArgs {
   double fac1[WPIC_MAXSP], txxx[WPIC_MAXSP], fac2[WPIC_MAXSP];  // mom_calc.f90:90-92 with delt/2
 };
 
-// stage the tile's cell-centred fields plus a one-cell halo (mom_calc.f90:68-81)
-__device__ inline void stage_fields(const Grid2D& g, const double* uf, double (*sf)[SFW * SFH], int i0, int j0) {
-  for (int k = threadIdx.x; k < 6 * SFW * SFH; k += NT) {
-    const int c = k / (SFW * SFH), rem = k - c * (SFW * SFH);
-    const int i = i0 - 1 + rem % SFW, j = j0 - 1 + rem / SFW;
-    if (i <= g.nxge + 1 && j <= g.nye + 1) sf[c][rem] = cell_field(g, uf, c, i, j);
-  }
-}
-
 // the seven moments of one particle times the CIC weight wx*wy, in the
 // reference's product order (mom_calc.f90:203-243)
 struct MomTerms {
@@ -63,7 +54,7 @@ struct MomTerms {
 // (mom_calc.f90:131-155); gp is slot-aligned with up, the id travels along.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(NT) void k_mom_accl(MomArgs a) {
-  __shared__ double sf[6][SFW * SFH];
+  __shared__ FieldTile sf;
   const Grid2D& g = a.g;
   const int ntiles = a.ntx * a.nty;
   const int tile = xcd_tile(blockIdx.x, ntiles);
@@ -88,7 +79,7 @@ __global__ __launch_bounds__(NT) void k_mom_accl(MomArgs a) {
         const int ia = a.ap ? a.ap[pi] : pi;
         const double x = a.A.x[ia], y = a.A.y[ia];
         double nxp, nyp, g3, g4, g5, gmv;
-        boris_push(sf, li, lj, i, j, g.d_delx, hdelt, g.c, true, a.fac1[s], a.txxx[s], a.fac2[s], x, y, a.A.ux[ia],
+        boris_push(sf, li, lj, i, j, hdelt, g.c, true, a.fac1[s], a.txxx[s], a.fac2[s], x, y, a.A.ux[ia],
                    a.A.uy[ia], a.A.uz[ia], nxp, nyp, g3, g4, g5, gmv);
         a.B.x[pi] = x;
         a.B.y[pi] = y;
@@ -130,7 +121,7 @@ __device__ inline void rotate7(double (&m)[7], int r) {
 template <bool KICK>
 __global__ __launch_bounds__(NT) void k_mom_tile(MomArgs a) {
   constexpr int G = MOM_G, NGRP = NT / G;  // lanes per cell, cells in flight
-  __shared__ double sf[KICK ? 6 : 1][SFW * SFH];
+  __shared__ FieldPair sf[KICK ? 3 : 1][SFW * SFH];
   __shared__ double mt[7][MTW * MTH];
   const Grid2D& g = a.g;
   const int ntiles = a.ntx * a.nty;
@@ -168,7 +159,7 @@ __global__ __launch_bounds__(NT) void k_mom_tile(MomArgs a) {
           x = a.A.x[ia];
           y = a.A.y[ia];
           double nxp, nyp, gmv;
-          boris_push(sf, li, lj, i, j, d_delx, hdelt, c, true, a.fac1[s], a.txxx[s], a.fac2[s], x, y, a.A.ux[ia],
+          boris_push(sf, li, lj, i, j, hdelt, c, true, a.fac1[s], a.txxx[s], a.fac2[s], x, y, a.A.ux[ia],
                      a.A.uy[ia], a.A.uz[ia], nxp, nyp, ux, uy, uz, gmv);
         } else {
           x = a.B.x[pi];

@@ -26,24 +26,68 @@ __device__ inline double cell_field(const Grid2D& g, const double* uf, int c, in
   }
 }
 
+// The staged cell-centred fields: pairs (Bx, By), (Bz, Ex), (Ey, Ez) of a cell
+// side by side, so that one 16-byte LDS read brings two components and every
+// read of the gather is an immediate offset from one address.
+struct alignas(16) FieldPair {
+  double a, b;
+};
+using FieldTile = FieldPair[3][SFW * SFH];
+
+__device__ inline void stage_fields(const Grid2D& g, const double* uf, FieldPair (*sf)[SFW * SFH], int i0, int j0) {
+  for (int k = threadIdx.x; k < 6 * SFW * SFH; k += NT) {
+    const int c = k / (SFW * SFH), rem = k - c * (SFW * SFH);
+    const int i = i0 - 1 + rem % SFW, j = j0 - 1 + rem / SFW;
+    if (i <= g.nxge + 1 && j <= g.nye + 1) {
+      const double v = cell_field(g, uf, c, i, j);
+      FieldPair& p = sf[c >> 1][rem];
+      if (c & 1)
+        p.b = v;
+      else
+        p.a = v;
+    }
+  }
+}
+
 // The six fields at a particle of cell (i, j) with the second-order shape
-// (particle.f90:96-133), from the tile's staged cell-centred values.
-__device__ inline void gather6(const double (*sf)[SFW * SFH], int li, int lj, int i, int j, double d_delx, double x,
-                               double y, double* fl) {
-  double sx0, sx1, sx2, sy0, sy1, sy2;
-  shape3(x * d_delx - 0.5 - i, sx0, sx1, sx2);
-  shape3(y * d_delx - 0.5 - j, sy0, sy1, sy2);
-  // re-read the cell's staged fields from LDS for every particle (the group's
-  // lanes read the same words: a broadcast) instead of holding all 54 in
-  // registers across the particle loop
-  int soff = (lj + 1) * SFW + (li + 1);
+// (particle.f90:96-133), from the tile's staged cell-centred values.  delx is
+// 1, the only cell width a context accepts: x * d_delx is x.
+//
+// Every particle re-reads the cell's staged fields (the group's lanes read the
+// same words: a broadcast) instead of holding all 54 in registers across the
+// particle loop.  The compiler, left alone, waits for each LDS read right
+// after issuing it (about 30 round trips a particle); here the nine reads of
+// the next pair are in flight while the current pair is combined.
+__device__ inline void gather6(const FieldPair (*sf)[SFW * SFH], int li, int lj, int i, int j, double x, double y,
+                               double* fl) {
+  int soff = lj * SFW + li;  // the cell's lower left neighbour
   asm volatile("" : "+v"(soff));
+  FieldPair v[2][9];
+  auto load = [&](int p) {
+    const FieldPair* f = &sf[p][soff];
+    FieldPair* d = v[p & 1];
 #pragma unroll
-  for (int cmp = 0; cmp < 6; cmp++) {
-    const double* f = &sf[cmp][soff];
-    fl[cmp] = +(+f[-SFW - 1] * sx0 + f[-SFW] * sx1 + f[-SFW + 1] * sx2) * sy0 +
-              (+f[-1] * sx0 + f[0] * sx1 + f[1] * sx2) * sy1 +
-              (+f[SFW - 1] * sx0 + f[SFW] * sx1 + f[SFW + 1] * sx2) * sy2;
+    for (int r = 0; r < 3; r++)
+#pragma unroll
+      for (int k = 0; k < 3; k++) d[3 * r + k] = f[r * SFW + k];
+  };
+  load(0);
+  __builtin_amdgcn_sched_barrier(0);
+  double sx0, sx1, sx2, sy0, sy1, sy2;
+  shape3(x - 0.5 - i, sx0, sx1, sx2);
+  shape3(y - 0.5 - j, sy0, sy1, sy2);
+#pragma unroll
+  for (int p = 0; p < 3; p++) {
+    if (p < 2) load(p + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    const FieldPair* f = v[p & 1];
+    fl[2 * p] = +(+f[0].a * sx0 + f[1].a * sx1 + f[2].a * sx2) * sy0 +
+                (+f[3].a * sx0 + f[4].a * sx1 + f[5].a * sx2) * sy1 +
+                (+f[6].a * sx0 + f[7].a * sx1 + f[8].a * sx2) * sy2;
+    fl[2 * p + 1] = +(+f[0].b * sx0 + f[1].b * sx1 + f[2].b * sx2) * sy0 +
+                    (+f[3].b * sx0 + f[4].b * sx1 + f[5].b * sx2) * sy1 +
+                    (+f[6].b * sx0 + f[7].b * sx1 + f[8].b * sx2) * sy2;
+    __builtin_amdgcn_sched_barrier(0);
   }
 }
 
@@ -51,12 +95,10 @@ __device__ inline void gather6(const double (*sf)[SFW * SFH], int li, int lj, in
 // fields gathered from the tile's staged cell-centred values.  Shared by the
 // parity and fast kernels, so both produce bit-identical gp.  gmv returns the
 // 1/gamma of the move.
-__device__ inline void boris_push(const double (*sf)[SFW * SFH], int li, int lj, int i, int j, double d_delx,
-                                  double delt, double c, bool unit_c, double fac1, double txxx, double fac2,
-                                  double x, double y, double ux, double uy, double uz, double& nxp, double& nyp,
+__device__ inline void boris_push(const FieldPair (*sf)[SFW * SFH], int li, int lj, int i, int j, double delt, double c, bool unit_c, double fac1, double txxx, double fac2, double x, double y, double ux, double uy, double uz, double& nxp, double& nyp,
                                   double& g3, double& g4, double& g5, double& gmv) {
   double fl[6];
-  gather6(sf, li, lj, i, j, d_delx, x, y, fl);
+  gather6(sf, li, lj, i, j, x, y, fl);
   const double bpx = fl[0], bpy = fl[1], bpz = fl[2], epx = fl[3], epy = fl[4], epz = fl[5];
   double uvm1 = ux + fac1 * epx;
   double uvm2 = uy + fac1 * epy;
@@ -85,12 +127,11 @@ __device__ inline void boris_push(const double (*sf)[SFW * SFH], int li, int lj,
 // gather, u' = u + fac2 E + (fac1/gam) u x B, tau = fac1 B / c, the new gamma
 // from sigma and u'.tau, then the implicit rotation; the move uses that gamma.
 // Same arguments as boris_push (txxx unused).
-__device__ inline void vay_push(const double (*sf)[SFW * SFH], int li, int lj, int i, int j, double d_delx,
-                                double delt, double c, double fac1, double fac2, double x, double y, double ux,
+__device__ inline void vay_push(const FieldPair (*sf)[SFW * SFH], int li, int lj, int i, int j, double delt, double c, double fac1, double fac2, double x, double y, double ux,
                                 double uy, double uz, double& nxp, double& nyp, double& g3, double& g4, double& g5,
                                 double& gmv) {
   double fl[6];
-  gather6(sf, li, lj, i, j, d_delx, x, y, fl);
+  gather6(sf, li, lj, i, j, x, y, fl);
   const double bpx = fl[0], bpy = fl[1], bpz = fl[2], epx = fl[3], epy = fl[4], epz = fl[5];
   double gam = sqrt(c * c + ux * ux + uy * uy + uz * uz);
   const double fac1r = fac1 / gam;

@@ -47,18 +47,17 @@ constexpr int NPJ = 65;
 // position relative to cell (i, j), ds = (shifted new shape) - s0
 __device__ inline void esirkepov_shapes(const Grid2D& g, double x, double y, double nxp, double nyp, int i, int j,
                                         double s0x[5], double s0y[5], double dsx[5], double dsy[5]) {
-  const double d_delx = g.d_delx;
   double t0, t1, t2;
-  shape3(x * d_delx - 0.5 - i, t0, t1, t2);
+  shape3(x - 0.5 - i, t0, t1, t2);
   s0x[0] = 0.0; s0x[1] = t0; s0x[2] = t1; s0x[3] = t2; s0x[4] = 0.0;
-  shape3(y * d_delx - 0.5 - j, t0, t1, t2);
+  shape3(y - 0.5 - j, t0, t1, t2);
   s0y[0] = 0.0; s0y[1] = t0; s0y[2] = t1; s0y[3] = t2; s0y[4] = 0.0;
 #pragma unroll
   for (int d = 0; d < 2; d++) {
     const double gp = d == 0 ? nxp : nyp;
     const int cell = d == 0 ? i : j;
-    const int i2 = (int)(gp * d_delx);
-    const double dh = gp * d_delx - 0.5 - i2;
+    const int i2 = (int)gp;
+    const double dh = gp - 0.5 - i2;
     const int inc = i2 - cell;
     const double s1_1 = 0.5 * (0.5 - dh) * (0.5 - dh);
     const double s1_2 = 0.75 - dh * dh;
@@ -85,14 +84,14 @@ __device__ inline void esirkepov_shapes(const Grid2D& g, double x, double y, dou
 // (0, 1, 0), so ds(-2) = ds(2) = 0 and ds(k) = s1(k) - s0(k) for k = -1..1,
 // the values esirkepov_shapes gives there (x * 1 and + 0 are exact), with
 // three of its ten live at a time
-__device__ inline void stayer_shapes(double d_delx, double x, double y, double nxp, double nyp, int i, int j,
+__device__ inline void stayer_shapes(double x, double y, double nxp, double nyp, int i, int j,
                                      double s0x[3], double s0y[3], double dsx[3], double dsy[3]) {
-  shape3(x * d_delx - 0.5 - i, s0x[0], s0x[1], s0x[2]);
-  shape3(y * d_delx - 0.5 - j, s0y[0], s0y[1], s0y[2]);
+  shape3(x - 0.5 - i, s0x[0], s0x[1], s0x[2]);
+  shape3(y - 0.5 - j, s0y[0], s0y[1], s0y[2]);
   double t0, t1, t2;
-  shape3(nxp * d_delx - 0.5 - i, t0, t1, t2);
+  shape3(nxp - 0.5 - i, t0, t1, t2);
   dsx[0] = t0 - s0x[0]; dsx[1] = t1 - s0x[1]; dsx[2] = t2 - s0x[2];
-  shape3(nyp * d_delx - 0.5 - j, t0, t1, t2);
+  shape3(nyp - 0.5 - j, t0, t1, t2);
   dsy[0] = t0 - s0y[0]; dsy[1] = t1 - s0y[1]; dsy[2] = t2 - s0y[2];
 }
 
@@ -137,13 +136,13 @@ __device__ inline void flush_block(double (&v)[N], double* pjbuf, double (*acc)[
 template <int BC>
 __device__ inline int wrap_code(const Grid2D& g, double& nxp, double& nyp, int j, int* err) {
   if (BC == WPIC_BC_PERIODIC) {
-    const int ipos = cell_rd(nxp, g.delx);
+    const int ipos = cell_of(nxp);
     if (ipos < g.nxgs)
       nxp = rd_add(nxp, g.spanx);
     else if (ipos >= g.nxge + 1)
       nxp = rd_add(nxp, -g.spanx);
   }
-  const int jpos = cell_rd(nyp, g.delx);
+  const int jpos = cell_of(nyp);
   if (jpos != j) {
     if (jpos <= g.nygs - 1)
       nyp = rd_add(nyp, g.spany);
@@ -246,7 +245,7 @@ __device__ inline void deposit_pass(const PushArgs& a, double (*acc)[ACW * ACH],
 //   slot order, so G = 1 reproduces the reference's sums.
 template <int G, bool PUSH, bool DEPOSIT, bool FUSED, bool PARITY, int BC>
 __global__ __launch_bounds__(NT) void k_push_deposit(PushArgs a) {
-  __shared__ double sf[6][SFW * SFH];
+  __shared__ FieldTile sf;
   __shared__ double acc[(DEPOSIT && !PARITY) ? 3 : 1][ACW * ACH];
 
   const Grid2D& g = a.g;
@@ -257,13 +256,7 @@ __global__ __launch_bounds__(NT) void k_push_deposit(PushArgs a) {
   const int j0 = g.nys + (tile / a.ntx) * TY;
   const int tid = threadIdx.x;
 
-  if (PUSH) {
-    for (int k = tid; k < 6 * SFW * SFH; k += NT) {
-      const int c = k / (SFW * SFH), rem = k - c * (SFW * SFH);
-      const int i = i0 - 1 + rem % SFW, j = j0 - 1 + rem / SFW;
-      if (i <= g.nxge + 1 && j <= g.nye + 1) sf[c][rem] = cell_field(g, a.uf, c, i, j);
-    }
-  }
+  if (PUSH) stage_fields(g, a.uf, sf, i0, j0);
   if (DEPOSIT && !PARITY) {
     for (int k = tid; k < 3 * ACW * ACH; k += NT) (&acc[0][0])[k] = 0.0;
   }
@@ -271,7 +264,7 @@ __global__ __launch_bounds__(NT) void k_push_deposit(PushArgs a) {
 
   const int grp = tid / G, lg = tid % G;
   constexpr int NGRP = NT / G;
-  const double d_delx = g.d_delx, delt = g.delt, c = g.c;
+  const double delt = g.delt, c = g.c;
   const double cc2 = c * c;
   const bool unit_c = cc2 == 1.0;  // x/(c*c) == x exactly: skip the division
   const double fac = 1.0 / 3.0;
@@ -299,10 +292,10 @@ __global__ __launch_bounds__(NT) void k_push_deposit(PushArgs a) {
         if (PUSH) {
           double gmv;
           if (a.vay)
-            vay_push(sf, li, lj, i, j, d_delx, delt, c, fac1, fac2, x, y, a.A.ux[ia], a.A.uy[ia], a.A.uz[ia], nxp,
+            vay_push(sf, li, lj, i, j, delt, c, fac1, fac2, x, y, a.A.ux[ia], a.A.uy[ia], a.A.uz[ia], nxp,
                      nyp, g3, g4, g5, gmv);
           else
-            boris_push(sf, li, lj, i, j, d_delx, delt, c, unit_c, fac1, txxx, fac2, x, y, a.A.ux[ia], a.A.uy[ia],
+            boris_push(sf, li, lj, i, j, delt, c, unit_c, fac1, txxx, fac2, x, y, a.A.ux[ia], a.A.uy[ia],
                        a.A.uz[ia], nxp, nyp, g3, g4, g5, gmv);
         } else {
           nxp = a.B.x[pi];
@@ -381,13 +374,13 @@ __device__ inline void deposit2_full(double (*acc)[ACW * ACH], int li, int lj, c
 // reflection that precedes the deposit in the reconnection order
 // (2d/proj/reconnection/app.f90:101-103; boundary_reconnection.f90:79-91).
 template <int BC, bool VAY>
-__device__ inline void push_reflect(const Grid2D& g, const double (*sf)[SFW * SFH], int li, int lj, int i, int j,
+__device__ inline void push_reflect(const Grid2D& g, const FieldPair (*sf)[SFW * SFH], int li, int lj, int i, int j,
                                     bool unit_c, const double* kc, double x, double y, double ux, double uy, double uz,
                                     double& nxp, double& nyp, double& g3, double& g4, double& g5, double& gmv) {
   if (VAY)
-    vay_push(sf, li, lj, i, j, g.d_delx, g.delt, g.c, kc[0], kc[2], x, y, ux, uy, uz, nxp, nyp, g3, g4, g5, gmv);
+    vay_push(sf, li, lj, i, j, g.delt, g.c, kc[0], kc[2], x, y, ux, uy, uz, nxp, nyp, g3, g4, g5, gmv);
   else
-    boris_push(sf, li, lj, i, j, g.d_delx, g.delt, g.c, unit_c, kc[0], kc[1], kc[2], x, y, ux, uy, uz, nxp, nyp, g3,
+    boris_push(sf, li, lj, i, j, g.delt, g.c, unit_c, kc[0], kc[1], kc[2], x, y, ux, uy, uz, nxp, nyp, g3,
                g4, g5, gmv);
   reflect_x<BC>(g, nxp, g3, g4, g5);
   // the injection edge sends ux to 2 u0 - ux, which changes gamma: vz of the
@@ -433,7 +426,7 @@ template <int G, bool FUSED, int BC, bool VAY>
 __global__ __launch_bounds__(NT, 2) void k_push_deposit_fast(PushArgs a) {
   constexpr int NW = NT / 64;
   static_assert(NW == TY && 64 / G * (TX / (64 / G)) == TX, "one wave per tile row, whole rounds");
-  __shared__ double sf[6][SFW * SFH];
+  __shared__ FieldTile sf;
   __shared__ double acc[3][ACW * ACH];
   __shared__ double spc[WPIC_MAXSP][5];  // fac1, txxx, fac2, qk, q
   __shared__ double xqd[NW][QW][5];      // x, y, unwrapped new x, y, q vz
@@ -448,11 +441,7 @@ __global__ __launch_bounds__(NT, 2) void k_push_deposit_fast(PushArgs a) {
   const int j0 = g.nys + (tile / a.ntx) * TY;
   const int tid = threadIdx.x;
 
-  for (int k = tid; k < 6 * SFW * SFH; k += NT) {
-    const int c = k / (SFW * SFH), rem = k - c * (SFW * SFH);
-    const int i = i0 - 1 + rem % SFW, j = j0 - 1 + rem / SFW;
-    if (i <= g.nxge + 1 && j <= g.nye + 1) sf[c][rem] = cell_field(g, a.uf, c, i, j);
-  }
+  stage_fields(g, a.uf, sf, i0, j0);
   for (int k = tid; k < 3 * ACW * ACH; k += NT) (&acc[0][0])[k] = 0.0;
   if (tid < NW) nxq[tid] = 0;
   // per-species constants (particle.f90:92-94, field.f90:274)
@@ -553,11 +542,11 @@ __global__ __launch_bounds__(NT, 2) void k_push_deposit_fast(PushArgs a) {
       a.B.id[pi] = id;  // particle.f90:173-177
 
       const double qvz = kc[4] * (g5 * gmv);
-      const int i2 = (int)(nxp * g.d_delx), j2 = (int)(nyp * g.d_delx);
+      const int i2 = (int)nxp, j2 = (int)nyp;
       if (i2 == i && j2 == j) {
         const double qk = kc[3];
         double s0x[3], s0y[3], dsx[3], dsy[3];
-        stayer_shapes(g.d_delx, x, y, nxp, nyp, i, j, s0x, s0y, dsx, dsy);
+        stayer_shapes(x, y, nxp, nyp, i, j, s0x, s0y, dsx, dsy);
         const double cx1 = 0.0 - dsx[0], cx2 = cx1 - dsx[1];
         const double cy1 = 0.0 - dsy[0], cy2 = cy1 - dsy[1];
 #pragma unroll

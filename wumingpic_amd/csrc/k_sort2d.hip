@@ -53,7 +53,7 @@ __global__ __launch_bounds__(SB) void k_wrapx(SortArgs a, int inj) {
       a.B.uy[p] = uy;
       a.B.uz[p] = uz;
     } else {
-      const int ipos = cell_rd(x, g.delx);
+      const int ipos = cell_of(x);
       if (ipos < g.nxgs)
         a.B.x[p] = rd_add(x, g.spanx);
       else if (ipos >= g.nxge + 1)
@@ -82,7 +82,7 @@ __global__ __launch_bounds__(SB) void k_rowscan(SortArgs a) {
       const int p = base + k;
       if (YWRAP) {
         double y = a.B.y[p];
-        const int jpos = cell_rd(y, g.delx);
+        const int jpos = cell_of(y);
         if (jpos != j) {
           if (jpos <= g.nygs - 1)
             a.B.y[p] = rd_add(y, g.spany);

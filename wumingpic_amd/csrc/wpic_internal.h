@@ -113,19 +113,11 @@ __host__ __device__ inline double rd_mul(double a, double b) {
   return p;
 }
 
-__host__ __device__ inline double rd_div(double a, double b) {
-  double q = a / b;
-  double r = __builtin_fma(-q, b, a);
-  if ((r < 0.0 && b > 0.0) || (r > 0.0 && b < 0.0)) q = next_down(q);
-  return q;
-}
-
 // int(x / delx) of the particle boundaries, under round-down
 // (boundary_periodic.f90:74) or round-to-nearest: with delx = 1, the only
 // cell width a context accepts (sort__bucket bins by int(x)), the quotient is
 // x itself in every rounding mode
-__host__ __device__ inline int cell_rd(double x, double delx) { return (int)(delx == 1.0 ? x : rd_div(x, delx)); }
-__host__ __device__ inline int cell_rn(double x, double delx) { return (int)(delx == 1.0 ? x : x / delx); }
+__host__ __device__ inline int cell_of(double x) { return (int)x; }
 
 // The x boundary that acts on a pushed particle before the deposit:
 // reconnection walls (boundary_reconnection.f90:79-91, WPIC_BC_WALLX) or the
@@ -135,7 +127,7 @@ __host__ __device__ inline int cell_rn(double x, double delx) { return (int)(del
 template <int BC, bool INJ = true>
 __host__ __device__ inline void reflect_x(const Grid2D& g, double& x, double& ux, double& uy, double& uz) {
   if (BC == WPIC_BC_PERIODIC) return;
-  const int ipos = cell_rn(x, g.delx);
+  const int ipos = cell_of(x);
   if (ipos < g.nxgs + 1) {
     x = g.wall_lo - x;
     ux = -ux; uy = -uy; uz = -uz;
