@@ -406,8 +406,8 @@ __global__ void k_adj_seed(Grid2D g, const double* uf, double* lamF, double seed
 // per-block partial sums of dL/d(udrift), dL/d(uth_e), dL/d(amp) from the
 // initial state (electrons = the last species; the beam sign alternates by
 // in-cell slot as the seeded state assigns it)
-__global__ __launch_bounds__(256) void k_adj_params(Grid2D g, Parts P, const uint64_t* id, const int* rowbase,
-                                                    const int* np2, const double* lamA, size_t N, const double* lamF,
+__global__ __launch_bounds__(256) void k_adj_params(Grid2D g, Parts P, const int* rowbase, const int* np2,
+                                                    const double* lamA, size_t N, const double* lamF,
                                                     double udrift, double uth_e, int mode, int n_ppc, double* out) {
   __shared__ double sh[3][256];
   double sd = 0.0, st = 0.0, sa = 0.0;
@@ -417,7 +417,7 @@ __global__ __launch_bounds__(256) void k_adj_params(Grid2D g, Parts P, const uin
     const int base = rowbase[rw], n = np2[rw];
     for (int k = threadIdx.x; k < n; k += 256) {
       const int p = base + k;
-      const long long pid = -(long long)id[p];
+      const long long pid = -(long long)P.id[p];
       const long long sl = (pid - 1) % n_ppc;
       const double sgn = (sl & 1) ? -1.0 : 1.0;
       const double lx = lamA[2 * N + p], ly = lamA[3 * N + p], lz = lamA[4 * N + p];
@@ -515,11 +515,11 @@ hipError_t launch_adj_seed(wpic_ctx* c, double* lamF, double seed) {
   return hipGetLastError();
 }
 
-hipError_t launch_adj_params(wpic_ctx* c, const Parts& P, const uint64_t* id, const int* rows, const double* lamA,
-                             size_t N, const double* lamF, double udrift, double uth_e, int mode, int n_ppc,
+hipError_t launch_adj_params(wpic_ctx* c, const Parts& P, const int* rows, const double* lamA, size_t N,
+                             const double* lamF, double udrift, double uth_e, int mode, int n_ppc,
                              double* out) {
   const int nr = c->g.nsp * c->g.ny;
-  hipLaunchKernelGGL(k_adj_params, dim3(256), dim3(256), 0, c->st, c->g, P, id, rows, rows + nr, lamA, N, lamF,
+  hipLaunchKernelGGL(k_adj_params, dim3(256), dim3(256), 0, c->st, c->g, P, rows, rows + nr, lamA, N, lamF,
                      udrift, uth_e, mode, n_ppc, out);
   return hipGetLastError();
 }

@@ -1,13 +1,14 @@
-// k_misc2d.hip -- layout conversion at the boundary (reference AoS <-> device
-// SoA), the seeded initial state, and diagnostics (energy sums, Gauss law).
+// k_misc2d.hip -- transfers at the boundary (the reference's padded rows <->
+// packed device records, field AoS <-> planes), the seeded initial state, and diagnostics (energy sums, Gauss law).
 #include "wpic_internal.h"
 
 namespace wpic {
 
 // ---------------------------------------------------------------------------
-// particles: compact AoS rows (ndim = 6 doubles per particle, the reference's
-// up(:, ii, j, isp) contiguous) <-> SoA, over all rows of A (which = 0) or B
-// (which = 1).  The AoS buffer holds species after species, rows in order.
+// particles: compact rows (ndim = 6 doubles per particle, the reference's
+// up(:, ii, j, isp) contiguous) <-> the device's records, over all rows of A
+// (which = 0) or B (which = 1).  The host's buffer holds species after
+// species, rows in order.
 // ---------------------------------------------------------------------------
 struct XferArgs {
   Grid2D g;
@@ -17,39 +18,25 @@ struct XferArgs {
   const long long* aosbase;  // [nsp*ny] start of each row in the AoS buffer
 };
 
-__global__ void k_aos_to_soa(XferArgs a, const double* __restrict__ aos) {
+// (raw 64-bit words: a record is the reference's own six)
+__global__ void k_records_in(XferArgs a, const uint64_t* __restrict__ aos) {
   const int rw = blockIdx.x;
   const int base = a.rowbase[rw], n = a.np2[rw];
-  const double* src = aos + a.aosbase[rw] * 6;
-  for (int k = threadIdx.x; k < n; k += blockDim.x) {
-    const double* s = src + (size_t)k * 6;
-    const int d = base + k;
-    a.P.x[d] = s[0];
-    a.P.y[d] = s[1];
-    a.P.ux[d] = s[2];
-    a.P.uy[d] = s[3];
-    a.P.uz[d] = s[4];
-    uint64_t b;
-    __builtin_memcpy(&b, &s[5], 8);
-    a.P.id[d] = b;
-  }
+  const uint64_t* src = aos + a.aosbase[rw] * PART_DOUBLES;
+  uint64_t* dst = reinterpret_cast<uint64_t*>(a.P.x.p) + (size_t)base * PART_DOUBLES;
+  for (int k = threadIdx.x; k < n * PART_DOUBLES; k += blockDim.x) dst[k] = src[k];
 }
 
-__global__ void k_soa_to_aos(XferArgs a, double* __restrict__ aos) {
+__global__ void k_records_out(XferArgs a, uint64_t* __restrict__ aos) {
   const int rw = blockIdx.x;
   const int base = a.rowbase[rw], n = a.np2[rw];
-  double* dst = aos + a.aosbase[rw] * 6;
+  const uint64_t* src = reinterpret_cast<const uint64_t*>(a.P.x.p);
+  uint64_t* dst = aos + a.aosbase[rw] * PART_DOUBLES;
   for (int k = threadIdx.x; k < n; k += blockDim.x) {
     int s = a.R ? a.R[base + k] : base + k;
     if ((unsigned)s >= (unsigned)(a.g.ncap * a.g.nsp)) s = 0;
-    double* d = dst + (size_t)k * 6;
-    d[0] = a.P.x[s];
-    d[1] = a.P.y[s];
-    d[2] = a.P.ux[s];
-    d[3] = a.P.uy[s];
-    d[4] = a.P.uz[s];
-    const uint64_t b = a.P.id[s];
-    __builtin_memcpy(&d[5], &b, 8);
+#pragma unroll
+    for (int q = 0; q < PART_DOUBLES; q++) dst[(size_t)k * PART_DOUBLES + q] = src[(size_t)s * PART_DOUBLES + q];
   }
 }
 
@@ -89,7 +76,8 @@ hipError_t launch_up_to_soa(wpic_ctx* c, const double* aos, long long n, int whi
   a.np2 = which == 0 ? c->np2A : c->np2B;
   a.R = nullptr;
   a.aosbase = c->aosbase;
-  hipLaunchKernelGGL(k_aos_to_soa, dim3(c->g.nsp * c->g.ny), dim3(256), 0, c->st, a, aos);
+  hipLaunchKernelGGL(k_records_in, dim3(c->g.nsp * c->g.ny), dim3(256), 0, c->st, a,
+                     reinterpret_cast<const uint64_t*>(aos));
   return hipGetLastError();
 }
 
@@ -111,7 +99,8 @@ hipError_t launch_soa_to_aos(wpic_ctx* c, double* aos, int which) {
     a.R = nullptr;
   }
   a.aosbase = c->aosbase;
-  hipLaunchKernelGGL(k_soa_to_aos, dim3(c->g.nsp * c->g.ny), dim3(256), 0, c->st, a, aos);
+  hipLaunchKernelGGL(k_records_out, dim3(c->g.nsp * c->g.ny), dim3(256), 0, c->st, a,
+                     reinterpret_cast<uint64_t*>(aos));
   return hipGetLastError();
 }
 
@@ -190,12 +179,7 @@ __global__ void k_gather_rows(Grid2D g, Parts src, const int* ap, Parts dst, con
   for (int k = threadIdx.x; k < n; k += blockDim.x) {
     const int d = base + k;
     const int s = ap ? ap[d] : d;
-    dst.x[d] = src.x[s];
-    dst.y[d] = src.y[s];
-    dst.ux[d] = src.ux[s];
-    dst.uy[d] = src.uy[s];
-    dst.uz[d] = src.uz[s];
-    if (dst.id) dst.id[d] = src.id[s];
+    store_rec(dst, d, load_rec(src, s));
   }
 }
 
@@ -233,7 +217,6 @@ struct IcArgs {
   Grid2D g;
   Parts A;
   PartsM M;
-  uint64_t* id;
   unsigned long long seed;
   int n_ppc;
   double udrift, uth_e, uth_i;
@@ -283,7 +266,10 @@ __global__ void k_ic_beams(IcArgs a) {
   }
   // id = -(pid), pid counted row by row from 1 (app.f90:455-470)
   const long long pid = k + 1;
-  a.id[d] = (uint64_t)(-pid);
+  if (MIXED)
+    a.M.id[d] = (uint64_t)(-pid);
+  else
+    a.A.id[d] = (uint64_t)(-pid);
 }
 
 static IcArgs ic_args(wpic_ctx* c, unsigned long long seed, int n_ppc, double udrift, double uth_e,
@@ -292,7 +278,6 @@ static IcArgs ic_args(wpic_ctx* c, unsigned long long seed, int n_ppc, double ud
   a.g = c->g;
   a.A = c->A;
   a.M = c->MA;
-  a.id = c->mixed ? c->MA.id : c->A.id;
   a.seed = seed;
   a.n_ppc = n_ppc;
   a.udrift = udrift;
@@ -589,12 +574,7 @@ __global__ __launch_bounds__(256) void k_inject(InjArgs a) {
   for (int k = threadIdx.x; k < n_old; k += 256) {
     const int ia = a.ap ? a.ap[bo + k] : bo + k;
     const int d = bn + k;
-    a.B.x[d] = a.A.x[ia];
-    a.B.y[d] = a.A.y[ia];
-    a.B.ux[d] = a.A.ux[ia];
-    a.B.uy[d] = a.A.uy[ia];
-    a.B.uz[d] = a.A.uz[ia];
-    a.B.id[d] = a.A.id[ia];
+    store_rec(a.B, d, load_rec(a.A, ia));
   }
   const double delx = g.delx, delt = g.delt, c = g.c;
   const int j = g.nys + r;

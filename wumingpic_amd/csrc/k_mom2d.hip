@@ -77,16 +77,11 @@ __global__ __launch_bounds__(NT) void k_mom_accl(MomArgs a) {
       const int pend = base + cr[i - g.nxgs + 1];
       for (int pi = base + cr[i - g.nxgs] + lg; pi < pend; pi += G) {
         const int ia = a.ap ? a.ap[pi] : pi;
-        const double x = a.A.x[ia], y = a.A.y[ia];
+        const Rec p = load_rec(a.A, ia);
         double nxp, nyp, g3, g4, g5, gmv;
-        boris_push(sf, li, lj, i, j, hdelt, g.c, true, a.fac1[s], a.txxx[s], a.fac2[s], x, y, a.A.ux[ia],
-                   a.A.uy[ia], a.A.uz[ia], nxp, nyp, g3, g4, g5, gmv);
-        a.B.x[pi] = x;
-        a.B.y[pi] = y;
-        a.B.ux[pi] = g3;
-        a.B.uy[pi] = g4;
-        a.B.uz[pi] = g5;
-        a.B.id[pi] = a.A.id[ia];
+        boris_push(sf, li, lj, i, j, hdelt, g.c, true, a.fac1[s], a.txxx[s], a.fac2[s], p.x, p.y, p.ux, p.uy, p.uz,
+                   nxp, nyp, g3, g4, g5, gmv);
+        store_rec(a.B, pi, Rec{p.x, p.y, g3, g4, g5, p.id});
       }
     }
   }

@@ -34,13 +34,17 @@ struct alignas(16) FieldPair {
 };
 using FieldTile = FieldPair[3][SFW * SFH];
 
-__device__ inline void stage_fields(const Grid2D& g, const double* uf, FieldPair (*sf)[SFW * SFH], int i0, int j0) {
-  for (int k = threadIdx.x; k < 6 * SFW * SFH; k += NT) {
-    const int c = k / (SFW * SFH), rem = k - c * (SFW * SFH);
-    const int i = i0 - 1 + rem % SFW, j = j0 - 1 + rem / SFW;
+// the fields of tw <= TX columns of cells and their halo
+__device__ inline void stage_fields(const Grid2D& g, const double* uf, FieldPair (*sf)[SFW * SFH], int i0, int j0,
+                                    int tw = TX) {
+  const int w = tw + 2, n = w * SFH;
+  for (int k = threadIdx.x; k < 6 * n; k += NT) {
+    const int c = k / n, rem = k - c * n;
+    const int r = rem / w, q = rem - r * w;
+    const int i = i0 - 1 + q, j = j0 - 1 + r;
     if (i <= g.nxge + 1 && j <= g.nye + 1) {
       const double v = cell_field(g, uf, c, i, j);
-      FieldPair& p = sf[c >> 1][rem];
+      FieldPair& p = sf[c >> 1][r * SFW + q];
       if (c & 1)
         p.b = v;
       else
@@ -91,6 +95,41 @@ __device__ inline void gather6(const FieldPair (*sf)[SFW * SFH], int li, int lj,
   }
 }
 
+// The correctly rounded square root of x and the correctly rounded reciprocal
+// of that root, as sqrt(x) and 1. / sqrt(x) give them.  The compiler's own
+// sequences scale against overflow and handle zeros and infinities, twice
+// over; for x within 2^-200 .. 2^200 none of that is needed and the
+// reciprocal starts from the root's own iterate instead of a new seed.
+//   y ~ 1/sqrt(x) from the hardware; g ~ sqrt(x) and h ~ 1/(2 sqrt(x)) refined
+//   together by Goldschmidt's iteration, then g corrected twice with the exact
+//   residual x - g g (a fused multiply-add), which rounds it correctly; the
+//   reciprocal of g from 2 h by one Newton step and one correction with the
+//   exact residual 1 - g r (P. Markstein, IBM J. Res. Dev. 34, 111 (1990)).
+__device__ inline void sqrt_and_inverse(double x, double& root, double& inv) {
+  const unsigned hi = (unsigned)__double2hiint(x);
+  if (__builtin_expect(hi - 0x33700000u >= 0x19000000u, 0)) {  // exponent outside [-200, 200), sign or NaN
+    root = sqrt(x);
+    inv = 1. / root;
+    return;
+  }
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  double e = fma(-h, g, 0.5);
+  g = fma(g, e, g);
+  h = fma(h, e, h);
+  e = fma(-g, g, x);
+  g = fma(e, h, g);
+  e = fma(-g, g, x);
+  g = fma(e, h, g);
+  double r = h + h;
+  e = fma(-g, r, 1.0);
+  r = fma(e, r, r);
+  e = fma(-g, r, 1.0);
+  r = fma(e, r, r);
+  root = g;
+  inv = r;
+}
+
 // Buneman-Boris push of one particle in cell (i, j) (particle.f90:98-163),
 // fields gathered from the tile's staged cell-centred values.  Shared by the
 // parity and fast kernels, so both produce bit-identical gp.  gmv returns the
@@ -103,8 +142,8 @@ __device__ inline void boris_push(const FieldPair (*sf)[SFW * SFH], int li, int 
   double uvm1 = ux + fac1 * epx;
   double uvm2 = uy + fac1 * epy;
   double uvm3 = uz + fac1 * epz;
-  double gam = sqrt(c * c + uvm1 * uvm1 + uvm2 * uvm2 + uvm3 * uvm3);
-  const double igam = 1. / gam;
+  double gam, igam;
+  sqrt_and_inverse(c * c + uvm1 * uvm1 + uvm2 * uvm2 + uvm3 * uvm3, gam, igam);
   const double fac1r = fac1 * igam;
   const double fac2r = fac2 / (gam + txxx * (bpx * bpx + bpy * bpy + bpz * bpz) * igam);
   const double uvm4 = uvm1 + fac1r * (+uvm2 * bpz - uvm3 * bpy);
@@ -117,7 +156,8 @@ __device__ inline void boris_push(const FieldPair (*sf)[SFW * SFH], int li, int 
   g4 = uvm2 + fac1 * epy;
   g5 = uvm3 + fac1 * epz;
   const double u2 = +g3 * g3 + g4 * g4 + g5 * g5;
-  gmv = 1.0 / sqrt(1.0 + (unit_c ? u2 : u2 / (c * c)));
+  double root;
+  sqrt_and_inverse(1.0 + (unit_c ? u2 : u2 / (c * c)), root, gmv);
   nxp = x + g3 * delt * gmv;
   nyp = y + g4 * delt * gmv;
 }

@@ -559,11 +559,11 @@ __global__ __launch_bounds__(p3::NT, 2) void k_push_deposit3d_fast(Push3Args a) 
     {
       int s_, p_, ia_n = 0;
       if (lg < ntot) {
-        cl.slot(lg, s_, p_);
+        cl.slot(g.nsp, lg, s_, p_);
         ia_n = a.ap ? a.ap[p_] : p_;
       }
       if (lg + GF < ntot) {
-        cl.slot(lg + GF, s_, p_);
+        cl.slot(g.nsp, lg + GF, s_, p_);
         ia_nn = a.ap ? a.ap[p_] : p_;
       }
       if (lg < ntot) {
@@ -574,7 +574,7 @@ __global__ __launch_bounds__(p3::NT, 2) void k_push_deposit3d_fast(Push3Args a) 
     }
     for (int t = lg; t < ntot; t += GF) {
       int sc, pc;
-      cl.slot(t, sc, pc);
+      cl.slot(g.nsp, t, sc, pc);
       const double x = px, y = py, z = pz, ux = pux, uy = puy, uz = puz;
       const uint64_t id = pid;
       if (t + GF < ntot) {
@@ -585,7 +585,7 @@ __global__ __launch_bounds__(p3::NT, 2) void k_push_deposit3d_fast(Push3Args a) 
       }
       if (t + 2 * GF < ntot) {
         int s_, p_;
-        cl.slot(t + 2 * GF, s_, p_);
+        cl.slot(g.nsp, t + 2 * GF, s_, p_);
         ia_nn = a.ap ? a.ap[p_] : p_;
       }
       const double* kc = spc[sc];

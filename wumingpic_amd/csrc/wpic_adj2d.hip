@@ -27,7 +27,6 @@ struct AdjState {
   int nr = 0, ncc = 0;
   size_t pl = 0, nc = 0;
   std::vector<double*> ck_part, ck_uf, ck_df;
-  std::vector<uint64_t*> ck_id;
   std::vector<int*> ck_rows, ck_cumcnt;
   std::vector<double*> st_part, st_uf;
   std::vector<int*> st_rows, st_perm;
@@ -48,7 +47,6 @@ void adj_free(wpic_ctx* c) {
   for (auto p : a->ck_part) fr(p);
   for (auto p : a->ck_uf) fr(p);
   for (auto p : a->ck_df) fr(p);
-  for (auto p : a->ck_id) fr(p);
   for (auto p : a->ck_rows) fr(p);
   for (auto p : a->ck_cumcnt) fr(p);
   for (auto p : a->st_part) fr(p);
@@ -72,22 +70,16 @@ hipError_t dal(T** p, size_t n) {
   return hipMalloc((void**)p, (n ? n : 1) * sizeof(T));
 }
 
-Parts parts_of(double* base, uint64_t* id, size_t N) {
-  return Parts{base, base + N, base + 2 * N, base + 3 * N, base + 4 * N, id};
-}
-
 int copy_d(wpic_ctx* c, void* dst, const void* src, size_t bytes) {
   HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, c->st));
   return 0;
 }
 
 // the sorted state (A, its ids, rows, cumcnt) and the field arrays
-int save_state(wpic_ctx* c, double* part, uint64_t* id, int* rows, int* cumcnt, double* uf, double* df) {
+int save_state(wpic_ctx* c, double* part, int* rows, int* cumcnt, double* uf, double* df) {
   AdjState& a = *c->adj;
-  const size_t N = a.N;
-  // the sorted particles and their ids in slot order (A is read through its
-  // permutation)
-  if (part) HIPCHK(launch_gather_rows(c, c->A, c->aperm, parts_of(part, id, N), c->rows[c->ra]));
+  // the sorted records in slot order (A is read through its permutation)
+  if (part) HIPCHK(launch_gather_rows(c, c->A, c->aperm, parts_at(part), c->rows[c->ra]));
   if (rows && copy_d(c, rows, c->rows[c->ra], sizeof(int) * 2 * a.nr)) return WPIC_EHIP;
   if (cumcnt && copy_d(c, cumcnt, c->cumcnt, sizeof(int) * a.ncc)) return WPIC_EHIP;
   if (uf && copy_d(c, uf, c->uf, sizeof(double) * 6 * a.pl)) return WPIC_EHIP;
@@ -97,12 +89,8 @@ int save_state(wpic_ctx* c, double* part, uint64_t* id, int* rows, int* cumcnt, 
 
 int restore_state(wpic_ctx* c, int s) {
   AdjState& a = *c->adj;
-  const size_t N = a.N;
-  double* dst[5] = {c->A.x, c->A.y, c->A.ux, c->A.uy, c->A.uz};
-  for (int k = 0; k < 5; k++)
-    if (copy_d(c, dst[k], a.ck_part[s] + k * N, sizeof(double) * N)) return WPIC_EHIP;
+  if (copy_d(c, c->A.x.p, a.ck_part[s], sizeof(double) * PART_DOUBLES * a.N)) return WPIC_EHIP;
   c->aperm = nullptr;
-  if (copy_d(c, c->A.id, a.ck_id[s], sizeof(uint64_t) * N)) return WPIC_EHIP;
   if (copy_d(c, c->rows[c->ra], a.ck_rows[s], sizeof(int) * 2 * a.nr)) return WPIC_EHIP;
   if (copy_d(c, c->cumcnt, a.ck_cumcnt[s], sizeof(int) * a.ncc)) return WPIC_EHIP;
   if (copy_d(c, c->uf, a.ck_uf[s], sizeof(double) * 6 * a.pl)) return WPIC_EHIP;
@@ -132,14 +120,12 @@ int alloc_adj(wpic_ctx* c, int nsteps, int every) {
   a.ck_part.assign(a.nseg, nullptr);
   a.ck_uf.assign(a.nseg, nullptr);
   a.ck_df.assign(a.nseg, nullptr);
-  a.ck_id.assign(a.nseg, nullptr);
   a.ck_rows.assign(a.nseg, nullptr);
   a.ck_cumcnt.assign(a.nseg, nullptr);
   for (int s = 0; s < a.nseg && e == hipSuccess; s++) {
-    e = dal(&a.ck_part[s], 5 * a.N);
+    e = dal(&a.ck_part[s], PART_DOUBLES * a.N);
     if (e == hipSuccess) e = dal(&a.ck_uf[s], 6 * a.pl);
     if (e == hipSuccess) e = dal(&a.ck_df[s], 6 * a.pl);
-    if (e == hipSuccess) e = dal(&a.ck_id[s], a.N);
     if (e == hipSuccess) e = dal(&a.ck_rows[s], (size_t)2 * a.nr);
     if (e == hipSuccess) e = dal(&a.ck_cumcnt[s], (size_t)a.ncc);
   }
@@ -149,7 +135,7 @@ int alloc_adj(wpic_ctx* c, int nsteps, int every) {
   a.st_perm.assign(K, nullptr);
   a.st_rows.assign(K + 1, nullptr);
   for (int t = 0; t < K && e == hipSuccess; t++) {
-    e = dal(&a.st_part[t], 5 * a.N);
+    e = dal(&a.st_part[t], PART_DOUBLES * a.N);
     if (e == hipSuccess) e = dal(&a.st_uf[t], 6 * a.pl);
     if (e == hipSuccess) e = dal(&a.st_perm[t], a.N);
   }
@@ -205,7 +191,7 @@ int wpic_adj_forward2d(wpic_ctx* c, int nsteps, int every, double* wb) {
   for (int it = 0; it < nsteps; it++) {
     if (it % every == 0) {
       const int s = it / every;
-      rc = save_state(c, a.ck_part[s], a.ck_id[s], a.ck_rows[s], a.ck_cumcnt[s], a.ck_uf[s], a.ck_df[s]);
+      rc = save_state(c, a.ck_part[s], a.ck_rows[s], a.ck_cumcnt[s], a.ck_uf[s], a.ck_df[s]);
       if (rc) return rc;
     }
     rc = step_once(c);
@@ -234,14 +220,14 @@ int wpic_adj_backward2d(wpic_ctx* c, double seed) {
     int rc = restore_state(c, s);
     if (rc) return rc;
     for (int t = 0; t < K; t++) {
-      rc = save_state(c, a.st_part[t], nullptr, a.st_rows[t], nullptr, a.st_uf[t], nullptr);
+      rc = save_state(c, a.st_part[t], a.st_rows[t], nullptr, a.st_uf[t], nullptr);
       if (rc) return rc;
       c->perm_out = a.st_perm[t];
       rc = step_once(c);
       c->perm_out = nullptr;
       if (rc) return rc;
     }
-    rc = save_state(c, nullptr, nullptr, a.st_rows[K], nullptr, nullptr, nullptr);
+    rc = save_state(c, nullptr, a.st_rows[K], nullptr, nullptr, nullptr);
     if (rc) return rc;
     for (int t = K - 1; t >= 0; t--) {
       HIPCHK(hipMemsetAsync(a.lamB, 0, sizeof(double) * 5 * N, c->st));
@@ -252,7 +238,7 @@ int wpic_adj_backward2d(wpic_ctx* c, double seed) {
       if (rc) return rc;
       HIPCHK(launch_adj_field2(c, a.lamF2, a.lamJ));
       HIPCHK(hipMemsetAsync(a.lamT, 0, sizeof(double) * 6 * a.nc, c->st));
-      HIPCHK(launch_adj_particles(c, parts_of(a.st_part[t], nullptr, N), a.st_rows[t], a.st_uf[t], a.lamB, a.lamJ, a.lamA2,
+      HIPCHK(launch_adj_particles(c, parts_at(a.st_part[t]), a.st_rows[t], a.st_uf[t], a.lamB, a.lamJ, a.lamA2,
                                   a.lamT, N));
       HIPCHK(launch_adj_t2f(c, a.lamT, a.lamF2));
       std::swap(a.lamF, a.lamF2);
@@ -274,7 +260,7 @@ int wpic_adj_param_grads2d(wpic_ctx* c, double udrift, double uth_e, int bz_mode
   const int n_ppc = rows[a.nr] / c->g.nx;
   if (n_ppc < 1 || rows[a.nr] != n_ppc * c->g.nx)
     return set_error(WPIC_EINVAL, "the recorded run did not start from a wpic_ic_beams2d state");
-  HIPCHK(launch_adj_params(c, parts_of(a.ck_part[0], a.ck_id[0], a.N), a.ck_id[0], a.ck_rows[0], a.lamA, a.N, a.lamF, udrift,
+  HIPCHK(launch_adj_params(c, parts_at(a.ck_part[0]), a.ck_rows[0], a.lamA, a.N, a.lamF, udrift,
                            uth_e, bz_mode, n_ppc, a.red));
   std::vector<double> h(256 * 3);
   HIPCHK(hipMemcpyAsync(h.data(), a.red, sizeof(double) * h.size(), hipMemcpyDeviceToHost, c->st));

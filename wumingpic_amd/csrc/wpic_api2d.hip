@@ -202,7 +202,9 @@ int field_after_deposit(wpic_ctx* c) {
   return 0;
 }
 
-int deposit(wpic_ctx* c, bool push, bool fused) {
+// the deposit, with the push, the boundaries and the exchange codes (push: the
+// fused step) or alone
+int deposit(wpic_ctx* c, bool push) {
   if (c->rcnt_fill) HIPCHK(hipMemsetAsync(c->rcnt, 0, sizeof(int) * (size_t)c->g.nsp * c->g.ny * c->g.nx, c->st));
   if (c->mixed) {
     HIPCHK(launch_zero(c, c->uj, (size_t)3 * c->g.fw * c->g.fh));
@@ -219,7 +221,7 @@ int deposit(wpic_ctx* c, bool push, bool fused) {
   }
   {
     Timed t(c, "push_deposit");
-    HIPCHK(launch_push_deposit(c, push, true, fused));
+    HIPCHK(launch_push_deposit(c, push, true));
   }
   if (parity) HIPCHK(launch_gather_pj(c));
   return 0;
@@ -287,7 +289,7 @@ int step_once(wpic_ctx* c) {
   // the mixed push counts each row's particles per x cell for the sort (in the
   // FP64 fast push the same counting costs more than the sort's counting pass)
   c->rcnt_fill = c->mixed;
-  int rc = deposit(c, true, true);
+  int rc = deposit(c, true);
   if (rc) {
     c->rcnt_fill = false;
     return rc;
@@ -410,18 +412,17 @@ int wpic_create2d(wpic_ctx** out, const wpic_params2d* p) {
   const size_t N = (size_t)g.ncap * g.nsp;
   const int nr = g.nsp * ny;
   const size_t pl = (size_t)g.fw * g.fh, nc = (size_t)nx * ny;
-  if (c->mixed) {
-    for (PartsM* m : {&c->MA, &c->MB}) {
-      if (e == hipSuccess) e = dalloc(&m->ix, N);
-      for (float** q : {&m->ox, &m->oy, &m->ux, &m->uy, &m->uz})
-        if (e == hipSuccess) e = dalloc(q, N);
+  for (int k = 0; k < 2; k++) {
+    if (c->mixed) {
+      float* r = nullptr;
+      if (e == hipSuccess) e = dalloc(&r, PARTM_FLOATS * N);
+      (k == 0 ? c->MA : c->MB) = partsm_at(r);
+    } else {
+      double* r = nullptr;
+      if (e == hipSuccess) e = dalloc(&r, PART_DOUBLES * N);
+      (k == 0 ? c->A : c->B) = parts_at(r);
     }
-  } else {
-    double** dp[] = {&c->A.x, &c->A.y, &c->A.ux, &c->A.uy, &c->A.uz, &c->B.x, &c->B.y, &c->B.ux, &c->B.uy, &c->B.uz};
-    for (auto q : dp)
-      if (e == hipSuccess) e = dalloc(q, N);
   }
-  for (int k = 0; k < 2 && e == hipSuccess; k++) e = dalloc(&c->id[k], N);
   int** ip[] = {&c->code, &c->R, &c->holes, &c->ulist, &c->dlist, &c->permbuf};
   for (auto q : ip)
     if (e == hipSuccess) e = dalloc(q, N);
@@ -460,8 +461,6 @@ int wpic_create2d(wpic_ctx** out, const wpic_params2d* p) {
   c->rb = 1;
   c->rn = 2;
   set_rows(c);
-  c->A.id = c->MA.id = c->id[0];
-  c->B.id = c->MB.id = c->id[1];
   for (int k = 0; k < 3; k++) c->h_rows_ok[k] = false;
   *out = c;
   return 0;
@@ -475,12 +474,10 @@ int wpic_destroy(wpic_ctx* c) {
     if (t.a) (void)hipEventDestroy(t.a);
     if (t.b) (void)hipEventDestroy(t.b);
   }
-  void* ps[] = {c->A.x, c->A.y, c->A.ux, c->A.uy, c->A.uz, c->B.x, c->B.y, c->B.ux, c->B.uy, c->B.uz,
-                c->id[0], c->id[1], c->code, c->R, c->holes, c->ulist, c->dlist, c->rows[0], c->rows[1],
-                c->rows[2], c->cumcnt, c->rowcnt, c->rcnt, c->aosbase, c->uf, c->df, c->uj, c->pjbuf, c->phi, c->pa,
-                c->pb, c->rr, c->bb, c->ap, c->part, c->scal, c->err, c->staging, c->gbuf, c->red, c->mom,
-                c->MA.ix, c->MA.ox, c->MA.oy, c->MA.ux, c->MA.uy, c->MA.uz,
-                c->MB.ix, c->MB.ox, c->MB.oy, c->MB.ux, c->MB.uy, c->MB.uz, c->permbuf};
+  void* ps[] = {c->A.x.p, c->B.x.p, c->MA.ix.p, c->MB.ix.p, c->code, c->R, c->holes, c->ulist, c->dlist, c->permbuf,
+                c->rows[0], c->rows[1], c->rows[2], c->cumcnt, c->rowcnt, c->rcnt, c->aosbase, c->uf, c->df, c->uj,
+                c->pjbuf, c->phi, c->pa, c->pb, c->rr, c->bb, c->ap, c->part, c->scal, c->err, c->staging, c->gbuf,
+                c->red, c->mom};
   for (void* q : ps)
     if (q) (void)hipFree(q);
   if (c->ev_push) (void)hipEventDestroy(c->ev_push);
@@ -555,6 +552,7 @@ static int upload_rows(wpic_ctx* c, int which, const double* up, const int* np2,
   HIPCHK(hipStreamSynchronize(c->st));
   c->h_rows[which] = hrows;
   c->h_rows_ok[which] = true;
+  c->npart = total;
   return 0;
 }
 
@@ -708,7 +706,7 @@ int wpic_particle_solv2d(wpic_ctx* c) {
   set_rows(c);
   {
     Timed t(c, "push");
-    HIPCHK(launch_push_deposit(c, true, false, false));
+    HIPCHK(launch_push_deposit(c, true, false));
   }
   c->b_valid = true;
   c->b_accl = false;
@@ -741,7 +739,7 @@ int wpic_field_fdtd_i2d(wpic_ctx* c) {
   if (c->mixed) return mixed_only_step();
   if (!c->b_valid || !c->b_aligned || c->exch_pending)
     return set_error(WPIC_EINVAL, "field__fdtd_i needs gp slot-aligned with up (call particle__solv first)");
-  int rc = deposit(c, false, false);
+  int rc = deposit(c, false);
   if (rc) return rc;
   rc = field_after_deposit(c);
   if (rc) return rc;
@@ -809,6 +807,8 @@ int wpic_ic_shock2d(wpic_ctx* c, unsigned long long seed, int n0, double v0, dou
   HIPCHK(launch_ic_shock(c, seed, np2, v0, sd, l_damp, b));
   const size_t pl = (size_t)g.fw * g.fh;
   HIPCHK(launch_zero(c, c->df, 6 * pl));
+  c->npart = 0;
+  for (int rw = 0; rw < nr; rw++) c->npart += hrows[nr + rw];
   c->h_rows[c->rb] = hrows;
   c->h_rows_ok[c->rb] = true;
   c->b_valid = true;
@@ -872,6 +872,8 @@ int grow_rows(wpic_ctx* c, unsigned long long seed, int it, const int* nl, doubl
   std::swap(c->MA, c->MB);
   std::swap(c->ra, c->rb);
   c->aperm = nullptr;
+  c->npart = 0;
+  for (int rw = 0; rw < nr; rw++) c->npart += hrows[nr + rw];
   c->h_rows[c->ra] = hrows;
   c->h_rows_ok[c->ra] = true;
   c->h_rows_ok[c->rb] = false;
@@ -1057,6 +1059,8 @@ int wpic_ic_beams2d(wpic_ctx* c, unsigned long long seed, int n_ppc, double udri
   HIPCHK(launch_fill(c, c->uf + 2 * pl, pl, b0));
   HIPCHK(launch_zero(c, c->df, 6 * pl));
   HIPCHK(hipStreamSynchronize(c->st));
+  c->npart = 0;
+  for (int rw = 0; rw < nr; rw++) c->npart += hrows[nr + rw];
   c->h_rows[c->ra] = hrows;
   c->h_rows_ok[c->ra] = true;
   c->b_valid = false;
@@ -1094,6 +1098,8 @@ int wpic_ic_weibel2d(wpic_ctx* c, unsigned long long seed, int n0, double v_thi,
   HIPCHK(launch_fill(c, c->uf + 2 * pl, pl, b0));
   HIPCHK(launch_zero(c, c->df, 6 * pl));
   HIPCHK(hipStreamSynchronize(c->st));
+  c->npart = 0;
+  for (int rw = 0; rw < nr; rw++) c->npart += hrows[nr + rw];
   c->h_rows[c->ra] = hrows;
   c->h_rows_ok[c->ra] = true;
   c->b_valid = false;
@@ -1134,6 +1140,8 @@ int wpic_ic_harris2d(wpic_ctx* c, unsigned long long seed, int nbg, int ncs, dou
   HIPCHK(launch_ic_harris(c, seed, np2, ibg, hp));
   const size_t pl = (size_t)g.fw * g.fh;
   HIPCHK(launch_zero(c, c->df, 6 * pl));
+  c->npart = 0;
+  for (int rw = 0; rw < nr; rw++) c->npart += hrows[nr + rw];
   c->h_rows[c->rb] = hrows;
   c->h_rows_ok[c->rb] = true;
   c->b_valid = true;

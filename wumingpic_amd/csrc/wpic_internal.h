@@ -51,20 +51,76 @@ __host__ __device__ inline size_t midx(const Grid2D& g, int i, int j, int s) {
   return (size_t)7 * ((size_t)(i - (g.nxgs - 1)) + (size_t)(g.nx + 2) * ((size_t)(j - (g.nys - 1)) + (size_t)(g.ny + 2) * s));
 }
 
-// a particle buffer: the record and the reference's id (raw 64 bits) travel
-// together
-struct Parts {
-  double *x, *y, *ux, *uy, *uz;
-  uint64_t* id;
+// One field of an array of particle records: record i's value lies i strides
+// (in units of T) from the first one's.
+template <class T, int STRIDE>
+struct Col {
+  T* p;
+  __host__ __device__ T& operator[](size_t i) const { return p[i * STRIDE]; }
 };
 
-// mixed-precision particles: x cell index, FP32 in-cell offsets (x - ix and
-// y - row, both in [0, 1)) and FP32 momenta; 32 B per particle with the id
-struct PartsM {
-  int* ix;
-  float *ox, *oy, *ux, *uy, *uz;
-  uint64_t* id;
+// A particle buffer: 48-byte records (x, y, ux, uy, uz, id) one after another,
+// the reference's own up(:, ii) layout; the id is raw 64 bits.  A record that
+// is read out of slot order (a particle that changed cell or row) then costs
+// the one or two cache lines it lies in instead of one line per field, and
+// the run of records a lane group reads or writes shares a line with its
+// neighbours only at its two ends.  The push reads and writes a record as
+// three 16-byte words.
+struct Parts {
+  Col<double, 6> x, y, ux, uy, uz;
+  Col<uint64_t, 6> id;
 };
+constexpr int PART_DOUBLES = 6;
+inline Parts parts_at(double* r) {
+  return Parts{{r}, {r + 1}, {r + 2}, {r + 3}, {r + 4}, {reinterpret_cast<uint64_t*>(r + 5)}};
+}
+
+struct Rec {
+  double x, y, ux, uy, uz;
+  uint64_t id;
+};
+__device__ inline Rec load_rec(const Parts& P, size_t i) {
+  const double2* r = reinterpret_cast<const double2*>(P.x.p + PART_DOUBLES * i);
+  const double2 a = r[0], b = r[1], c = r[2];
+  return Rec{a.x, a.y, b.x, b.y, c.x, (uint64_t)__double_as_longlong(c.y)};
+}
+__device__ inline void store_rec(const Parts& P, size_t i, const Rec& q) {
+  double2* r = reinterpret_cast<double2*>(P.x.p + PART_DOUBLES * i);
+  r[0] = make_double2(q.x, q.y);
+  r[1] = make_double2(q.ux, q.uy);
+  r[2] = make_double2(q.uz, __longlong_as_double((long long)q.id));
+}
+
+// mixed-precision particles: 32-byte records of x cell index, FP32 in-cell
+// offsets (x - ix and y - row, both in [0, 1)), FP32 momenta and the id, two
+// 16-byte words
+struct PartsM {
+  Col<int, 8> ix;
+  Col<float, 8> ox, oy, ux, uy, uz;
+  Col<uint64_t, 4> id;
+};
+constexpr int PARTM_FLOATS = 8;
+inline PartsM partsm_at(float* r) {
+  return PartsM{{reinterpret_cast<int*>(r)}, {r + 1}, {r + 2}, {r + 3}, {r + 4}, {r + 5},
+                {reinterpret_cast<uint64_t*>(r + 6)}};
+}
+
+struct RecM {
+  int ix;
+  float ox, oy, ux, uy, uz;
+  uint64_t id;
+};
+__device__ inline RecM load_rec(const PartsM& P, size_t i) {
+  const int4* r = reinterpret_cast<const int4*>(P.ix.p + PARTM_FLOATS * i);
+  const int4 a = r[0], b = r[1];
+  return RecM{a.x, __int_as_float(a.y), __int_as_float(a.z), __int_as_float(a.w), __int_as_float(b.x),
+              __int_as_float(b.y), (uint64_t)(uint32_t)b.z | ((uint64_t)(uint32_t)b.w << 32)};
+}
+__device__ inline void store_rec(const PartsM& P, size_t i, const RecM& q) {
+  int4* r = reinterpret_cast<int4*>(P.ix.p + PARTM_FLOATS * i);
+  r[0] = make_int4(q.ix, __float_as_int(q.ox), __float_as_int(q.oy), __float_as_int(q.ux));
+  r[1] = make_int4(__float_as_int(q.uy), __float_as_int(q.uz), (int)(uint32_t)q.id, (int)(uint32_t)(q.id >> 32));
+}
 
 // an in-cell offset in [0, 1) as FP32: rounding up to 1 is pulled back below
 __host__ __device__ inline float to_offset(double f) {
@@ -155,7 +211,8 @@ __host__ __device__ inline void shape3(double dh, double& s0, double& s1, double
 // beg[s] + t - cum[s] of species s, the last s with cum[s] <= t (species
 // beyond nsp carry cum = INT_MAX).  Kept as named scalars and resolved with
 // masks: a chain of selects over an array is turned by the compiler into an
-// indexed table in scratch memory.
+// indexed table in scratch memory.  Most runs have two species, so the masks
+// of the third and fourth sit behind one scalar branch.
 struct CellList {
   int o0, d1, d2, d3, c1, c2, c3;  // slot offset of species 0, its steps to 1..3, their first elements
   int ob;                          // the offset of the species set last (building d1..d3)
@@ -167,11 +224,16 @@ struct CellList {
     if (s == 3) { d3 = o - ob; c3 = cum; }
     ob = o;
   }
-  __device__ void slot(int t, int& s, int& p) const {
+  __device__ void slot(int nsp, int t, int& s, int& p) const {
     static_assert(WPIC_MAXSP == 4, "CellList holds four species");
-    const int m1 = -(int)(t >= c1), m2 = -(int)(t >= c2), m3 = -(int)(t >= c3);
-    s = -(m1 + m2 + m3);
-    p = t + o0 + (m1 & d1) + (m2 & d2) + (m3 & d3);
+    const int m1 = -(int)(t >= c1);
+    s = -m1;
+    p = t + o0 + (m1 & d1);
+    if (nsp > 2) {
+      const int m2 = -(int)(t >= c2), m3 = -(int)(t >= c3);
+      s -= m2 + m3;
+      p += (m2 & d2) + (m3 & d3);
+    }
   }
 };
 
@@ -229,6 +291,61 @@ __device__ inline T row8_sum(T v) {
   return v;
 }
 
+// Sums over the G lanes of a group (4, half a DPP row or a whole one) of N
+// values at once, each sum left in one lane.  Every step halves both the
+// lanes that still differ and the values each holds: of a pair of values a
+// lane keeps one and hands the other to its partner (lane l and l ^ 8, then
+// 7 - l, l ^ 2 and l ^ 1 within the half row and the quad), so N values cost
+// about N exchanges in all instead of N per step.  group_index gives the value
+// that a lane's f-th result is the sum of, or -1 for a copy of another
+// lane's.
+template <int CTRL, class T>
+__device__ inline T dpp_get(T v) {
+  if constexpr (sizeof(T) == 8)
+    return dpp_f64<CTRL>(v);
+  else
+    return dpp_f32<CTRL>(v);
+}
+template <int N, int CTRL, class T>
+__device__ inline void halve(T* v, bool hi) {
+#pragma unroll
+  for (int k = 0; k < N / 2; k++) {
+    const T keep = hi ? v[2 * k + 1] : v[2 * k], give = hi ? v[2 * k] : v[2 * k + 1];
+    v[k] = keep + dpp_get<CTRL>(give);
+  }
+  if constexpr (N & 1) v[N / 2] = v[N - 1] + dpp_get<CTRL>(v[N - 1]);
+}
+constexpr int group_left(int n, int g) { return g == 1 ? n : group_left((n + 1) / 2, g / 2); }
+// leaves group_left(N, G) results in v
+template <int N, int G, class T>
+__device__ inline void group_reduce(T* v, int lane) {
+  static_assert(G == 4 || G == 8 || G == 16, "groups within a DPP row");
+  if constexpr (G == 16) {
+    halve<N, DPP_ROW_ROR8>(v, lane & 8);
+    group_reduce<(N + 1) / 2, 8>(v, lane);
+  } else if constexpr (G == 8) {
+    halve<N, DPP_ROW_HALF_MIRROR>(v, lane & 4);
+    group_reduce<(N + 1) / 2, 4>(v, lane);
+  } else {
+    halve<N, DPP_QUAD_XOR2>(v, lane & 2);
+    halve<(N + 1) / 2, DPP_QUAD_XOR1>(v, lane & 1);
+  }
+}
+template <int N, int G>
+__device__ inline int group_index(int f, int lane) {
+  constexpr int n1 = (N + 1) / 2;
+  if constexpr (G == 1) {
+    return f;
+  } else {
+    // the half row's mirror flips the lower bits of its upper quad: the
+    // partner of l < 4 is 7 - l
+    const int k = group_index<n1, G / 2>(f, lane);
+    if (k < 0) return -1;
+    const int i = 2 * k + ((lane & (G / 2)) ? 1 : 0);
+    return i < N ? i : -1;
+  }
+}
+
 // The sort's per-cell counts kept by a fused push: every cell of the tile
 // keeps its particles (cumcnt, added when the tile's counts are flushed)
 // except those that leave it, each of which moves one count from its own cell
@@ -251,19 +368,19 @@ __device__ inline void count_leaver(const Grid2D& g, int (*hcn)[TYC + 2][TXC + 2
     atomicAdd(&rcnt[((size_t)s * g.ny + (jn - g.nys)) * g.nx + (cn - g.nxgs)], 1);
   }
 }
-// the tile's counts, with its cells' own particles, added to rcnt (rows wrap
-// periodically in y)
+// the counts of a tile tw columns wide, with its cells' own particles, added
+// to rcnt (rows wrap periodically in y)
 template <int TXC, int TYC>
 __device__ inline void flush_counts(const Grid2D& g, int (*hcn)[TYC + 2][TXC + 2], int* rcnt, const int* cumcnt,
-                                    int i0, int j0) {
-  constexpr int N = (TYC + 2) * (TXC + 2);
-  for (int k = threadIdx.x; k < g.nsp * N; k += blockDim.x) {
-    const int s = k / N, rem = k - s * N;
-    const int hr = rem / (TXC + 2), hx = rem % (TXC + 2);
+                                    int i0, int j0, int tw) {
+  const int w = TXC + 2, n = (TYC + 2) * w;
+  for (int k = threadIdx.x; k < g.nsp * n; k += blockDim.x) {
+    const int s = k / n, rem = k - s * n;
+    const int hr = rem / w, hx = rem % w;
     int v = hcn[s][hr][hx];
     const int cx = i0 - 1 + hx;
     int jn = j0 - 1 + hr;
-    if (hr >= 1 && hr <= TYC && hx >= 1 && hx <= TXC && cx <= g.nxge && jn <= g.nye) {
+    if (hr >= 1 && hr <= TYC && hx >= 1 && hx <= tw && cx <= g.nxge && jn <= g.nye) {
       const int* cr = cumcnt + ((size_t)s * g.ny + (jn - g.nys)) * (g.nx + 1) + (cx - g.nxgs);
       v += cr[1] - cr[0];
     }
@@ -294,6 +411,16 @@ __device__ inline int xcd_tile(int bid, int ntiles) {
   return (bid & 7) * per + (bid >> 3);
 }
 inline int xcd_grid(int ntiles) { return ((ntiles + 7) >> 3) << 3; }
+
+// Columns of cells a push workgroup takes (of four rows): 32, or 16 or 8 where
+// the grid would not give each of the 256 CUs two workgroups otherwise (a
+// narrow tile stages and flushes more halo per cell).
+inline int tile_width(const Grid2D& g) {
+  const int nty = (g.ny + 3) / 4;
+  int w = 32;
+  while (w > 8 && ((g.nx + w - 1) / w) * nty < 512) w >>= 1;
+  return w;
+}
 
 // ---------------------------------------------------------------------------
 // Context
@@ -332,7 +459,6 @@ struct wpic_ctx {
   wpic::PartsM MA, MB;
   int* aperm;            // A's slot -> record in A's buffer, or null
   int* permbuf;          // [N] the sort's permutation
-  uint64_t* id[2];  // the two id buffers (A's and B's)
   int *code, *R, *holes, *ulist, *dlist;
   int* rows[3];                   // row structures: rowbase [nsp*ny] then np2 [nsp*ny]
   int ra, rb, rn;                 // which row structure belongs to A, B, the exchange
@@ -348,6 +474,7 @@ struct wpic_ctx {
   bool b_valid;       // B holds a gp array
   bool b_aligned;     // B's slots are A's slots (after particle__solv)
   int pusher;         // WPIC_PUSHER_BORIS or WPIC_PUSHER_VAY
+  long long npart;    // particles at the last load or injection (all species): picks the push's lane groups
   bool b_accl;        // B is mom_calc__accl's gp: A's positions, A's cell order
   bool exch_pending;  // R / N rows describe B after bc__particle_y
   std::vector<int> h_rows[3];  // host mirrors of the row structures
@@ -391,7 +518,7 @@ int hip_fail(hipError_t e, const char* what);
 
 // launchers (each enqueues on ctx->st) -------------------------------------
 // push / deposit
-hipError_t launch_push_deposit(wpic_ctx* c, bool push, bool deposit, bool fused);
+hipError_t launch_push_deposit(wpic_ctx* c, bool push, bool deposit);
 hipError_t launch_gather_pj(wpic_ctx* c);
 // fields
 hipError_t launch_zero(wpic_ctx* c, double* p, size_t n);
@@ -457,8 +584,8 @@ hipError_t launch_adj_particles(wpic_ctx* c, const Parts& P, const int* rows, co
                                 const double* lamJ, double* lamA, double* lamT, size_t N);
 hipError_t launch_adj_t2f(wpic_ctx* c, const double* lamT, double* lamF);
 hipError_t launch_adj_seed(wpic_ctx* c, double* lamF, double seed);
-hipError_t launch_adj_params(wpic_ctx* c, const Parts& P, const uint64_t* id, const int* rows, const double* lamA,
-                             size_t N, const double* lamF, double udrift, double uth_e, int mode, int n_ppc,
+hipError_t launch_adj_params(wpic_ctx* c, const Parts& P, const int* rows, const double* lamA, size_t N,
+                             const double* lamF, double udrift, double uth_e, int mode, int n_ppc,
                              double* out);
 hipError_t launch_perturb_bz(wpic_ctx* c, double amp, int mode);
 hipError_t launch_adj_lamF_to_planes(wpic_ctx* c, const double* lamF, double* planes);
