@@ -183,208 +183,376 @@ __global__ void k_adj_t2f(Grid2D g, const double* __restrict__ lamT, double* __r
 struct AdjPArgs {
   Grid2D g;
   Parts P;
-  const int *rowbase, *np2;
+  const int *rowbase, *cumcnt;
   const double* uf;
   const double* lamB;  // [5][N]
   const double* lamJ;  // [3][nx*ny]
   double* lamA;        // [5][N]
   double* lamT;        // [6][nx*ny]
   size_t N;
+  int ntx, nty, tw;
 };
 
-__global__ __launch_bounds__(256) void k_adj_particles(AdjPArgs a) {
+// (a, b, c) at nodes 0..4 of five, shifted from 1..3 by inc in {-1, 0, 1}
+__device__ inline void spread5(const double a[3], int inc, double o[5]) {
+  const bool l = inc < 0, r = inc > 0;
+  o[0] = l ? a[0] : 0.0;
+  o[1] = l ? a[1] : (r ? 0.0 : a[0]);
+  o[2] = l ? a[2] : (r ? a[0] : a[1]);
+  o[3] = l ? 0.0 : (r ? a[1] : a[2]);
+  o[4] = r ? a[2] : 0.0;
+}
+// its transpose: the three values of five that spread5 fills
+__device__ inline void pick3(const double o[5], int inc, double a[3]) {
+  const bool l = inc < 0, r = inc > 0;
+#pragma unroll
+  for (int k = 0; k < 3; k++) a[k] = l ? o[k] : (r ? o[k + 2] : o[k + 1]);
+}
+
+// One workgroup per tile of cells, as in the push: the tile's cell-centred
+// fields (one-cell halo) and the current's adjoint (two-cell halo) are read
+// from LDS, the fields' adjoint is summed there and added to HBM once per
+// node.  Eight lanes share a cell, so their LDS reads are broadcasts, and the
+// 54 terms a particle adds to the fields' adjoint are summed over the eight
+// before they meet in LDS.
+//
+// Bound by its FP64 instructions at 2 waves a SIMD (256 registers).  One thread
+// per particle with every field, current and atomic in HBM took 6.57 ms at
+// 256x256, 16 ppc (54 field stencils, read twice, 65 current reads and 54
+// atomics a particle, and arrays indexed by the cell step in scratch); this
+// takes 0.255 ms.  At 1 wave a SIMD, without its 200 bytes of spills, it takes
+// 3 % of a whole backward pass longer.
+__global__ __launch_bounds__(256, 2) void k_adj_particles(AdjPArgs a) {
+  constexpr int TX = 32, TY = 4, NT = 256, G = 8;
+  constexpr int SFW = TX + 2, SFH = TY + 2, ACW = TX + 4, ACH = TY + 4;
+  __shared__ double sf[6][SFW * SFH], lt[6][SFW * SFH];
+  __shared__ double lj_[3][ACW * ACH];
+  __shared__ double spc[WPIC_MAXSP][5];  // fac1, txxx, fac2, q, qk
   const Grid2D& g = a.g;
-  const int rw = blockIdx.x;
-  const int s = rw / g.ny, j = g.nys + rw % g.ny;
-  const int base = a.rowbase[rw], n = a.np2[rw];
-  const double q = g.q[s], rm = g.r[s], delt = g.delt, dx1 = g.d_delx, c2 = g.c * g.c;
-  const double fac1 = q / rm * 0.5 * delt, txxx = fac1 * fac1, fac2 = q * delt / rm;
-  const double qk = q * g.delx * g.d_delt;
-  const int ncell = g.nx * g.ny;
+  const int ntiles = a.ntx * a.nty;
+  const int tile = xcd_tile(blockIdx.x, ntiles);
+  if (tile >= ntiles) return;
+  const int i0 = g.nxgs + (tile % a.ntx) * a.tw, j0 = g.nys + (tile / a.ntx) * TY;
+  const int tid = threadIdx.x, ncell = g.nx * g.ny;
+  const int sw = a.tw + 2, aw = a.tw + 4;
+  for (int k = tid; k < sw * SFH; k += NT) {
+    const int r = k / sw, q = k - r * sw;
+    const int i = i0 - 1 + q, j = j0 - 1 + r;
+    const bool in = i <= g.nxge + 1 && j <= g.nye + 1;
+#pragma unroll
+    for (int c = 0; c < 6; c++) {
+      sf[c][r * SFW + q] = in ? cell_field_a(g, a.uf, c, i, j) : 0.0;
+      lt[c][r * SFW + q] = 0.0;
+    }
+  }
+  for (int k = tid; k < aw * ACH; k += NT) {
+    const int r = k / aw, q = k - r * aw;
+    const int i = i0 - 2 + q, j = j0 - 2 + r;
+    const bool in = i <= g.nxge + 2 && j <= g.nye + 2;
+#pragma unroll
+    for (int c = 0; c < 3; c++) lj_[c][r * ACW + q] = in ? a.lamJ[(size_t)c * ncell + pix(g, i, j)] : 0.0;
+  }
+#pragma unroll
+  for (int s = 0; s < WPIC_MAXSP; s++)
+    if (tid == s && s < g.nsp) {
+      const double q = g.q[s], rm = g.r[s], fac1 = q / rm * 0.5 * g.delt;
+      spc[s][0] = fac1;
+      spc[s][1] = fac1 * fac1;
+      spc[s][2] = q * g.delt / rm;
+      spc[s][3] = q;
+      spc[s][4] = q * g.delx * g.d_delt;
+    }
+  __syncthreads();
+
+  const double delt = g.delt, c2 = g.c * g.c;
   const size_t N = a.N;
-  const double *LJx = a.lamJ, *LJy = a.lamJ + ncell, *LJz = a.lamJ + 2 * ncell;
-  for (int kk = threadIdx.x; kk < n; kk += blockDim.x) {
-    const int p = base + kk;
-    const double x = a.P.x[p], y = a.P.y[p];
-    const double u[3] = {a.P.ux[p], a.P.uy[p], a.P.uz[p]};
-    const int i = (int)(x * dx1);
-    // ---- forward recomputation ----
-    double sx[3], dsxdh[3], sy[3], dsydh[3];
-    shape_d(x * dx1 - 0.5 - i, sx, dsxdh);
-    shape_d(y * dx1 - 0.5 - j, sy, dsydh);
-    double F[6];
-    for (int cm = 0; cm < 6; cm++) {
-      double f = 0.0;
-      for (int bb = 0; bb < 3; bb++)
-        for (int aa = 0; aa < 3; aa++) f += cell_field_a(g, a.uf, cm, i - 1 + aa, j - 1 + bb) * sx[aa] * sy[bb];
-      F[cm] = f;
-    }
-    const double B[3] = {F[0], F[1], F[2]}, E[3] = {F[3], F[4], F[5]};
-    double uvm[3];
-    for (int d = 0; d < 3; d++) uvm[d] = u[d] + fac1 * E[d];
-    const double gam = sqrt(c2 + uvm[0] * uvm[0] + uvm[1] * uvm[1] + uvm[2] * uvm[2]);
-    const double igam = 1.0 / gam;
-    const double fac1r = fac1 * igam;
-    const double B2 = B[0] * B[0] + B[1] * B[1] + B[2] * B[2];
-    const double D = gam + txxx * B2 * igam;
-    const double fac2r = fac2 / D;
-    double v2[3], t[3], w[3], up_[3], gv[3];
-    cross(uvm, B, v2);
-    for (int d = 0; d < 3; d++) t[d] = uvm[d] + fac1r * v2[d];
-    cross(t, B, w);
-    for (int d = 0; d < 3; d++) up_[d] = uvm[d] + fac2r * w[d];
-    for (int d = 0; d < 3; d++) gv[d] = up_[d] + fac1 * E[d];
-    const double g2 = gv[0] * gv[0] + gv[1] * gv[1] + gv[2] * gv[2];
-    const double gmv = 1.0 / sqrt(1.0 + g2 / c2);
-    const double xn = x + gv[0] * delt * gmv, yn = y + gv[1] * delt * gmv;
-    // deposit shapes (fast-mode factored form of field.f90:274-298)
-    const int i2 = (int)(xn * dx1), j2 = (int)(yn * dx1);
-    const int incx = i2 - i, incy = j2 - j;
-    double s1x[3], ds1x[3], s1y[3], ds1y[3];
-    shape_d(xn * dx1 - 0.5 - i2, s1x, ds1x);
-    shape_d(yn * dx1 - 0.5 - j2, s1y, ds1y);
-    double s0x[5] = {0.0, sx[0], sx[1], sx[2], 0.0}, s0y[5] = {0.0, sy[0], sy[1], sy[2], 0.0};
-    double dsx[5], dsy[5];
-    for (int m = 0; m < 5; m++) {
-      const int ax = m - 1 - incx, ay = m - 1 - incy;
-      dsx[m] = (ax >= 0 && ax < 3 ? s1x[ax] : 0.0) - s0x[m];
-      dsy[m] = (ay >= 0 && ay < 3 ? s1y[ay] : 0.0) - s0y[m];
-    }
-    double cx[4], cy[4];
-    {
-      double rx = 0.0, ry = 0.0;
-      for (int m = 0; m < 4; m++) {
-        rx -= dsx[m];
-        ry -= dsy[m];
-        cx[m] = rx;
-        cy[m] = ry;
-      }
-    }
-    double wx[5], wy[5], Ay[5], By[5];
-    for (int m = 0; m < 5; m++) {
-      wy[m] = s0y[m] + 0.5 * dsy[m];
-      wx[m] = s0x[m] + 0.5 * dsx[m];
-      Ay[m] = wy[m];
-      By[m] = 0.5 * s0y[m] + dsy[m] / 3.0;
-    }
-    const double qvz = q * (gv[2] * gmv);
-    // ---- reverse: deposit ----
-    double G_dsx[5] = {0, 0, 0, 0, 0}, G_dsy[5] = {0, 0, 0, 0, 0};
-    double G_s0x[5] = {0, 0, 0, 0, 0}, G_s0y[5] = {0, 0, 0, 0, 0};
-    double G_cx[4] = {0, 0, 0, 0}, G_cy[4] = {0, 0, 0, 0};
-    double G_wx[5] = {0, 0, 0, 0, 0}, G_wy[5] = {0, 0, 0, 0, 0}, G_Ay[5] = {0, 0, 0, 0, 0}, G_By[5] = {0, 0, 0, 0, 0};
-    double G_qvz = 0.0;
-    for (int jp = 0; jp < 5; jp++)
-      for (int m = 0; m < 4; m++) {
-        const double L = LJx[pix(g, i + m - 1, j + jp - 2)];
-        G_cx[m] += qk * L * wy[jp];
-        G_wy[jp] += qk * L * cx[m];
-      }
-    for (int m = 0; m < 4; m++)
-      for (int ip = 0; ip < 5; ip++) {
-        const double L = LJy[pix(g, i + ip - 2, j + m - 1)];
-        G_cy[m] += qk * L * wx[ip];
-        G_wx[ip] += qk * L * cy[m];
-      }
-    for (int jp = 0; jp < 5; jp++)
-      for (int ip = 0; ip < 5; ip++) {
-        const double L = LJz[pix(g, i + ip - 2, j + jp - 2)];
-        G_s0x[ip] += qvz * L * Ay[jp];
-        G_dsx[ip] += qvz * L * By[jp];
-        G_Ay[jp] += qvz * L * s0x[ip];
-        G_By[jp] += qvz * L * dsx[ip];
-        G_qvz += L * (s0x[ip] * Ay[jp] + dsx[ip] * By[jp]);
-      }
-    for (int k = 0; k < 4; k++)
-      for (int m = k; m < 4; m++) {
-        G_dsx[k] -= G_cx[m];
-        G_dsy[k] -= G_cy[m];
-      }
-    for (int m = 0; m < 5; m++) {
-      G_s0y[m] += G_wy[m] + G_Ay[m] + 0.5 * G_By[m];
-      G_dsy[m] += 0.5 * G_wy[m] + 0.5 * G_Ay[m] + G_By[m] / 3.0;
-      G_s0x[m] += G_wx[m];
-      G_dsx[m] += 0.5 * G_wx[m];
-    }
-    double G_xn = a.lamB[p], G_yn = a.lamB[N + p];
-    for (int m = 0; m < 5; m++) {
-      G_s0x[m] -= G_dsx[m];
-      G_s0y[m] -= G_dsy[m];
-      const int ax = m - 1 - incx, ay = m - 1 - incy;
-      if (ax >= 0 && ax < 3) G_xn += G_dsx[m] * ds1x[ax] * dx1;
-      if (ay >= 0 && ay < 3) G_yn += G_dsy[m] * ds1y[ay] * dx1;
-    }
-    // ---- reverse: move, x' = x + g dt gmv ----
-    double G_g[3] = {a.lamB[2 * N + p], a.lamB[3 * N + p], a.lamB[4 * N + p]};
-    double G_gmv = q * gv[2] * G_qvz + gv[0] * delt * G_xn + gv[1] * delt * G_yn;
-    G_g[2] += q * gmv * G_qvz;
-    G_g[0] += delt * gmv * G_xn;
-    G_g[1] += delt * gmv * G_yn;
-    const double dgmv = -gmv * gmv * gmv / c2;
-    for (int d = 0; d < 3; d++) G_g[d] += G_gmv * dgmv * gv[d];
-    double G_x = G_xn, G_y = G_yn;
-    // ---- reverse: Boris ----
-    double G_E[3], G_B[3] = {0, 0, 0}, G_up[3], G_uvm[3];
-    for (int d = 0; d < 3; d++) {
-      G_up[d] = G_g[d];
-      G_E[d] = fac1 * G_g[d];
-    }
-    // up_ = uvm + fac2r w, w = t x B
-    double G_w[3], G_t[3], tmp[3];
-    double G_fac2r = G_up[0] * w[0] + G_up[1] * w[1] + G_up[2] * w[2];
-    for (int d = 0; d < 3; d++) {
-      G_uvm[d] = G_up[d];
-      G_w[d] = fac2r * G_up[d];
-    }
-    cross(B, G_w, G_t);  // d(t x B).v / dt = B x v
-    cross(G_w, t, tmp);  // d(t x B).v / dB = v x t
-    for (int d = 0; d < 3; d++) G_B[d] += tmp[d];
-    // t = uvm + fac1r v2, v2 = uvm x B
-    double G_fac1r = G_t[0] * v2[0] + G_t[1] * v2[1] + G_t[2] * v2[2];
-    double G_v2[3];
-    for (int d = 0; d < 3; d++) {
-      G_uvm[d] += G_t[d];
-      G_v2[d] = fac1r * G_t[d];
-    }
-    cross(B, G_v2, tmp);
-    for (int d = 0; d < 3; d++) G_uvm[d] += tmp[d];
-    cross(G_v2, uvm, tmp);
-    for (int d = 0; d < 3; d++) G_B[d] += tmp[d];
-    // fac2r = fac2 / D, D = gam + txxx |B|^2 igam, fac1r = fac1 igam, igam = 1/gam
-    const double G_D = -fac2r / D * G_fac2r;
-    double G_gam = G_D;
-    double G_igam = txxx * B2 * G_D + fac1 * G_fac1r;
-    for (int d = 0; d < 3; d++) G_B[d] += 2.0 * txxx * igam * B[d] * G_D;
-    G_gam += -igam * igam * G_igam;
-    for (int d = 0; d < 3; d++) G_uvm[d] += uvm[d] / gam * G_gam;
-    // uvm = u + fac1 E
-    double G_u[3];
-    for (int d = 0; d < 3; d++) {
-      G_u[d] = G_uvm[d];
-      G_E[d] += fac1 * G_uvm[d];
-    }
-    // ---- reverse: gather F_c = sum T sx sy ----
-    const double G_F[6] = {G_B[0], G_B[1], G_B[2], G_E[0], G_E[1], G_E[2]};
-    double G_sx[3] = {0, 0, 0}, G_sy[3] = {0, 0, 0};
-    for (int cm = 0; cm < 6; cm++) {
-      if (G_F[cm] == 0.0) continue;
-      for (int bb = 0; bb < 3; bb++)
-        for (int aa = 0; aa < 3; aa++) {
-          const double T = cell_field_a(g, a.uf, cm, i - 1 + aa, j - 1 + bb);
-          G_sx[aa] += G_F[cm] * T * sy[bb];
-          G_sy[bb] += G_F[cm] * T * sx[aa];
-          unsafeAtomicAdd(&a.lamT[(size_t)cm * ncell + pix(g, i - 1 + aa, j - 1 + bb)], G_F[cm] * sx[aa] * sy[bb]);
+  const int w = tid >> 6, lane = tid & 63, lg = lane % G;
+  const int lj = w, j = j0 + lj;
+  // where this lane's sums of two components' 18 terms go in lt: component
+  // (0 or 1) and the node's offset from the cell's lower left neighbour
+  constexpr int NRES = group_left(18, G);
+  int node[NRES];
+#pragma unroll
+  for (int f = 0; f < NRES; f++) {
+    const int q = group_index<18, G>(f, lane);
+    node[f] = q < 0 ? -1 : (q / 9) * (SFW * SFH) + (q % 9 / 3) * SFW + q % 3;
+  }
+  for (int l0 = 0; l0 < a.tw; l0 += 64 / G) {
+    const int li = l0 + lane / G, i = i0 + li;
+    const bool live = i <= g.nxge && j <= g.nye;  // uniform within a group
+    CellList cl;
+    int tot = 0;
+#pragma unroll
+    for (int s = 0; s < WPIC_MAXSP; s++) {
+      if (s < g.nsp) {
+        int b0 = 0, b1 = 0, rb = 0;
+        if (live) {
+          const int rw = s * g.ny + (j - g.nys);
+          const int* cr = a.cumcnt + (size_t)rw * (g.nx + 1) + (i - g.nxgs);
+          b0 = cr[0];
+          b1 = cr[1];
+          rb = a.rowbase[rw];
         }
+        cl.set(s, rb + b0, tot);
+        tot += b1 - b0;
+      } else {
+        cl.set(s, 0, 0x7fffffff);
+      }
     }
-    for (int aa = 0; aa < 3; aa++) {
-      G_x += (G_sx[aa] + G_s0x[aa + 1]) * dsxdh[aa] * dx1;
-      G_y += (G_sy[aa] + G_s0y[aa + 1]) * dsydh[aa] * dx1;
+    const int so = lj * SFW + li;  // the cell's lower left neighbour in sf and lt
+    const int ao = lj * ACW + li;  // node (-2, -2) in lj_
+    for (int t = lg; __any(t < tot); t += G) {
+      const bool act = t < tot;
+      int s, p;
+      cl.slot(g.nsp, t, s, p);
+      Rec P = {i + 0.5, j + 0.5, 0.0, 0.0, 0.0, 0};
+      double G_xn = 0.0, G_yn = 0.0, G_g[3] = {0.0, 0.0, 0.0};
+      if (act) {
+        P = load_rec(a.P, p);
+        G_xn = a.lamB[p];
+        G_yn = a.lamB[N + p];
+#pragma unroll
+        for (int d = 0; d < 3; d++) G_g[d] = a.lamB[(2 + d) * N + p];
+      }
+      const double x = P.x, y = P.y, u[3] = {P.ux, P.uy, P.uz};
+      const double fac1 = spc[s][0], txxx = spc[s][1], fac2 = spc[s][2], q = spc[s][3], qk = spc[s][4];
+      // ---- forward recomputation ----
+      double sx[3], dsxdh[3], sy[3], dsydh[3];
+      shape_d(x - 0.5 - i, sx, dsxdh);
+      shape_d(y - 0.5 - j, sy, dsydh);
+      double F[6];
+#pragma unroll
+      for (int cm = 0; cm < 6; cm++) {
+        double f = 0.0;
+#pragma unroll
+        for (int b = 0; b < 3; b++) {
+          const double* r = &sf[cm][so + b * SFW];
+          f = fma(fma(r[2], sx[2], fma(r[1], sx[1], r[0] * sx[0])), sy[b], f);
+        }
+        F[cm] = f;
+      }
+      const double B[3] = {F[0], F[1], F[2]}, E[3] = {F[3], F[4], F[5]};
+      double uvm[3];
+#pragma unroll
+      for (int d = 0; d < 3; d++) uvm[d] = u[d] + fac1 * E[d];
+      const double gam = sqrt(c2 + uvm[0] * uvm[0] + uvm[1] * uvm[1] + uvm[2] * uvm[2]);
+      const double igam = 1.0 / gam;
+      const double fac1r = fac1 * igam;
+      const double B2 = B[0] * B[0] + B[1] * B[1] + B[2] * B[2];
+      const double iD = 1.0 / (gam + txxx * B2 * igam);
+      const double fac2r = fac2 * iD;
+      double v2[3], tt[3], ww[3], gv[3];
+      cross(uvm, B, v2);
+#pragma unroll
+      for (int d = 0; d < 3; d++) tt[d] = uvm[d] + fac1r * v2[d];
+      cross(tt, B, ww);
+#pragma unroll
+      for (int d = 0; d < 3; d++) gv[d] = uvm[d] + fac2r * ww[d] + fac1 * E[d];
+      const double g2 = gv[0] * gv[0] + gv[1] * gv[1] + gv[2] * gv[2];
+      const double gmv = 1.0 / sqrt(1.0 + g2 / c2);
+      const double xn = x + gv[0] * delt * gmv, yn = y + gv[1] * delt * gmv;
+      // deposit shapes (fast-mode factored form of field.f90:274-298)
+      const int i2 = (int)xn, j2 = (int)yn;
+      const int incx = i2 - i, incy = j2 - j;
+      double ds1x[3], ds1y[3];
+      double s0x[5] = {0.0, sx[0], sx[1], sx[2], 0.0}, s0y[5] = {0.0, sy[0], sy[1], sy[2], 0.0};
+      double dsx[5], dsy[5];
+      {
+        double s1[3];
+        shape_d(xn - 0.5 - i2, s1, ds1x);
+        spread5(s1, incx, dsx);
+        shape_d(yn - 0.5 - j2, s1, ds1y);
+        spread5(s1, incy, dsy);
+      }
+#pragma unroll
+      for (int m = 0; m < 5; m++) {
+        dsx[m] -= s0x[m];
+        dsy[m] -= s0y[m];
+      }
+      const double qvz = q * (gv[2] * gmv);
+      // ---- reverse: deposit ----
+      double G_dsx[5], G_dsy[5], G_s0x[5], G_s0y[5];
+      {
+        // Jx = cx(m) qk wy(n): cx(m) = -sum_{k<=m} dsx(k), wy = s0y + dsy/2
+        double G_wy[5], G_cx[4] = {0.0, 0.0, 0.0, 0.0}, cx[4];
+        cx[0] = -dsx[0];
+#pragma unroll
+        for (int m = 1; m < 4; m++) cx[m] = cx[m - 1] - dsx[m];
+#pragma unroll
+        for (int n = 0; n < 5; n++) {
+          const double* r = &lj_[0][ao + n * ACW + 1];
+          const double wy = fma(0.5, dsy[n], s0y[n]);
+          double gw = 0.0;
+#pragma unroll
+          for (int m = 0; m < 4; m++) {
+            G_cx[m] = fma(r[m], wy, G_cx[m]);
+            gw = fma(r[m], cx[m], gw);
+          }
+          G_wy[n] = gw;
+        }
+        double run = 0.0;
+        G_dsx[4] = 0.0;
+#pragma unroll
+        for (int m = 3; m >= 0; m--) {
+          run -= G_cx[m];
+          G_dsx[m] = qk * run;
+        }
+#pragma unroll
+        for (int n = 0; n < 5; n++) {
+          G_s0y[n] = qk * G_wy[n];
+          G_dsy[n] = 0.5 * G_s0y[n];
+        }
+      }
+      {
+        double G_wx[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, G_cy[4], cy = 0.0;
+        double wx[5];
+#pragma unroll
+        for (int n = 0; n < 5; n++) wx[n] = fma(0.5, dsx[n], s0x[n]);
+#pragma unroll
+        for (int m = 0; m < 4; m++) {
+          cy -= dsy[m];
+          const double* r = &lj_[1][ao + (m + 1) * ACW];
+          double gc = 0.0;
+#pragma unroll
+          for (int n = 0; n < 5; n++) {
+            gc = fma(r[n], wx[n], gc);
+            G_wx[n] = fma(r[n], cy, G_wx[n]);
+          }
+          G_cy[m] = gc;
+        }
+        double run = 0.0;
+#pragma unroll
+        for (int m = 3; m >= 0; m--) {
+          run -= G_cy[m];
+          G_dsy[m] = fma(qk, run, G_dsy[m]);
+        }
+#pragma unroll
+        for (int n = 0; n < 5; n++) {
+          G_s0x[n] = qk * G_wx[n];
+          G_dsx[n] = fma(0.5, G_s0x[n], G_dsx[n]);
+        }
+      }
+      double G_qvz = 0.0;
+#pragma unroll
+      for (int n = 0; n < 5; n++) {
+        // Jz = qvz (s0x(m) A(n) + dsx(m) B(n)), A = s0y + dsy/2, B = s0y/2 + dsy/3
+        const double* r = &lj_[2][ao + n * ACW];
+        const double A = fma(0.5, dsy[n], s0y[n]), Bn = fma(1.0 / 3.0, dsy[n], 0.5 * s0y[n]);
+        double ga = 0.0, gb = 0.0;
+#pragma unroll
+        for (int m = 0; m < 5; m++) {
+          const double L = r[m];
+          G_s0x[m] = fma(qvz * L, A, G_s0x[m]);
+          G_dsx[m] = fma(qvz * L, Bn, G_dsx[m]);
+          ga = fma(L, s0x[m], ga);
+          gb = fma(L, dsx[m], gb);
+        }
+        G_qvz = fma(ga, A, fma(gb, Bn, G_qvz));
+        G_s0y[n] = fma(qvz, fma(0.5, gb, ga), G_s0y[n]);
+        G_dsy[n] = fma(qvz, fma(0.5, ga, gb * (1.0 / 3.0)), G_dsy[n]);
+      }
+      double h[3];
+      pick3(G_dsx, incx, h);
+      G_xn += h[0] * ds1x[0] + h[1] * ds1x[1] + h[2] * ds1x[2];
+      pick3(G_dsy, incy, h);
+      G_yn += h[0] * ds1y[0] + h[1] * ds1y[1] + h[2] * ds1y[2];
+      double G_sx[3], G_sy[3];
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        G_sx[k] = G_s0x[k + 1] - G_dsx[k + 1];
+        G_sy[k] = G_s0y[k + 1] - G_dsy[k + 1];
+      }
+      // ---- reverse: move, x' = x + g dt gmv ----
+      double G_gmv = q * gv[2] * G_qvz + gv[0] * delt * G_xn + gv[1] * delt * G_yn;
+      G_g[2] += q * gmv * G_qvz;
+      G_g[0] += delt * gmv * G_xn;
+      G_g[1] += delt * gmv * G_yn;
+      const double dgmv = -gmv * gmv * gmv / c2;
+#pragma unroll
+      for (int d = 0; d < 3; d++) G_g[d] += G_gmv * dgmv * gv[d];
+      double G_x = G_xn, G_y = G_yn;
+      // ---- reverse: Boris ----
+      double G_E[3], G_B[3], G_uvm[3], G_w[3], G_t[3], tmp[3], G_v2[3];
+      const double G_fac2r = G_g[0] * ww[0] + G_g[1] * ww[1] + G_g[2] * ww[2];
+#pragma unroll
+      for (int d = 0; d < 3; d++) {
+        G_E[d] = fac1 * G_g[d];
+        G_uvm[d] = G_g[d];
+        G_w[d] = fac2r * G_g[d];
+      }
+      cross(B, G_w, G_t);   // d(t x B).v / dt = B x v
+      cross(G_w, tt, G_B);  // d(t x B).v / dB = v x t
+      const double G_fac1r = G_t[0] * v2[0] + G_t[1] * v2[1] + G_t[2] * v2[2];
+#pragma unroll
+      for (int d = 0; d < 3; d++) {
+        G_uvm[d] += G_t[d];
+        G_v2[d] = fac1r * G_t[d];
+      }
+      cross(B, G_v2, tmp);
+#pragma unroll
+      for (int d = 0; d < 3; d++) G_uvm[d] += tmp[d];
+      cross(G_v2, uvm, tmp);
+#pragma unroll
+      for (int d = 0; d < 3; d++) G_B[d] += tmp[d];
+      // fac2r = fac2 / D, D = gam + txxx |B|^2 igam, fac1r = fac1 igam, igam = 1/gam
+      const double G_D = -fac2r * iD * G_fac2r;
+      const double G_igam = txxx * B2 * G_D + fac1 * G_fac1r;
+      const double G_gam = G_D - igam * igam * G_igam;
+#pragma unroll
+      for (int d = 0; d < 3; d++) {
+        G_B[d] += 2.0 * txxx * igam * B[d] * G_D;
+        G_uvm[d] += uvm[d] * igam * G_gam;
+        G_E[d] += fac1 * G_uvm[d];  // uvm = u + fac1 E
+      }
+      // ---- reverse: gather F_c = sum T sx sy ----
+      double G_F[6] = {G_B[0], G_B[1], G_B[2], G_E[0], G_E[1], G_E[2]};
+#pragma unroll
+      for (int cm = 0; cm < 6; cm++) {
+#pragma unroll
+        for (int b = 0; b < 3; b++) {
+          const double* r = &sf[cm][so + b * SFW];
+          const double gy = G_F[cm] * sy[b];
+          G_sx[0] = fma(r[0], gy, G_sx[0]);
+          G_sx[1] = fma(r[1], gy, G_sx[1]);
+          G_sx[2] = fma(r[2], gy, G_sx[2]);
+          G_sy[b] = fma(G_F[cm], fma(r[2], sx[2], fma(r[1], sx[1], r[0] * sx[0])), G_sy[b]);
+        }
+        if (!act) G_F[cm] = 0.0;
+      }
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        G_x += G_sx[k] * dsxdh[k];
+        G_y += G_sy[k] * dsydh[k];
+      }
+      if (act) {
+        a.lamA[p] = G_x;
+        a.lamA[N + p] = G_y;
+#pragma unroll
+        for (int d = 0; d < 3; d++) a.lamA[(2 + d) * N + p] = G_uvm[d];
+      }
+#pragma unroll
+      for (int cp = 0; cp < 6; cp += 2) {
+        double v[18];
+#pragma unroll
+        for (int k = 0; k < 18; k++) v[k] = G_F[cp + k / 9] * sx[k % 3] * sy[k % 9 / 3];
+        group_reduce<18, G>(v, lane);
+#pragma unroll
+        for (int f = 0; f < NRES; f++)
+          if (live && node[f] >= 0) atomicAdd(&lt[cp][0] + (node[f] + so), v[f]);
+      }
     }
-    a.lamA[p] = G_x;
-    a.lamA[N + p] = G_y;
-    a.lamA[2 * N + p] = G_u[0];
-    a.lamA[3 * N + p] = G_u[1];
-    a.lamA[4 * N + p] = G_u[2];
+  }
+  __syncthreads();
+  for (int k = tid; k < sw * SFH; k += NT) {
+    const int r = k / sw, q = k - r * sw;
+    const int i = i0 - 1 + q, j = j0 - 1 + r;
+    if (i > g.nxge + 1 || j > g.nye + 1) continue;
+    const int n = pix(g, i, j);
+#pragma unroll
+    for (int c = 0; c < 6; c++) {
+      const double v = lt[c][r * SFW + q];
+      if (v != 0.0) unsafeAtomicAdd(&a.lamT[(size_t)c * ncell + n], v);
+    }
   }
 }
 
@@ -487,21 +655,23 @@ hipError_t launch_adj_field2(wpic_ctx* c, double* lamF2, double* lamJ) {
   return hipGetLastError();
 }
 
-hipError_t launch_adj_particles(wpic_ctx* c, const Parts& P, const int* rows, const double* uf, const double* lamB,
-                                const double* lamJ, double* lamA, double* lamT, size_t N) {
+hipError_t launch_adj_particles(wpic_ctx* c, const Parts& P, const int* rows, const int* cumcnt, const double* uf,
+                                const double* lamB, const double* lamJ, double* lamA, double* lamT, size_t N) {
   AdjPArgs a;
   a.g = c->g;
   a.P = P;
-  const int nr = c->g.nsp * c->g.ny;
   a.rowbase = rows;
-  a.np2 = rows + nr;
+  a.cumcnt = cumcnt;
   a.uf = uf;
   a.lamB = lamB;
   a.lamJ = lamJ;
   a.lamA = lamA;
   a.lamT = lamT;
   a.N = N;
-  hipLaunchKernelGGL(k_adj_particles, dim3(nr), dim3(256), 0, c->st, a);
+  a.tw = tile_width(c->g);
+  a.ntx = (c->g.nx + a.tw - 1) / a.tw;
+  a.nty = (c->g.ny + 3) / 4;
+  hipLaunchKernelGGL(k_adj_particles, dim3(xcd_grid(a.ntx * a.nty)), dim3(256), 0, c->st, a);
   return hipGetLastError();
 }
 

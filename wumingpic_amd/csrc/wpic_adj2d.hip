@@ -29,7 +29,7 @@ struct AdjState {
   std::vector<double*> ck_part, ck_uf, ck_df;
   std::vector<int*> ck_rows, ck_cumcnt;
   std::vector<double*> st_part, st_uf;
-  std::vector<int*> st_rows, st_perm;
+  std::vector<int*> st_rows, st_perm, st_cumcnt;
   double *lamA = nullptr, *lamA2 = nullptr, *lamB = nullptr;
   double *lamF = nullptr, *lamF2 = nullptr, *lamJ = nullptr, *lamT = nullptr;
   double* red = nullptr;
@@ -53,6 +53,7 @@ void adj_free(wpic_ctx* c) {
   for (auto p : a->st_uf) fr(p);
   for (auto p : a->st_rows) fr(p);
   for (auto p : a->st_perm) fr(p);
+  for (auto p : a->st_cumcnt) fr(p);
   for (void* p : {(void*)a->lamA, (void*)a->lamA2, (void*)a->lamB, (void*)a->lamF, (void*)a->lamF2, (void*)a->lamJ,
                   (void*)a->lamT, (void*)a->red})
     fr(p);
@@ -133,11 +134,13 @@ int alloc_adj(wpic_ctx* c, int nsteps, int every) {
   a.st_part.assign(K, nullptr);
   a.st_uf.assign(K, nullptr);
   a.st_perm.assign(K, nullptr);
+  a.st_cumcnt.assign(K, nullptr);
   a.st_rows.assign(K + 1, nullptr);
   for (int t = 0; t < K && e == hipSuccess; t++) {
     e = dal(&a.st_part[t], PART_DOUBLES * a.N);
     if (e == hipSuccess) e = dal(&a.st_uf[t], 6 * a.pl);
     if (e == hipSuccess) e = dal(&a.st_perm[t], a.N);
+    if (e == hipSuccess) e = dal(&a.st_cumcnt[t], (size_t)a.ncc);
   }
   for (int t = 0; t <= K && e == hipSuccess; t++) e = dal(&a.st_rows[t], (size_t)2 * a.nr);
   for (double** p : {&a.lamA, &a.lamA2, &a.lamB})
@@ -220,7 +223,7 @@ int wpic_adj_backward2d(wpic_ctx* c, double seed) {
     int rc = restore_state(c, s);
     if (rc) return rc;
     for (int t = 0; t < K; t++) {
-      rc = save_state(c, a.st_part[t], a.st_rows[t], nullptr, a.st_uf[t], nullptr);
+      rc = save_state(c, a.st_part[t], a.st_rows[t], a.st_cumcnt[t], a.st_uf[t], nullptr);
       if (rc) return rc;
       c->perm_out = a.st_perm[t];
       rc = step_once(c);
@@ -238,8 +241,8 @@ int wpic_adj_backward2d(wpic_ctx* c, double seed) {
       if (rc) return rc;
       HIPCHK(launch_adj_field2(c, a.lamF2, a.lamJ));
       HIPCHK(hipMemsetAsync(a.lamT, 0, sizeof(double) * 6 * a.nc, c->st));
-      HIPCHK(launch_adj_particles(c, parts_at(a.st_part[t]), a.st_rows[t], a.st_uf[t], a.lamB, a.lamJ, a.lamA2,
-                                  a.lamT, N));
+      HIPCHK(launch_adj_particles(c, parts_at(a.st_part[t]), a.st_rows[t], a.st_cumcnt[t], a.st_uf[t], a.lamB,
+                                  a.lamJ, a.lamA2, a.lamT, N));
       HIPCHK(launch_adj_t2f(c, a.lamT, a.lamF2));
       std::swap(a.lamF, a.lamF2);
       std::swap(a.lamA, a.lamA2);

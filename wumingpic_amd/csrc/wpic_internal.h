@@ -580,8 +580,8 @@ hipError_t launch_adj_unsort(wpic_ctx* c, const int* rows, const int* perm, cons
                              size_t N);
 hipError_t launch_adj_field1(wpic_ctx* c, const double* lamF, double* lamF2, double* lamJ);
 hipError_t launch_adj_field2(wpic_ctx* c, double* lamF2, double* lamJ);
-hipError_t launch_adj_particles(wpic_ctx* c, const Parts& P, const int* rows, const double* uf, const double* lamB,
-                                const double* lamJ, double* lamA, double* lamT, size_t N);
+hipError_t launch_adj_particles(wpic_ctx* c, const Parts& P, const int* rows, const int* cumcnt, const double* uf,
+                                const double* lamB, const double* lamJ, double* lamA, double* lamT, size_t N);
 hipError_t launch_adj_t2f(wpic_ctx* c, const double* lamT, double* lamF);
 hipError_t launch_adj_seed(wpic_ctx* c, double* lamF, double seed);
 hipError_t launch_adj_params(wpic_ctx* c, const Parts& P, const int* rows, const double* lamA, size_t N,
