@@ -11,7 +11,7 @@
 // fused kernel's (k_push_deposit3d_fast): 8x4x4-cell tiles, 8 lanes per cell,
 // the 54 current values of a particle that stays in its cell in registers, a
 // particle that changes cell queued (per wave) with its offsets and added with
-// its 3 x 4 x 4 window per component after the wave's round of cells.  The push writes the exchange code
+// its window when 64 have gathered.  The push writes the exchange code
 // ((new x cell - nxgs) << 4 | y-z direction) itself: the x wrap is a cell
 // wrap and the y-z offsets are already relative to the destination column.
 #include "wpic_internal3d.h"
@@ -25,7 +25,8 @@ namespace m3 {
 constexpr int TX = 8, TY = 4, TZ = 4, NT = 256, G = 8;
 constexpr int SW = TX + 2, SH = TY + 2, SD = TZ + 2, SN = SW * SH * SD;  // staged tmpf
 constexpr int AW = TX + 4, AH = TY + 4, AD = TZ + 4, AN = AW * AH * AD;  // current tile
-constexpr int QW = 128;    // queued cell-changing particles per wave and round (beyond: added at once)
+constexpr int KP = 5;    // passes between two deposits of what stays
+constexpr int QW = 128;  // queued cell-changing particles per wave: 63 left over and 64 of a pass at most
 }  // namespace m3
 
 struct Mix3Args {
@@ -63,6 +64,15 @@ __device__ inline void shape3m(float dh, float& s0, float& s1, float& s2) {
   s2 = 0.5f * (0.5f + dh) * (0.5f + dh);
 }
 
+// the staged fields of a cell: (Bx, By, Bz, Ex) in one 16-byte LDS read and
+// (Ey, Ez) in one of 8
+struct alignas(16) Field4M {
+  float v[4];
+};
+struct alignas(8) Field2M {
+  float v[2];
+};
+
 struct Mix3Const {
   float delt, ic2, cc2;  // dt, 1/c^2, c^2
 };
@@ -76,26 +86,53 @@ struct Mix3Push {
   float g4, g5, g6, gmv;
 };
 
-__device__ inline Mix3Push mixed_push3(const Mix3Const& mc, const float (*sf)[m3::SN], int so, const float* kc,
-                                       float ox, float oy, float oz, float ux, float uy, float uz) {
+__device__ inline Mix3Push mixed_push3(const Mix3Const& mc, const Field4M* fa, const Field2M* fb, int so,
+                                       const float* kc, const RecM3& p) {
 #pragma clang fp contract(fast)
   using namespace m3;
   const float fac1 = kc[0], txxx = kc[1], fac2 = kc[2];
+  const float ux = p.ux, uy = p.uy, uz = p.uz;
   Mix3Push r;
-  shape3m(ox - 0.5f, r.sh[0], r.sh[1], r.sh[2]);
-  shape3m(oy - 0.5f, r.sh[3], r.sh[4], r.sh[5]);
-  shape3m(oz - 0.5f, r.sh[6], r.sh[7], r.sh[8]);
-  asm volatile("" : "+v"(so));
-  float fl[6];
+  // the gather: nine rows of three cells, the next two rows' reads in flight
+  // while one is combined
+  constexpr int AHEAD = 2;
+  int off = so - SW * SH - SW - 1;  // the cell's lowest neighbour
+  asm volatile("" : "+v"(off));
+  Field4M va[AHEAD + 1][3];
+  Field2M vb[AHEAD + 1][3];
+  auto load = [&](int q) {
 #pragma unroll
-  for (int cm = 0; cm < 6; cm++) {
-    const float* f = &sf[cm][so];
-#define RX(o) (f[(o)-1] * r.sh[0] + f[o] * r.sh[1] + f[(o) + 1] * r.sh[2])
-#define RY(o) (RX((o)-SW) * r.sh[3] + RX(o) * r.sh[4] + RX((o) + SW) * r.sh[5])
-    fl[cm] = RY(-SW * SH) * r.sh[6] + RY(0) * r.sh[7] + RY(SW * SH) * r.sh[8];
-#undef RY
-#undef RX
+    for (int e = 0; e < 3; e++) {
+      const int o = off + (q / 3) * (SW * SH) + (q % 3) * SW + e;
+      va[q % (AHEAD + 1)][e] = fa[o];
+      vb[q % (AHEAD + 1)][e] = fb[o];
+    }
+  };
+#pragma unroll
+  for (int q = 0; q < AHEAD; q++) load(q);
+  __builtin_amdgcn_sched_barrier(0);
+  shape3m(p.ox - 0.5f, r.sh[0], r.sh[1], r.sh[2]);
+  shape3m(p.oy - 0.5f, r.sh[3], r.sh[4], r.sh[5]);
+  shape3m(p.oz - 0.5f, r.sh[6], r.sh[7], r.sh[8]);
+  float fl[6], ya[6];
+#pragma unroll
+  for (int q = 0; q < 9; q++) {
+    if (q + AHEAD < 9) load(q + AHEAD);
+    __builtin_amdgcn_sched_barrier(0);
+    const Field4M* A = va[q % (AHEAD + 1)];
+    const Field2M* B = vb[q % (AHEAD + 1)];
+    const int n = q % 3, m = q / 3;
+#pragma unroll
+    for (int c = 0; c < 6; c++) {
+      const float t = c < 4 ? A[0].v[c & 3] * r.sh[0] + A[1].v[c & 3] * r.sh[1] + A[2].v[c & 3] * r.sh[2]
+                            : B[0].v[c & 1] * r.sh[0] + B[1].v[c & 1] * r.sh[1] + B[2].v[c & 1] * r.sh[2];
+      ya[c] = n == 0 ? t * r.sh[3] : ya[c] + t * r.sh[3 + n];
+      if (n == 2) fl[c] = m == 0 ? ya[c] * r.sh[6] : fl[c] + ya[c] * r.sh[6 + m];
+    }
+    __builtin_amdgcn_sched_barrier(0);
   }
+  // (combined here, not where a later block uses them)
+  asm volatile("" : "+v"(fl[0]), "+v"(fl[1]), "+v"(fl[2]), "+v"(fl[3]), "+v"(fl[4]), "+v"(fl[5]));
   const float bpx = fl[0], bpy = fl[1], bpz = fl[2], epx = fl[3], epy = fl[4], epz = fl[5];
   float uvm1 = ux + fac1 * epx;
   float uvm2 = uy + fac1 * epy;
@@ -114,7 +151,7 @@ __device__ inline Mix3Push mixed_push3(const Mix3Const& mc, const float (*sf)[m3
   r.g5 = uvm2 + fac1 * epy;
   r.g6 = uvm3 + fac1 * epz;
   r.gmv = 1.0f / sqrtf(1.0f + (r.g4 * r.g4 + r.g5 * r.g5 + r.g6 * r.g6) * mc.ic2);
-  const float o[3] = {ox, oy, oz}, u[3] = {r.g4, r.g5, r.g6};
+  const float o[3] = {p.ox, p.oy, p.oz}, u[3] = {r.g4, r.g5, r.g6};
 #pragma unroll
   for (int d = 0; d < 3; d++) {
     const float np = o[d] + u[d] * mc.delt * r.gmv;
@@ -129,60 +166,77 @@ __device__ inline Mix3Push mixed_push3(const Mix3Const& mc, const float (*sf)[m3
   return r;
 }
 
-// Current of one particle that changes cell, with the 4-node window per axis
-// of k_push_deposit3d_fast (|inc| <= 1): add(comp, xo, yo, zo, v) receives
-// each non-zero value with its node offset from the particle's old cell.
-template <class Add>
-__device__ inline void deposit3_window_m(const Mix3Push& r, float qd, Add add) {
+// Current of one particle that changes cell, added to the FP64 tile with the
+// window of k_push_deposit3d_fast (|inc| <= 1): o is the tile's Jx at the
+// particle's cell.
+__device__ inline void deposit3_window_m(double* o, const float dh0[3], const float dh1[3], const int inc[3],
+                                         float qd) {
 #pragma clang fp contract(fast)
-  float S0[3][4], DS[3][4], cq[3][3];
-  int lo[3];
+  using namespace m3;
+  constexpr int SY = AW, SZ = AW * AH;
+  float S[3][4], D[3][4], cq[3][3];
+  bool mv[3];
 #pragma unroll
   for (int d = 0; d < 3; d++) {
-    const int in = r.inc[d];
-    float s11, s12, s13;
-    shape3m(r.f[d] - 0.5f, s11, s12, s13);
-    const float a = (float)abs(in);
-    const float smo1 = in < 0 ? a : 0.0f, smo2 = 1.0f - a, smo3 = in > 0 ? a : 0.0f;
-    const float s0m = r.sh[3 * d], s00 = r.sh[3 * d + 1], s0p = r.sh[3 * d + 2];
-    const float f0 = s11 * smo1;
-    const float f1 = s11 * smo2 + s12 * smo1 - s0m;
-    const float f2 = s12 * smo2 + s13 * smo1 + s11 * smo3 - s00;
-    const float f3 = s13 * smo2 + s12 * smo3 - s0p;
-    const float f4 = s13 * smo3;
-    const bool left = in < 0;
-    lo[d] = left ? 0 : 1;
-    S0[d][0] = left ? 0.0f : s0m;
-    S0[d][1] = left ? s0m : s00;
-    S0[d][2] = left ? s00 : s0p;
-    S0[d][3] = left ? s0p : 0.0f;
-    DS[d][0] = left ? f0 : f1;
-    DS[d][1] = left ? f1 : f2;
-    DS[d][2] = left ? f2 : f3;
-    DS[d][3] = left ? f3 : f4;
+    float t0, t1, t2, u0, u1, u2;
+    shape3m(dh0[d], t0, t1, t2);
+    shape3m(dh1[d], u0, u1, u2);
+    const bool left = inc[d] < 0, right = inc[d] > 0;
+    mv[d] = left || right;
+    o += (left ? -2 : -1) * (d == 0 ? 1 : (d == 1 ? SY : SZ));  // window node 0 of the axis
+    S[d][0] = left ? 0.0f : t0;
+    S[d][1] = left ? t0 : t1;
+    S[d][2] = left ? t1 : t2;
+    S[d][3] = left ? t2 : 0.0f;
+    D[d][0] = (right ? 0.0f : u0) - S[d][0];
+    D[d][1] = (right ? u0 : u1) - S[d][1];
+    D[d][2] = (right ? u1 : u2) - S[d][2];
+    D[d][3] = (right ? u2 : 0.0f) - S[d][3];
     float run = 0.0f;
 #pragma unroll
     for (int m = 0; m < 3; m++) {
-      run -= DS[d][m];
+      run -= D[d][m];
       cq[d][m] = run * qd;
     }
   }
+  // face m lies between window nodes m and m + 1, at the offset of node m + 1
 #pragma unroll
-  for (int u = 0; u < 4; u++) {
-    const float ax = S0[0][u] + 0.5f * DS[0][u], bx = 0.5f * S0[0][u] + (1.0f / 3.0f) * DS[0][u];
-    const float ay = S0[1][u] + 0.5f * DS[1][u], by = 0.5f * S0[1][u] + (1.0f / 3.0f) * DS[1][u];
+  for (int v = 0; v < 4; v++) {  // z node
+    if (v == 3 && !mv[2]) break;
+    const float Sz = S[2][v], Dz = D[2][v], az = Sz + 0.5f * Dz, bz = 0.5f * Sz + (1.0f / 3.0f) * Dz;
+    double* const r = o + v * SZ;
 #pragma unroll
-    for (int v = 0; v < 4; v++) {
-      const float wx = ay * S0[2][v] + by * DS[2][v];  // y node u, z node v
-      const float wy = ax * S0[2][v] + bx * DS[2][v];  // x node u, z node v
-      const float wz = ax * S0[1][v] + bx * DS[1][v];  // x node u, y node v
+    for (int u = 0; u < 4; u++) {  // y node of Jx
+      if (u == 3 && !mv[1]) break;
+      const float w = S[1][u] * az + D[1][u] * bz;
+      tile_add(r + u * SY + 1, cq[0][0] * w);
+      tile_add(r + u * SY + 2, cq[0][1] * w);
+      if (mv[0]) tile_add(r + u * SY + 3, cq[0][2] * w);
+      __builtin_amdgcn_sched_barrier(0);
+    }
 #pragma unroll
-      for (int m = 0; m < 3; m++) {
-        const float vx = cq[0][m] * wx, vy = cq[1][m] * wy, vz = cq[2][m] * wz;
-        if (vx != 0.0f) add(0, lo[0] + m - 1, lo[1] + u - 2, lo[2] + v - 2, vx);
-        if (vy != 0.0f) add(1, lo[0] + u - 2, lo[1] + m - 1, lo[2] + v - 2, vy);
-        if (vz != 0.0f) add(2, lo[0] + u - 2, lo[1] + v - 2, lo[2] + m - 1, vz);
-      }
+    for (int u = 0; u < 4; u++) {  // x node of Jy
+      if (u == 3 && !mv[0]) break;
+      const float w = S[0][u] * az + D[0][u] * bz;
+      tile_add(r + AN + u + SY, cq[1][0] * w);
+      tile_add(r + AN + u + 2 * SY, cq[1][1] * w);
+      if (mv[1]) tile_add(r + AN + u + 3 * SY, cq[1][2] * w);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+#pragma unroll
+  for (int v = 0; v < 4; v++) {  // y node of Jz
+    if (v == 3 && !mv[1]) break;
+    const float Sy = S[1][v], Dy = D[1][v], ay = Sy + 0.5f * Dy, by = 0.5f * Sy + (1.0f / 3.0f) * Dy;
+#pragma unroll
+    for (int u = 0; u < 4; u++) {  // x node
+      if (u == 3 && !mv[0]) break;
+      const float w = S[0][u] * ay + D[0][u] * by;
+      double* const r = o + 2 * AN + v * SY + u;
+      tile_add(r + SZ, cq[2][0] * w);
+      tile_add(r + 2 * SZ, cq[2][1] * w);
+      if (mv[2]) tile_add(r + 3 * SZ, cq[2][2] * w);
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
 }
@@ -194,19 +248,23 @@ __device__ inline void tile_origin_m(const Grid3D& g, int tile, int ntx, int nty
   k0 = g.nzs + (rest / nty) * m3::TZ;
 }
 
+// Its structure is that of k_push_deposit3d_fast.  What bounds it (256^3, 2
+// species of 16 ppc, 537 M particles): VALU issue and 43 GB of traffic in 20.3
+// ms, where one pass with the sums kept, one array per field, single LDS reads
+// and per-round queues took 28.5.  KP = 3, 4, 5, 6: 22.0, 21.4, 20.4, 20.4 ms.
 __global__ __launch_bounds__(m3::NT, 3) void k_push_deposit_mixed3d(Mix3Args a) {
 #pragma clang fp contract(fast)
   using namespace m3;
-  __shared__ float sf[6][SN];
+  constexpr int NW = NT / 64;
+  static_assert(64 / G == TX && NW == TY, "a wave takes a row of the tile at a time");
+  __shared__ Field4M sfa[SN];
+  __shared__ Field2M sfb[SN];
   __shared__ double acc[3][AN];
   __shared__ float spc[WPIC_MAXSP][4];  // fac1, txxx, fac2, q delx / delt
-  // each wave's cell-changing particles of the round: old and new in-cell
-  // offsets, and cell in the tile | species << 7 | (inc + 1) per axis << 9,
-  // 11, 13
-  constexpr int NW = NT / 64;
-  __shared__ float xqo[NW][QW][6];
+  // the waves' queued particles: old and new shape arguments, and cell in the
+  // tile | species << 7 | (inc + 1) per axis << 9, 11, 13
+  __shared__ float xqo[NW][6][QW];
   __shared__ int xqc[NW][QW];
-  __shared__ int nxq[NW];
   const Grid3D& g = a.g;
   const int ntiles = a.ntx * a.nty * a.ntz;
   const int tile = xcd_tile(blockIdx.x, ntiles);
@@ -217,10 +275,15 @@ __global__ __launch_bounds__(m3::NT, 3) void k_push_deposit_mixed3d(Mix3Args a) 
   for (int q = tid; q < 6 * SN; q += NT) {
     const int c = q / SN, rem = q - c * SN;
     const int i = i0 - 1 + rem % SW, j = j0 - 1 + (rem / SW) % SH, k = k0 - 1 + rem / (SW * SH);
-    if (i <= g.nxge + 1 && j <= g.nye + 1 && k <= g.nze + 1) sf[c][rem] = (float)tmpf3m(g, a.uf, c, i, j, k);
+    if (i <= g.nxge + 1 && j <= g.nye + 1 && k <= g.nze + 1) {
+      const float v = (float)tmpf3m(g, a.uf, c, i, j, k);
+      if (c < 4)
+        sfa[rem].v[c] = v;
+      else
+        sfb[rem].v[c - 4] = v;
+    }
   }
-  for (int q = tid; q < 3 * AN; q += NT) (&acc[0][0])[q] = 0.0f;
-  if (tid < NW) nxq[tid] = 0;
+  for (int q = tid; q < 3 * AN; q += NT) (&acc[0][0])[q] = 0.0;
 #pragma unroll
   for (int s = 0; s < WPIC_MAXSP; s++) {
     if (tid == s && s < g.nsp) {
@@ -233,162 +296,207 @@ __global__ __launch_bounds__(m3::NT, 3) void k_push_deposit_mixed3d(Mix3Args a) 
   }
   __syncthreads();
 
-  const int grp = tid / G, lg = tid % G;
-  constexpr int NGRP = NT / G;
   Mix3Const mc;
   mc.delt = (float)g.delt;
   mc.ic2 = (float)(1.0 / (g.c * g.c));
   mc.cc2 = (float)(g.c * g.c);
-  const int w = tid >> 6, lane = tid & 63;
-  int* const nq_r = &nxq[w];
-  // rounds of NGRP cells (one per group, 64 / G per wave), each wave
-  // draining its own queue after its cells of the round
-  for (int rnd = 0; rnd < (TX * TY * TZ) / NGRP; rnd++) {
-    const int cc = rnd * NGRP + grp;
-    const int li = cc % TX, lj = (cc / TX) % TY, lk = cc / (TX * TY);
-    const int i = i0 + li, j = j0 + lj, k = k0 + lk;
-    if (i <= g.nxge && j <= g.nye && k <= g.nze) {  // uniform within a group
-    const int col = (j - g.nys) + g.ny * (k - g.nzs);
-    const int so = (lk + 1) * (SW * SH) + (lj + 1) * SW + (li + 1);
-    const int bx = li + 2, by = lj + 2, bz = lk + 2;
-    // stayers' current: [m][u][v], face m, nodes u - 1, v - 1 of the other two
-    // axes in the order (y, z) for Jx, (x, z) for Jy, (x, y) for Jz
-    float jx[18], jy[18], jz[18];
+  // (the wave's number, the same in its lanes, and with it j and k stay in
+  // scalar registers)
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, lg = lane % G;
+  const int li = lane / G, lj = w;
+  const int i = i0 + li, j = j0 + lj;
+  int nq = 0;  // queued particles, the same in all lanes
+
+  // the currents of the last (at most 64) queued particles
+  auto drain = [&]() {
+    // written by this wave's own lanes: LDS operations of one wave complete in order
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const int n0 = nq > 64 ? nq - 64 : 0, q = n0 + lane;
+    if (q < nq) {
+      const int e = xqc[w][q];
+      const int cc = e & 127, s = (e >> 7) & 3;
+      const int inc[3] = {((e >> 9) & 3) - 1, ((e >> 11) & 3) - 1, ((e >> 13) & 3) - 1};
+      const float o[3] = {xqo[w][0][q], xqo[w][1][q], xqo[w][2][q]};
+      const float f[3] = {xqo[w][3][q], xqo[w][4][q], xqo[w][5][q]};
+      deposit3_window_m(&acc[0][((cc / (TX * TY) + 2) * AH + (cc / TX % TY + 2)) * AW + (cc % TX + 2)], o, f, inc,
+                        spc[s][3]);
+    }
+    nq = n0;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+
+  for (int lk = 0; lk < TZ; lk++) {
+    const int k = k0 + lk;
+    const bool live = i <= g.nxge && j <= g.nye && k <= g.nze;  // uniform within a group
+    CellList cl;
+    int tot = 0;
 #pragma unroll
-    for (int q = 0; q < 18; q++) jx[q] = jy[q] = jz[q] = 0.0f;
-    for (int s = 0; s < g.nsp; s++) {
-      const int rw = s * g.ncol + col;
-      const int* cr = a.cumcnt + (size_t)rw * (g.nx + 1);
-      const int base = a.colbase[rw];
-      const int pbeg = base + cr[i - g.nxgs], pend = base + cr[i - g.nxgs + 1];
+    for (int s = 0; s < WPIC_MAXSP; s++) {
+      if (s < g.nsp) {
+        int c0 = 0, c1 = 0, cb = 0;
+        if (live) {
+          const int rw = s * g.ncol + (j - g.nys) + g.ny * (k - g.nzs);
+          const int* cr = a.cumcnt + (size_t)rw * (g.nx + 1) + (i - g.nxgs);
+          c0 = cr[0];
+          c1 = cr[1];
+          cb = a.colbase[rw];
+        }
+        cl.set(s, cb + c0, tot);
+        tot += c1 - c0;
+      } else {
+        cl.set(s, 0, 0x7fffffff);
+      }
+    }
+    const int so = (lk + 1) * (SW * SH) + (lj + 1) * SW + (li + 1);
+
+    int ia_nn = 0;
+    // (a cell's surplus lanes push a particle at rest at its centre)
+    RecM3 pr = {i, 0.5f, 0.5f, 0.5f, 0.0f, 0.0f, 0.0f, 0, 0};
+    {
+      int s_, p_, ia_n = 0;
+      if (lg < tot) {
+        cl.slot(g.nsp, lg, s_, p_);
+        ia_n = a.ap ? a.ap[p_] : p_;
+      }
+      if (lg + G < tot) {
+        cl.slot(g.nsp, lg + G, s_, p_);
+        ia_nn = a.ap ? a.ap[p_] : p_;
+      }
+      if (lg < tot) pr = load_rec(a.A, ia_n);
+    }
+    // KP passes at a time: the pushes, one straight line for all lanes as in 2D
+    // (a lane past its cell's last particle repeats one with zero charge and
+    // stores nothing), then the current of those that stay
+    int t = lg;
+    while (__any(t < tot)) {
+    float pd[KP][6];  // old and new shape arguments of the last KP passes, the latest first
+    int ps[KP];    // species, or -1: no current from it
+#pragma unroll
+    for (int h = 0; h < KP; h++) {
+      ps[h] = -1;
+#pragma unroll
+      for (int d = 0; d < 6; d++) pd[h][d] = 0.0f;
+    }
+    for (int h = 0; h < KP && __any(t < tot); h++, t += G) {
+      const bool act = t < tot;
+      int s, pi;
+      cl.slot(g.nsp, t, s, pi);
+      const RecM3 cur = pr;
+      if (t + G < tot) pr = load_rec(a.A, ia_nn);
+      if (t + 2 * G < tot) {
+        int s_, p_;
+        cl.slot(g.nsp, t + 2 * G, s_, p_);
+        ia_nn = a.ap ? a.ap[p_] : p_;
+      }
       const float* kc = spc[s];
-      const float qd = kc[3];
-      for (int pi = pbeg + lg; pi < pend; pi += G) {
-        const int ia = a.ap ? a.ap[pi] : pi;
-        const float o[3] = {a.A.ox[ia], a.A.oy[ia], a.A.oz[ia]};
-        const Mix3Push r = mixed_push3(mc, sf, so, kc, o[0], o[1], o[2], a.A.ux[ia], a.A.uy[ia], a.A.uz[ia]);
-        a.B.ux[pi] = r.g4;
-        a.B.uy[pi] = r.g5;
-        a.B.uz[pi] = r.g6;
-        a.B.id[pi] = a.A.id[ia];
+      const Mix3Push r = mixed_push3(mc, sfa, sfb, so, kc, cur);
+      const bool stays = (r.inc[0] | r.inc[1] | r.inc[2]) == 0;
+      const bool mover = act && !stays;
+      if (act) {
+        // the x wrap is a cell wrap; the y-z step goes to the exchange
         int dj = r.inc[1], dk = r.inc[2];
-        if (r.inc[0] < -1 || r.inc[0] > 1 || dj < -1 || dj > 1 || dk < -1 || dk > 1) {
+        int cx = i + r.inc[0];
+        if (cx < g.nxgs)
+          cx += g.nx;
+        else if (cx > g.nxge)
+          cx -= g.nx;
+        if ((unsigned)(r.inc[0] + 1) > 2u || (unsigned)(dj + 1) > 2u || (unsigned)(dk + 1) > 2u || cx < g.nxgs ||
+            cx > g.nxge) {
           atomicOr(a.err, ERR_DOMAIN);
           dj = dj < -1 ? -1 : (dj > 1 ? 1 : dj);
           dk = dk < -1 ? -1 : (dk > 1 ? 1 : dk);
+          cx = cx < g.nxgs ? g.nxgs : (cx > g.nxge ? g.nxge : cx);
         }
-        if ((r.inc[0] | r.inc[1] | r.inc[2]) == 0) {
-          float s0[3][3], ds[3][3], A[3][3], B[3][3], cq[3][2];
-#pragma unroll
-          for (int d = 0; d < 3; d++) {
-            float s1[3];
-            shape3m(r.f[d] - 0.5f, s1[0], s1[1], s1[2]);
-#pragma unroll
-            for (int n = 0; n < 3; n++) {
-              s0[d][n] = r.sh[3 * d + n];
-              ds[d][n] = s1[n] - s0[d][n];
-              A[d][n] = s0[d][n] + 0.5f * ds[d][n];
-              B[d][n] = 0.5f * s0[d][n] + (1.0f / 3.0f) * ds[d][n];
-            }
-            cq[d][0] = -ds[d][0] * qd;
-            cq[d][1] = (-ds[d][0] - ds[d][1]) * qd;
-          }
-#pragma unroll
-          for (int u = 0; u < 3; u++)
-#pragma unroll
-            for (int v = 0; v < 3; v++) {
-              const float wx = A[1][u] * s0[2][v] + B[1][u] * ds[2][v];
-              const float wy = A[0][u] * s0[2][v] + B[0][u] * ds[2][v];
-              const float wz = A[0][u] * s0[1][v] + B[0][u] * ds[1][v];
-#pragma unroll
-              for (int m = 0; m < 2; m++) {
-                const int q = (m * 3 + u) * 3 + v;
-                jx[q] += cq[0][m] * wx;
-                jy[q] += cq[1][m] * wy;
-                jz[q] += cq[2][m] * wz;
-              }
-            }
-        } else {
-          const int slot = wave_enqueue(nq_r);
-          if (slot < QW) {
-#pragma unroll
-            for (int d = 0; d < 3; d++) {
-              xqo[w][slot][d] = o[d];
-              xqo[w][slot][3 + d] = r.f[d];
-            }
-            xqc[w][slot] = cc | (s << 7) | ((r.inc[0] + 1) << 9) | ((r.inc[1] + 1) << 11) | ((r.inc[2] + 1) << 13);
-          } else {
-            deposit3_window_m(r, qd, [&](int comp, int xo, int yo, int zo, float v) {
-              tile_add(&acc[comp][((bz + zo) * AH + (by + yo)) * AW + (bx + xo)], v);
-            });
-          }
-        }
-        // the x wrap is a cell wrap; the y-z step goes to the exchange
-        int cx = i + r.inc[0];
-        if (cx < g.nxgs) cx += g.nx;
-        else if (cx > g.nxge) cx -= g.nx;
-        if (cx < g.nxgs || cx > g.nxge) {
-          atomicOr(a.err, ERR_DOMAIN);
-          cx = cx < g.nxgs ? g.nxgs : g.nxge;
-        }
-        a.B.ix[pi] = cx;
-        a.B.ox[pi] = r.f[0];
-        a.B.oy[pi] = r.f[1];
-        a.B.oz[pi] = r.f[2];
         a.code[pi] = ((cx - g.nxgs) << CODE_SHIFT3) | ((dk + 1) * 3 + (dj + 1));
+        store_rec(a.B, pi, RecM3{cx, r.f[0], r.f[1], r.f[2], r.g4, r.g5, r.g6, cur.id0, cur.id1});
       }
-    }
-    // reduce the stayers' current over the group, spread the LDS atomics
 #pragma unroll
-    for (int q = 0; q < 54; q++) {
-      float v = q < 18 ? jx[q] : (q < 36 ? jy[q - 18] : jz[q - 36]);
-      static_assert(G == 8, "the group is one half of a DPP row");
-      v = row8_sum(v);
-      if ((q % G) == lg && v != 0.0f) {
-        const int comp = q / 18, rr = q % 18, m = rr / 9, u = (rr / 3) % 3, b = rr % 3;
-        int xo, yo, zo;
-        if (comp == 0) {
-          xo = m; yo = u - 1; zo = b - 1;
-        } else if (comp == 1) {
-          xo = u - 1; yo = m; zo = b - 1;
-        } else {
-          xo = u - 1; yo = b - 1; zo = m;
+      for (int q = KP - 1; q > 0; q--) {
+        ps[q] = ps[q - 1];
+#pragma unroll
+        for (int d = 0; d < 6; d++) pd[q][d] = pd[q - 1][d];
+      }
+      ps[0] = act && stays ? s : -1;
+      pd[0][0] = cur.ox - 0.5f;
+      pd[0][1] = cur.oy - 0.5f;
+      pd[0][2] = cur.oz - 0.5f;
+#pragma unroll
+      for (int d = 0; d < 3; d++) pd[0][3 + d] = r.f[d] - 0.5f;
+      const uint64_t mm = __ballot(mover);
+      if (mm) {
+        if (mover) {
+          const int slot = nq + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mm >> 32),
+                                                               __builtin_amdgcn_mbcnt_lo((uint32_t)mm, 0));
+#pragma unroll
+          for (int d = 0; d < 6; d++) xqo[w][d][slot] = pd[0][d];
+          xqc[w][slot] = ((lk * TY + lj) * TX + li) | (s << 7) | (((r.inc[0] + 1) & 3) << 9) |
+                         (((r.inc[1] + 1) & 3) << 11) | (((r.inc[2] + 1) & 3) << 13);
         }
-        tile_add(&acc[comp][((bz + zo) * AH + (by + yo)) * AW + (bx + xo)], v);
+        nq += __popcll(mm);
+        if (nq >= 64) drain();
       }
     }
-    }  // the cell
-
-    // the wave's queued particles of the round, from their offsets: the queue
-    // was written by this wave's own lanes, and LDS operations of one wave
-    // complete in order
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    const int nq = *nq_r < QW ? *nq_r : QW;
-    for (int q = lane; q < nq; q += 64) {
-      const int e = xqc[w][q];
-      const int qcc = e & 127, s = (e >> 7) & 3;
-      const int qbx = qcc % TX + 2, qby = (qcc / TX) % TY + 2, qbz = qcc / (TX * TY) + 2;
-      Mix3Push r;
+    // the current of the particles that stay: sum 18 c + 9 m + 3 u + b of
+    // component c, face m along its own axis, nodes u - 1, b - 1 of the other
+    // two in the order x, y, z
+    float v[54];
+#pragma unroll
+    for (int q = 0; q < 54; q++) v[q] = 0.0f;
+#pragma unroll
+    for (int h = 0; h < KP; h++) {
+      if (!__any(ps[h] >= 0)) continue;
+      const float qd = ps[h] >= 0 ? spc[ps[h] & 3][3] : 0.0f;
+      float S[3][3], D[3][3], cq[3][2];  // s0, ds = s1 - s0, -sum ds
 #pragma unroll
       for (int d = 0; d < 3; d++) {
-        shape3m(xqo[w][q][d] - 0.5f, r.sh[3 * d], r.sh[3 * d + 1], r.sh[3 * d + 2]);
-        r.f[d] = xqo[w][q][3 + d];
-        r.inc[d] = ((e >> (9 + 2 * d)) & 3) - 1;
+        float t0, t1, t2;
+        shape3m(pd[h][d], S[d][0], S[d][1], S[d][2]);
+        shape3m(pd[h][3 + d], t0, t1, t2);
+        D[d][0] = t0 - S[d][0];
+        D[d][1] = t1 - S[d][1];
+        D[d][2] = t2 - S[d][2];
+        cq[d][0] = (0.0f - D[d][0]) * qd;
+        cq[d][1] = ((0.0f - D[d][0]) - D[d][1]) * qd;
       }
-      deposit3_window_m(r, spc[s][3], [&](int comp, int xo, int yo, int zo, float v) {
-        tile_add(&acc[comp][((qbz + zo) * AH + (qby + yo)) * AW + (qbx + xo)], v);
-      });
+#pragma unroll
+      for (int b = 0; b < 3; b++) {
+        const float az = 0.5f * D[2][b] + S[2][b], bz = (1.0f / 3.0f) * D[2][b] + 0.5f * S[2][b];
+        const float ay = 0.5f * D[1][b] + S[1][b], by = (1.0f / 3.0f) * D[1][b] + 0.5f * S[1][b];
+#pragma unroll
+        for (int u = 0; u < 3; u++) {
+          const float wx = S[1][u] * az + D[1][u] * bz;  // y node u, z node b
+          const float wy = S[0][u] * az + D[0][u] * bz;  // x node u, z node b
+          const float wz = S[0][u] * ay + D[0][u] * by;  // x node u, y node b
+#pragma unroll
+          for (int m = 0; m < 2; m++) {
+            const int q = 9 * m + 3 * u + b;
+            v[q] = cq[0][m] * wx + v[q];
+            v[18 + q] = cq[1][m] * wy + v[18 + q];
+            v[36 + q] = cq[2][m] * wz + v[36 + q];
+          }
+        }
+      }
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    if (lane == 0) *nq_r = 0;
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    // over the group, spread over its lanes
+    group_reduce<54, G>(v, lane);
+    // (the places are worked out here: kept over the passes they would spill)
+    int ln = lane;
+    asm volatile("" : "+v"(ln));
+    double* const o = &acc[0][0] + ((lk + 2) * AH + (lj + 2)) * AW + (li + 2);
+#pragma unroll
+    for (int f = 0; f < group_left(54, G); f++) {
+      const int q = group_index<54, G>(f, ln);
+      const int c = q / 18, m = q % 18 / 9, u = q % 9 / 3 - 1, b = q % 3 - 1;
+      const int xo = c == 0 ? m : u, yo = c == 0 ? u : (c == 1 ? m : b), zo = c == 2 ? m : b;
+      if (live && q >= 0 && v[f] != 0.0f) tile_add(o + (c * AN + (zo * AH + yo) * AW + xo), v[f]);
+    }
+    }
   }
+  if (nq) drain();
 
   __syncthreads();
   const size_t pl = plane3(g);

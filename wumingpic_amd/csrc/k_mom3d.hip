@@ -36,15 +36,6 @@ __host__ __device__ inline size_t midx3(const Grid3D& g, int i, int j, int k, in
           (size_t)(g.nx + 2) * ((size_t)(j - (g.nys - 1)) + (size_t)(g.ny + 2) * ((size_t)(k - (g.nzs - 1)) + (size_t)(g.nz + 2) * s)));
 }
 
-__device__ inline void stage_fields3(const Grid3D& g, const double* uf, double (*sf)[p3::SN], int i0, int j0, int k0) {
-  using namespace p3;
-  for (int q = threadIdx.x; q < 6 * SN; q += NT) {
-    const int c = q / SN, rem = q - c * SN;
-    const int i = i0 - 1 + rem % SW, j = j0 - 1 + (rem / SW) % SH, k = k0 - 1 + rem / (SW * SH);
-    if (i <= g.nxge + 1 && j <= g.nye + 1 && k <= g.nze + 1) sf[c][rem] = tmpf3(g, uf, c, i, j, k);
-  }
-}
-
 // the seven moments of one particle times wx*wy*wz, in the reference's
 // product order (mom_calc.f90:253-324)
 struct Mom3Terms {
@@ -87,7 +78,7 @@ struct Cic3 {
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(p3::NT) void k_mom_accl3d(Mom3Args a) {
   using namespace p3;
-  __shared__ double sf[6][SN];
+  __shared__ FieldTile3 sf;
   const Grid3D& g = a.g;
   const int ntiles = a.ntx * a.nty * a.ntz;
   const int tile = xcd_tile(blockIdx.x, ntiles);
@@ -114,8 +105,8 @@ __global__ __launch_bounds__(p3::NT) void k_mom_accl3d(Mom3Args a) {
         const int ia = a.ap ? a.ap[pi] : pi;
         const double x = a.A.x[ia], y = a.A.y[ia], z = a.A.z[ia];
         double nxp, nyp, nzp, g4, g5, g6, sh[9];
-        boris_push3(sf, so, i, j, k, g.d_delx, hdelt, g.c, a.fac1[s], a.txxx[s], a.fac2[s], x, y, z, a.A.ux[ia],
-                    a.A.uy[ia], a.A.uz[ia], nxp, nyp, nzp, g4, g5, g6, sh);
+        boris_push3(sf, so, i, j, k, hdelt, g.c, a.fac1[s], a.txxx[s], a.fac2[s], x, y, z, a.A.ux[ia],
+                    a.A.uy[ia], a.A.uz[ia], nxp, nyp, nzp, g4, g5, g6);
         a.B.x[pi] = x;
         a.B.y[pi] = y;
         a.B.z[pi] = z;
@@ -159,7 +150,7 @@ __global__ __launch_bounds__(p3::NT) void k_mom3d_tile(Mom3Args a) {
   using namespace p3;
   using namespace m3;
   constexpr int GM = MOM3_G, NGRP = NT / GM;  // lanes per cell, cells in flight
-  __shared__ double sf[KICK ? 6 : 1][SN];
+  __shared__ FieldPair sf[KICK ? 3 : 1][SN];
   __shared__ double mt[7][MN];
   const Grid3D& g = a.g;
   const int ntiles = a.ntx * a.nty * a.ntz;
@@ -197,8 +188,8 @@ __global__ __launch_bounds__(p3::NT) void k_mom3d_tile(Mom3Args a) {
           y = a.A.y[ia];
           z = a.A.z[ia];
           double nxp, nyp, nzp, sh[9];
-          boris_push3(sf, so, i, j, k, g.d_delx, hdelt, c, a.fac1[s], a.txxx[s], a.fac2[s], x, y, z, a.A.ux[ia],
-                      a.A.uy[ia], a.A.uz[ia], nxp, nyp, nzp, ux, uy, uz, sh);
+          boris_push3(sf, so, i, j, k, hdelt, c, a.fac1[s], a.txxx[s], a.fac2[s], x, y, z, a.A.ux[ia],
+                      a.A.uy[ia], a.A.uz[ia], nxp, nyp, nzp, ux, uy, uz);
         } else {
           x = a.B.x[pi];
           y = a.B.y[pi];

@@ -29,9 +29,6 @@ __device__ inline double cell_field(const Grid2D& g, const double* uf, int c, in
 // The staged cell-centred fields: pairs (Bx, By), (Bz, Ex), (Ey, Ez) of a cell
 // side by side, so that one 16-byte LDS read brings two components and every
 // read of the gather is an immediate offset from one address.
-struct alignas(16) FieldPair {
-  double a, b;
-};
 using FieldTile = FieldPair[3][SFW * SFH];
 
 // the fields of tw <= TX columns of cells and their halo
@@ -93,41 +90,9 @@ __device__ inline void gather6(const FieldPair (*sf)[SFW * SFH], int li, int lj,
                     (+f[6].b * sx0 + f[7].b * sx1 + f[8].b * sx2) * sy2;
     __builtin_amdgcn_sched_barrier(0);
   }
-}
-
-// The correctly rounded square root of x and the correctly rounded reciprocal
-// of that root, as sqrt(x) and 1. / sqrt(x) give them.  The compiler's own
-// sequences scale against overflow and handle zeros and infinities, twice
-// over; for x within 2^-200 .. 2^200 none of that is needed and the
-// reciprocal starts from the root's own iterate instead of a new seed.
-//   y ~ 1/sqrt(x) from the hardware; g ~ sqrt(x) and h ~ 1/(2 sqrt(x)) refined
-//   together by Goldschmidt's iteration, then g corrected twice with the exact
-//   residual x - g g (a fused multiply-add), which rounds it correctly; the
-//   reciprocal of g from 2 h by one Newton step and one correction with the
-//   exact residual 1 - g r (P. Markstein, IBM J. Res. Dev. 34, 111 (1990)).
-__device__ inline void sqrt_and_inverse(double x, double& root, double& inv) {
-  const unsigned hi = (unsigned)__double2hiint(x);
-  if (__builtin_expect(hi - 0x33700000u >= 0x19000000u, 0)) {  // exponent outside [-200, 200), sign or NaN
-    root = sqrt(x);
-    inv = 1. / root;
-    return;
-  }
-  const double y = __builtin_amdgcn_rsq(x);
-  double g = x * y, h = 0.5 * y;
-  double e = fma(-h, g, 0.5);
-  g = fma(g, e, g);
-  h = fma(h, e, h);
-  e = fma(-g, g, x);
-  g = fma(e, h, g);
-  e = fma(-g, g, x);
-  g = fma(e, h, g);
-  double r = h + h;
-  e = fma(-g, r, 1.0);
-  r = fma(e, r, r);
-  e = fma(-g, r, 1.0);
-  r = fma(e, r, r);
-  root = g;
-  inv = r;
+  // combined here: sums that only a later block uses would sink into it and
+  // leave their terms live until then
+  asm volatile("" : "+v"(fl[0]), "+v"(fl[1]), "+v"(fl[2]), "+v"(fl[3]), "+v"(fl[4]), "+v"(fl[5]));
 }
 
 // Buneman-Boris push of one particle in cell (i, j) (particle.f90:98-163),

@@ -30,8 +30,6 @@ struct Push3Args {
   const int* colbase;
   const int* cumcnt;
   const int* ap;  // A's slot -> record in A's buffer (null: identity)
-  int* nov;       // fused fast kernel: count of the overflow list below
-  int *ovslot, *ovcell;
   const double* uf;
   double* uj;
   double* pjbuf;
@@ -43,7 +41,7 @@ struct Push3Args {
 
 __global__ __launch_bounds__(p3::NT) void k_push3d(Push3Args a) {
   using namespace p3;
-  __shared__ double sf[6][SN];
+  __shared__ FieldTile3 sf;
   const Grid3D& g = a.g;
   const int ntiles = a.ntx * a.nty * a.ntz;
   const int tile = xcd_tile(blockIdx.x, ntiles);
@@ -51,16 +49,12 @@ __global__ __launch_bounds__(p3::NT) void k_push3d(Push3Args a) {
   int i0, j0, k0;
   tile_origin(g, tile, a.ntx, a.nty, i0, j0, k0);
   const int tid = threadIdx.x;
-  for (int q = tid; q < 6 * SN; q += NT) {
-    const int c = q / SN, rem = q - c * SN;
-    const int i = i0 - 1 + rem % SW, j = j0 - 1 + (rem / SW) % SH, k = k0 - 1 + rem / (SW * SH);
-    if (i <= g.nxge + 1 && j <= g.nye + 1 && k <= g.nze + 1) sf[c][rem] = tmpf3(g, a.uf, c, i, j, k);
-  }
+  stage_fields3(g, a.uf, sf, i0, j0, k0);
   __syncthreads();
 
   const int grp = tid / G, lg = tid % G;
   constexpr int NGRP = NT / G;
-  const double d_delx = g.d_delx, delt = g.delt, c = g.c;
+  const double delt = g.delt, c = g.c;
   for (int cc = grp; cc < TX * TY * TZ; cc += NGRP) {
     const int li = cc % TX, lj = (cc / TX) % TY, lk = cc / (TX * TY);
     const int i = i0 + li, j = j0 + lj, k = k0 + lk;
@@ -77,22 +71,15 @@ __global__ __launch_bounds__(p3::NT) void k_push3d(Push3Args a) {
       const double fac2 = q * delt / rm;
       for (int pi = pbeg + lg; pi < pend; pi += G) {
         const int ia = a.ap ? a.ap[pi] : pi;
-        const double x = a.A.x[ia], y = a.A.y[ia], z = a.A.z[ia];
-        double nxp, nyp, nzp, g4, g5, g6, sh[9];
+        const Rec3 p = load_rec(a.A, ia);
+        double nxp, nyp, nzp, g4, g5, g6;
         const int so = (lk + 1) * (SW * SH) + (lj + 1) * SW + (li + 1);
         if (a.vay)
-          vay_push3(sf, so, i, j, k, d_delx, delt, c, fac1, fac2, x, y, z, a.A.ux[ia], a.A.uy[ia], a.A.uz[ia], nxp,
-                    nyp, nzp, g4, g5, g6, sh);
+          vay_push3(sf, so, i, j, k, delt, c, fac1, fac2, p.x, p.y, p.z, p.ux, p.uy, p.uz, nxp, nyp, nzp, g4, g5, g6);
         else
-          boris_push3(sf, so, i, j, k, d_delx, delt, c, fac1, txxx, fac2, x, y, z, a.A.ux[ia], a.A.uy[ia],
-                      a.A.uz[ia], nxp, nyp, nzp, g4, g5, g6, sh);
-        a.B.x[pi] = nxp;
-        a.B.y[pi] = nyp;
-        a.B.z[pi] = nzp;
-        a.B.ux[pi] = g4;
-        a.B.uy[pi] = g5;
-        a.B.uz[pi] = g6;
-        a.B.id[pi] = a.A.id[ia];  // particle.f90:227-231
+          boris_push3(sf, so, i, j, k, delt, c, fac1, txxx, fac2, p.x, p.y, p.z, p.ux, p.uy, p.uz, nxp, nyp, nzp, g4,
+                      g5, g6);
+        store_rec(a.B, pi, Rec3{nxp, nyp, nzp, g4, g5, g6, p.id});  // particle.f90:227-231
       }
     }
   }
@@ -325,168 +312,134 @@ __global__ __launch_bounds__(256) void k_gather_pj3d(Grid3D g, const double* __r
   uj[2 * n + q] = sz;
 }
 
-// Current of one particle that changes cell (field.f90:253-380, factored as
-// below): the 4-node window [lo, lo+3] (of the 5 nodes -2..2) per axis holds
-// every non-zero s0 and ds when |inc| <= 1; smo_* as field.f90:258-266.
-// add(comp, xo, yo, zo, v) receives each non-zero value with its node offset
-// from the particle's cell (i, j, k).
-template <class Add>
-__device__ inline void deposit3_window(const Grid3D& g, const Parts3& A, const Parts3& B, const int* ap, int pc,
-                                       const int cell[3], double qd, Add add) {
-  const int ia = ap ? ap[pc] : pc;
-  const double old[3] = {A.x[ia], A.y[ia], A.z[ia]};
-  const double nw[3] = {B.x[pc], B.y[pc], B.z[pc]};
-  const double d_delx = g.d_delx;
-  double S0[3][4], DS[3][4], cq[3][3];
-  int lo[3];
+// Current of one particle that changes cell, in the factored form of
+// k_push_deposit3d_fast, from its old and new in-cell shape arguments
+// (x - 0.5 - cell per axis, field.f90:253-266) and its cell increments, added
+// to the LDS tile: o is the tile's Jx at the particle's cell.  The 4-node
+// window [lo, lo + 3] of the 5 nodes -2..2 per axis, lo = 0 for a step to the
+// left and 1 otherwise, holds every non-zero s0 and ds when |inc| <= 1.  An
+// axis along which the particle keeps its cell has nothing on its fourth node
+// and only rounding on its third face, so a step along one axis costs 75
+// atomics and one along all three 144.
+__device__ inline void deposit3_window(double* o, const double dh0[3], const double dh1[3], const int inc[3],
+                                       double qd) {
+  using namespace p3;
+  constexpr int SY = AW, SZ = AW * AH;
+  double S[3][4], D[3][4], cq[3][3];
+  bool mv[3];
 #pragma unroll
   for (int d = 0; d < 3; d++) {
-    double s0m, s00, s0p, s11, s12, s13;
-    shape3(old[d] * d_delx - 5e-1 - cell[d], s0m, s00, s0p);
-    const int i2 = (int)(nw[d] * d_delx);
-    const double dh = nw[d] * d_delx - 5e-1 - i2;
-    const int in = i2 - cell[d];
-    shape3(dh, s11, s12, s13);
-    const double smo1 = in < 0 ? (double)(-in) : 0.0;
-    const double smo2 = (double)(-abs(in) + 1);
-    const double smo3 = in > 0 ? (double)in : 0.0;
-    const double f0 = s11 * smo1 - 0e0;
-    const double f1 = s11 * smo2 + s12 * smo1 - s0m;
-    const double f2 = s12 * smo2 + s13 * smo1 + s11 * smo3 - s00;
-    const double f3 = s13 * smo2 + s12 * smo3 - s0p;
-    const double f4 = s13 * smo3 - 0e0;
-    const bool left = in < 0;
-    lo[d] = left ? 0 : 1;
-    S0[d][0] = left ? 0.0 : s0m;
-    S0[d][1] = left ? s0m : s00;
-    S0[d][2] = left ? s00 : s0p;
-    S0[d][3] = left ? s0p : 0.0;
-    DS[d][0] = left ? f0 : f1;
-    DS[d][1] = left ? f1 : f2;
-    DS[d][2] = left ? f2 : f3;
-    DS[d][3] = left ? f3 : f4;
+    double t0, t1, t2, u0, u1, u2;
+    shape3(dh0[d], t0, t1, t2);
+    shape3(dh1[d], u0, u1, u2);
+    const bool left = inc[d] < 0, right = inc[d] > 0;
+    mv[d] = left || right;
+    o += (left ? -2 : -1) * (d == 0 ? 1 : (d == 1 ? SY : SZ));  // window node 0 of the axis
+    S[d][0] = left ? 0.0 : t0;
+    S[d][1] = left ? t0 : t1;
+    S[d][2] = left ? t1 : t2;
+    S[d][3] = left ? t2 : 0.0;
+    D[d][0] = (right ? 0.0 : u0) - S[d][0];
+    D[d][1] = (right ? u0 : u1) - S[d][1];
+    D[d][2] = (right ? u1 : u2) - S[d][2];
+    D[d][3] = (right ? u2 : 0.0) - S[d][3];
     double run = 0.0;
 #pragma unroll
     for (int m = 0; m < 3; m++) {
-      run = run - DS[d][m];
+      run = run - D[d][m];
       cq[d][m] = run * qd;
     }
   }
-  // window node u of an axis is node lo + u - 2 of the cell; face m lies
-  // between window nodes m and m + 1, at offset lo + m - 1
+  // face m lies between window nodes m and m + 1, at the offset of node m + 1
+  // (the barriers keep the compiler from forming all the products first)
 #pragma unroll
-  for (int u = 0; u < 4; u++) {
-    const double ax = fma(0.5, DS[0][u], S0[0][u]), bxu = fma(1.0 / 3.0, DS[0][u], 0.5 * S0[0][u]);
-    const double ay = fma(0.5, DS[1][u], S0[1][u]), byu = fma(1.0 / 3.0, DS[1][u], 0.5 * S0[1][u]);
+  for (int v = 0; v < 4; v++) {  // z node
+    if (v == 3 && !mv[2]) break;
+    const double Sz = S[2][v], Dz = D[2][v], az = fma(0.5, Dz, Sz), bz = fma(1.0 / 3.0, Dz, 0.5 * Sz);
+    double* const r = o + v * SZ;
 #pragma unroll
-    for (int v = 0; v < 4; v++) {
-      const double wx = fma(ay, S0[2][v], byu * DS[2][v]);  // y node u, z node v
-      const double wy = fma(ax, S0[2][v], bxu * DS[2][v]);  // x node u, z node v
-      const double wz = fma(ax, S0[1][v], bxu * DS[1][v]);  // x node u, y node v
+    for (int u = 0; u < 4; u++) {  // y node of Jx
+      if (u == 3 && !mv[1]) break;
+      const double w = fma(S[1][u], az, D[1][u] * bz);
+      atomicAdd(r + u * SY + 1, cq[0][0] * w);
+      atomicAdd(r + u * SY + 2, cq[0][1] * w);
+      if (mv[0]) atomicAdd(r + u * SY + 3, cq[0][2] * w);
+      __builtin_amdgcn_sched_barrier(0);
+    }
 #pragma unroll
-      for (int m = 0; m < 3; m++) {
-        const double vx = cq[0][m] * wx, vy = cq[1][m] * wy, vz = cq[2][m] * wz;
-        if (vx != 0.0) add(0, lo[0] + m - 1, lo[1] + u - 2, lo[2] + v - 2, vx);
-        if (vy != 0.0) add(1, lo[0] + u - 2, lo[1] + m - 1, lo[2] + v - 2, vy);
-        if (vz != 0.0) add(2, lo[0] + u - 2, lo[1] + v - 2, lo[2] + m - 1, vz);
-      }
+    for (int u = 0; u < 4; u++) {  // x node of Jy
+      if (u == 3 && !mv[0]) break;
+      const double w = fma(S[0][u], az, D[0][u] * bz);
+      atomicAdd(r + AN + u + SY, cq[1][0] * w);
+      atomicAdd(r + AN + u + 2 * SY, cq[1][1] * w);
+      if (mv[1]) atomicAdd(r + AN + u + 3 * SY, cq[1][2] * w);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+#pragma unroll
+  for (int v = 0; v < 4; v++) {  // y node of Jz
+    if (v == 3 && !mv[1]) break;
+    const double Sy = S[1][v], Dy = D[1][v], ay = fma(0.5, Dy, Sy), by = fma(1.0 / 3.0, Dy, 0.5 * Sy);
+#pragma unroll
+    for (int u = 0; u < 4; u++) {  // x node
+      if (u == 3 && !mv[0]) break;
+      const double w = fma(S[0][u], ay, D[0][u] * by);
+      double* const r = o + 2 * AN + v * SY + u;
+      atomicAdd(r + SZ, cq[2][0] * w);
+      atomicAdd(r + 2 * SZ, cq[2][1] * w);
+      if (mv[2]) atomicAdd(r + 3 * SZ, cq[2][2] * w);
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
 }
 
-// The same window from the particle's old and new in-cell shape arguments
-// (dh = x/dx - 0.5 - cell per axis, field.f90:253-266) and its cell increments.
-template <class Add>
-__device__ inline void deposit3_window_dh(const double dh0[3], const double dh1[3], const int inc[3], double qd,
-                                          Add add) {
-  double S0[3][4], DS[3][4], cq[3][3];
-  int lo[3];
-#pragma unroll
-  for (int d = 0; d < 3; d++) {
-    double s0m, s00, s0p, s11, s12, s13;
-    shape3(dh0[d], s0m, s00, s0p);
-    shape3(dh1[d], s11, s12, s13);
-    const int in = inc[d];
-    const double smo1 = in < 0 ? (double)(-in) : 0.0;
-    const double smo2 = (double)(-abs(in) + 1);
-    const double smo3 = in > 0 ? (double)in : 0.0;
-    const double f0 = s11 * smo1 - 0e0;
-    const double f1 = s11 * smo2 + s12 * smo1 - s0m;
-    const double f2 = s12 * smo2 + s13 * smo1 + s11 * smo3 - s00;
-    const double f3 = s13 * smo2 + s12 * smo3 - s0p;
-    const double f4 = s13 * smo3 - 0e0;
-    const bool left = in < 0;
-    lo[d] = left ? 0 : 1;
-    S0[d][0] = left ? 0.0 : s0m;
-    S0[d][1] = left ? s0m : s00;
-    S0[d][2] = left ? s00 : s0p;
-    S0[d][3] = left ? s0p : 0.0;
-    DS[d][0] = left ? f0 : f1;
-    DS[d][1] = left ? f1 : f2;
-    DS[d][2] = left ? f2 : f3;
-    DS[d][3] = left ? f3 : f4;
-    double run = 0.0;
-#pragma unroll
-    for (int m = 0; m < 3; m++) {
-      run = run - DS[d][m];
-      cq[d][m] = run * qd;
-    }
-  }
-#pragma unroll
-  for (int u = 0; u < 4; u++) {
-    const double ax = fma(0.5, DS[0][u], S0[0][u]), bxu = fma(1.0 / 3.0, DS[0][u], 0.5 * S0[0][u]);
-    const double ay = fma(0.5, DS[1][u], S0[1][u]), byu = fma(1.0 / 3.0, DS[1][u], 0.5 * S0[1][u]);
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-      const double wx = fma(ay, S0[2][v], byu * DS[2][v]);  // y node u, z node v
-      const double wy = fma(ax, S0[2][v], bxu * DS[2][v]);  // x node u, z node v
-      const double wz = fma(ax, S0[1][v], bxu * DS[1][v]);  // x node u, y node v
-#pragma unroll
-      for (int m = 0; m < 3; m++) {
-        const double vx = cq[0][m] * wx, vy = cq[1][m] * wy, vz = cq[2][m] * wz;
-        if (vx != 0.0) add(0, lo[0] + m - 1, lo[1] + u - 2, lo[2] + v - 2, vx);
-        if (vy != 0.0) add(1, lo[0] + u - 2, lo[1] + m - 1, lo[2] + v - 2, vy);
-        if (vz != 0.0) add(2, lo[0] + u - 2, lo[1] + v - 2, lo[2] + m - 1, vz);
-      }
-    }
-  }
-}
-
-// Fast mode, push and deposit in one pass over each particle.  The push is the
-// shared bit-exact boris_push3; the deposit uses the factored weights of
-// k_deposit3d's fast path,
-//   Jx(m, j, k) += cx(m) (ay(j) s0z(k) + by(j) dsz(k)),  cx(m) = -sum_{n<=m} dsx(n),
-//   ay = s0y + dsy/2,  by = s0y/2 + dsy/3,
+// Fast mode, push and deposit in one kernel.  The push is the shared bit-exact
+// boris_push3; the deposit uses the factored weights of k_deposit3d's fast path,
+//   Jx(m, j, k) += cx(m) (s0y(j) az(k) + dsy(j) bz(k)),  cx(m) = -sum_{n<=m} dsx(n),
+//   az = s0z + dsz/2,  bz = s0z/2 + dsz/3,
 // and Jy, Jz with the axes permuted (field.f90:335-380 expanded term by term).
 // A particle that stays in its cell along every axis has ds = 0 on the outer
 // nodes and cx = 0 on the outer faces (the last one up to rounding), so its
-// current lives on 2 x 3 x 3 nodes per component: every lane accumulates
-// those 54 values in registers over the particles of the cell it handles and
-// the lane group reduces them once per cell.  A particle that changes cell is
-// queued in LDS, private to the wave; after the wave's cells of a round, its
-// lanes add the queued particles' 3 x 4 x 4 windows per component
-// (deposit3_window) to the LDS tile.  The tile is added to uj with one HBM
-// atomic per node.
+// current lives on 2 x 3 x 3 nodes per component: every lane sums those 54
+// values over the particles it handles and the lane group adds them up.  A
+// particle that changes cell is queued in its wave's LDS queue; whenever 64
+// have gathered, over as many passes and cells as that takes, all the wave's
+// lanes add one particle's window each (deposit3_window) to the LDS tile.  The
+// tile is added to uj with one HBM atomic per node.
+//
+// Work mapping: wave w walks row w of each of the tile's four layers, 8 cells
+// of 8 lanes, each lane every eighth particle of its cell (all species as one
+// list) with the two-deep load pipeline of the 2D kernel.  Up to KP passes
+// push and leave their particles' six shape arguments in registers, then the
+// 54 sums are formed from those: kept over the pushes themselves, next to the
+// gather's 16-byte reads in flight, the sums spilled (10.0 ms, half of it
+// scratch traffic).
+//
+// What bounds it (160x144x128, 2 species of 16 ppc, 94 M particles): VALU
+// issue in 71 % of the cycles at 2 waves a SIMD; 12.9 GB of traffic (11.3
+// algorithmic) in 6.1 ms.  One pass with the sums kept, one array per field,
+// single LDS reads and per-round queues took 8.2 ms.  KP = 3, 4, 5, 6: 6.2,
+// 6.2, 6.1, 6.2 ms.
 namespace p3f {
 constexpr int G = 8;     // lanes per cell
-constexpr int QW = 128;  // queued cell-changing particles per wave and round (beyond: a global list)
-}
+constexpr int KP = 5;    // passes between two deposits of what stays
+constexpr int QW = 128;  // queued cell-changing particles per wave: 63 left over and 64 of a pass at most
+}  // namespace p3f
 
 template <bool VAY>
 __global__ __launch_bounds__(p3::NT, 2) void k_push_deposit3d_fast(Push3Args a) {
   using namespace p3;
-  constexpr int GF = p3f::G;
-  __shared__ double sf[6][SN];
+  constexpr int GF = p3f::G, NW = NT / 64;
+  using p3f::QW;
+  using p3f::KP;
+  static_assert(64 / GF == TX && NW == TY, "a wave takes a row of the tile at a time");
+  __shared__ FieldTile3 sf;
   __shared__ double acc[3][AN];
   __shared__ double spc[WPIC_MAXSP][4];  // fac1, txxx, fac2, q delx / delt
-  // each wave's cell-changing particles of the round: old and new shape
-  // arguments per axis, and cell in the tile | species << 7 | (inc + 1) per
-  // axis << 9, 11, 13
-  constexpr int NW = NT / 64;
-  using p3f::QW;
-  __shared__ double xqd[NW][QW][6];
+  // the waves' queued particles: old and new shape arguments per axis, and
+  // cell in the tile | species << 7 | (inc + 1) per axis << 9, 11, 13
+  __shared__ double xqd[NW][6][QW];
   __shared__ int xqc[NW][QW];
-  __shared__ int nxq[NW];
   const Grid3D& g = a.g;
   const int ntiles = a.ntx * a.nty * a.ntz;
   const int tile = xcd_tile(blockIdx.x, ntiles);
@@ -494,13 +447,8 @@ __global__ __launch_bounds__(p3::NT, 2) void k_push_deposit3d_fast(Push3Args a) 
   int i0, j0, k0;
   tile_origin(g, tile, a.ntx, a.nty, i0, j0, k0);
   const int tid = threadIdx.x;
-  for (int q = tid; q < 6 * SN; q += NT) {
-    const int c = q / SN, rem = q - c * SN;
-    const int i = i0 - 1 + rem % SW, j = j0 - 1 + (rem / SW) % SH, k = k0 - 1 + rem / (SW * SH);
-    if (i <= g.nxge + 1 && j <= g.nye + 1 && k <= g.nze + 1) sf[c][rem] = tmpf3(g, a.uf, c, i, j, k);
-  }
+  stage_fields3(g, a.uf, sf, i0, j0, k0);
   for (int q = tid; q < 3 * AN; q += NT) (&acc[0][0])[q] = 0.0;
-  if (tid < NW) nxq[tid] = 0;
 #pragma unroll
   for (int s = 0; s < WPIC_MAXSP; s++) {
     if (tid == s && s < g.nsp) {
@@ -514,214 +462,208 @@ __global__ __launch_bounds__(p3::NT, 2) void k_push_deposit3d_fast(Push3Args a) 
   }
   __syncthreads();
 
-  const int grp = tid / GF, lg = tid % GF;
-  constexpr int NGRP = NT / GF;
-  const double d_delx = g.d_delx, delt = g.delt, c = g.c;
-  const int w = tid >> 6, lane = tid & 63;
-  int* const nq_r = &nxq[w];
-  // rounds of NGRP cells (one per group, 64 / G per wave), each wave
-  // draining its own queue after its cells of the round
-  for (int rnd = 0; rnd < (TX * TY * TZ) / NGRP; rnd++) {
-    const int cc = rnd * NGRP + grp;
-    const int li = cc % TX, lj = (cc / TX) % TY, lk = cc / (TX * TY);
-    const int i = i0 + li, j = j0 + lj, k = k0 + lk;
-    if (i <= g.nxge && j <= g.nye && k <= g.nze) {  // uniform within a group
-    const int col = (j - g.nys) + g.ny * (k - g.nzs);
+  // (the wave's number, the same in its lanes, and with it j and k stay in
+  // scalar registers)
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, lg = lane % GF;
+  const int li = lane / GF, lj = w;
+  const int i = i0 + li, j = j0 + lj;
+  int nq = 0;  // queued particles, the same in all lanes
+
+  // the currents of the last (at most 64) queued particles
+  auto drain = [&]() {
+    // written by this wave's own lanes: LDS operations of one wave complete in order
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const int n0 = nq > 64 ? nq - 64 : 0, q = n0 + lane;
+    if (q < nq) {
+      const int e = xqc[w][q];
+      const int cc = e & 127, s = (e >> 7) & 3;
+      const int inc[3] = {((e >> 9) & 3) - 1, ((e >> 11) & 3) - 1, ((e >> 13) & 3) - 1};
+      const double dh0[3] = {xqd[w][0][q], xqd[w][1][q], xqd[w][2][q]};
+      const double dh1[3] = {xqd[w][3][q], xqd[w][4][q], xqd[w][5][q]};
+      deposit3_window(&acc[0][((cc / (TX * TY) + 2) * AH + (cc / TX % TY + 2)) * AW + (cc % TX + 2)], dh0, dh1, inc,
+                      spc[s][3]);
+    }
+    nq = n0;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+
+  for (int lk = 0; lk < TZ; lk++) {
+    const int k = k0 + lk;
+    const bool live = i <= g.nxge && j <= g.nye && k <= g.nze;  // uniform within a group
     CellList cl;
-    int ntot = 0;
+    int tot = 0;
 #pragma unroll
     for (int s = 0; s < WPIC_MAXSP; s++) {
       if (s < g.nsp) {
-        const int rw = s * g.ncol + col;
-        const int* cr = a.cumcnt + (size_t)rw * (g.nx + 1);
-        const int c0 = cr[i - g.nxgs], c1 = cr[i - g.nxgs + 1];
-        cl.set(s, a.colbase[rw] + c0, ntot);
-        ntot += c1 - c0;
+        int c0 = 0, c1 = 0, cb = 0;
+        if (live) {
+          const int rw = s * g.ncol + (j - g.nys) + g.ny * (k - g.nzs);
+          const int* cr = a.cumcnt + (size_t)rw * (g.nx + 1) + (i - g.nxgs);
+          c0 = cr[0];
+          c1 = cr[1];
+          cb = a.colbase[rw];
+        }
+        cl.set(s, cb + c0, tot);
+        tot += c1 - c0;
       } else {
         cl.set(s, 0, 0x7fffffff);
       }
     }
-    // stayers' current: [m][a][b] with m the face (offset m along the
-    // component's axis) and a, b the nodes (offsets a-1, b-1) of the other two
-    // axes in the order (y, z) for Jx, (x, z) for Jy, (x, y) for Jz
-    double jx[18], jy[18], jz[18];
-#pragma unroll
-    for (int q = 0; q < 18; q++) jx[q] = jy[q] = jz[q] = 0.0;
     const int so = (lk + 1) * (SW * SH) + (lj + 1) * SW + (li + 1);
-    const int bx = li + 2, by = lj + 2, bz = lk + 2;  // the cell in the current tile
 
-    // two-deep load pipeline: the record of element t + G and the
-    // permutation entry of element t + 2G are in flight while element t is
-    // pushed
     int ia_nn = 0;
-    double px = 0.0, py = 0.0, pz = 0.0, pux = 0.0, puy = 0.0, puz = 0.0;
-    uint64_t pid = 0;
+    // (a cell's surplus lanes push a particle at rest at its centre)
+    Rec3 pr = {i + 0.5, j + 0.5, k + 0.5, 0.0, 0.0, 0.0, 0};
     {
       int s_, p_, ia_n = 0;
-      if (lg < ntot) {
+      if (lg < tot) {
         cl.slot(g.nsp, lg, s_, p_);
         ia_n = a.ap ? a.ap[p_] : p_;
       }
-      if (lg + GF < ntot) {
+      if (lg + GF < tot) {
         cl.slot(g.nsp, lg + GF, s_, p_);
         ia_nn = a.ap ? a.ap[p_] : p_;
       }
-      if (lg < ntot) {
-        px = a.A.x[ia_n]; py = a.A.y[ia_n]; pz = a.A.z[ia_n];
-        pux = a.A.ux[ia_n]; puy = a.A.uy[ia_n]; puz = a.A.uz[ia_n];
-        pid = a.A.id[ia_n];
-      }
+      if (lg < tot) pr = load_rec(a.A, ia_n);
     }
-    for (int t = lg; t < ntot; t += GF) {
-      int sc, pc;
-      cl.slot(g.nsp, t, sc, pc);
-      const double x = px, y = py, z = pz, ux = pux, uy = puy, uz = puz;
-      const uint64_t id = pid;
-      if (t + GF < ntot) {
-        const int ia = ia_nn;
-        px = a.A.x[ia]; py = a.A.y[ia]; pz = a.A.z[ia];
-        pux = a.A.ux[ia]; puy = a.A.uy[ia]; puz = a.A.uz[ia];
-        pid = a.A.id[ia];
-      }
-      if (t + 2 * GF < ntot) {
+    // KP passes at a time: the pushes, one straight line for all lanes as in 2D
+    // (a lane past its cell's last particle repeats one with zero charge and
+    // stores nothing), then the current of those that stay
+    int t = lg;
+    while (__any(t < tot)) {
+    double pd[KP][6];  // old and new shape arguments of the last KP passes, the latest first
+    int ps[KP];    // species, or -1: no current from it
+#pragma unroll
+    for (int h = 0; h < KP; h++) {
+      ps[h] = -1;
+#pragma unroll
+      for (int d = 0; d < 6; d++) pd[h][d] = 0.0;
+    }
+    for (int h = 0; h < KP && __any(t < tot); h++, t += GF) {
+      const bool act = t < tot;
+      int s, pi;
+      cl.slot(g.nsp, t, s, pi);
+      const Rec3 cur = pr;
+      if (t + GF < tot) pr = load_rec(a.A, ia_nn);
+      if (t + 2 * GF < tot) {
         int s_, p_;
         cl.slot(g.nsp, t + 2 * GF, s_, p_);
         ia_nn = a.ap ? a.ap[p_] : p_;
       }
-      const double* kc = spc[sc];
-      double nw[3], g4, g5, g6, sh[9];
+      const double* kc = spc[s];
+      const double x = cur.x, y = cur.y, z = cur.z;
+      double nxp, nyp, nzp, g4, g5, g6;
       if (VAY)
-        vay_push3(sf, so, i, j, k, d_delx, delt, c, kc[0], kc[2], x, y, z, ux, uy, uz, nw[0], nw[1], nw[2], g4, g5,
-                  g6, sh);
+        vay_push3(sf, so, i, j, k, g.delt, g.c, kc[0], kc[2], x, y, z, cur.ux, cur.uy, cur.uz, nxp, nyp, nzp, g4, g5,
+                  g6);
       else
-        boris_push3(sf, so, i, j, k, d_delx, delt, c, kc[0], kc[1], kc[2], x, y, z, ux, uy, uz, nw[0], nw[1], nw[2],
-                    g4, g5, g6, sh);
-      a.B.ux[pc] = g4;
-      a.B.uy[pc] = g5;
-      a.B.uz[pc] = g6;
-      a.B.id[pc] = id;
-
-      // new shape and cell increment per axis (field.f90:253-329)
-      const double qd = kc[3];
-      const int cell[3] = {i, j, k};
-      double s1[3][3], dh1[3];
-      int inc[3];
+        boris_push3(sf, so, i, j, k, g.delt, g.c, kc[0], kc[1], kc[2], x, y, z, cur.ux, cur.uy, cur.uz, nxp, nyp, nzp,
+                    g4, g5, g6);
+      const int i2 = (int)nxp, j2 = (int)nyp, k2 = (int)nzp;
+      const bool stays = i2 == i && j2 == j && k2 == k;
+      const bool mover = act && !stays;
+      if (act) {
+        // the x wrap, the y-z wraps and the exchange code: particle_x and
+        // particle_yz act on gp after the deposit, which uses the unwrapped
+        // position
+        double wx = nxp, wy = nyp, wz = nzp;
+        int code = ((i2 - g.nxgs) << CODE_SHIFT3) | ((k2 - k + 1) * 3 + (j2 - j + 1));
+        if ((unsigned)(i2 - g.nxgs) >= (unsigned)g.nx || (unsigned)(j2 - g.nys) >= (unsigned)g.ny ||
+            (unsigned)(k2 - g.nzs) >= (unsigned)g.nz || (unsigned)(j2 - j + 1) > 2u || (unsigned)(k2 - k + 1) > 2u) {
+          bool moved;
+          code = wrap3_code<true>(g, wx, wy, wz, j, k, a.err, moved);
+        }
+        a.code[pi] = code;
+        store_rec(a.B, pi, Rec3{wx, wy, wz, g4, g5, g6, cur.id});
+      }
+#pragma unroll
+      for (int q = KP - 1; q > 0; q--) {
+        ps[q] = ps[q - 1];
+#pragma unroll
+        for (int d = 0; d < 6; d++) pd[q][d] = pd[q - 1][d];
+      }
+      ps[0] = act && stays ? s : -1;
+      pd[0][0] = x - 5e-1 - i;
+      pd[0][1] = y - 5e-1 - j;
+      pd[0][2] = z - 5e-1 - k;
+      pd[0][3] = nxp - 5e-1 - i2;
+      pd[0][4] = nyp - 5e-1 - j2;
+      pd[0][5] = nzp - 5e-1 - k2;
+      const uint64_t mm = __ballot(mover);
+      if (mm) {
+        if (mover) {
+          const int slot = nq + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mm >> 32),
+                                                               __builtin_amdgcn_mbcnt_lo((uint32_t)mm, 0));
+#pragma unroll
+          for (int d = 0; d < 6; d++) xqd[w][d][slot] = pd[0][d];
+          xqc[w][slot] = ((lk * TY + lj) * TX + li) | (s << 7) | (((i2 - i + 1) & 3) << 9) |
+                         (((j2 - j + 1) & 3) << 11) | (((k2 - k + 1) & 3) << 13);
+        }
+        nq += __popcll(mm);
+        if (nq >= 64) drain();
+      }
+    }
+    // the current of the particles that stay: sum 18 c + 9 m + 3 u + b of
+    // component c, face m along its own axis, nodes u - 1, b - 1 of the other
+    // two in the order x, y, z
+    double v[54];
+#pragma unroll
+    for (int q = 0; q < 54; q++) v[q] = 0.0;
+#pragma unroll
+    for (int h = 0; h < KP; h++) {
+      if (!__any(ps[h] >= 0)) continue;
+      const double qd = ps[h] >= 0 ? spc[ps[h] & 3][3] : 0.0;
+      double S[3][3], D[3][3], cq[3][2];  // s0, ds = s1 - s0, -sum ds
 #pragma unroll
       for (int d = 0; d < 3; d++) {
-        const int i2 = (int)(nw[d] * d_delx);
-        dh1[d] = nw[d] * d_delx - 5e-1 - i2;
-        inc[d] = i2 - cell[d];
-        shape3(dh1[d], s1[d][0], s1[d][1], s1[d][2]);
+        double t0, t1, t2;
+        shape3(pd[h][d], S[d][0], S[d][1], S[d][2]);
+        shape3(pd[h][3 + d], t0, t1, t2);
+        D[d][0] = t0 - S[d][0];
+        D[d][1] = t1 - S[d][1];
+        D[d][2] = t2 - S[d][2];
+        cq[d][0] = (0.0 - D[d][0]) * qd;
+        cq[d][1] = ((0.0 - D[d][0]) - D[d][1]) * qd;
       }
-      bool over = false;
-      if ((inc[0] | inc[1] | inc[2]) == 0) {
-        // nodes -1..1 of each axis: s0, ds = s1 - s0, a = s0 + ds/2, b = s0/2 + ds/3
-        double s0[3][3], ds[3][3], A[3][3], B[3][3], cq[3][2];
 #pragma unroll
-        for (int d = 0; d < 3; d++) {
+      for (int b = 0; b < 3; b++) {
+        const double az = fma(0.5, D[2][b], S[2][b]), bz = fma(1.0 / 3.0, D[2][b], 0.5 * S[2][b]);
+        const double ay = fma(0.5, D[1][b], S[1][b]), by = fma(1.0 / 3.0, D[1][b], 0.5 * S[1][b]);
 #pragma unroll
-          for (int n = 0; n < 3; n++) {
-            s0[d][n] = sh[3 * d + n];
-            ds[d][n] = s1[d][n] - s0[d][n];
-            A[d][n] = fma(0.5, ds[d][n], s0[d][n]);
-            B[d][n] = fma(1.0 / 3.0, ds[d][n], 0.5 * s0[d][n]);
+        for (int u = 0; u < 3; u++) {
+          const double wx = fma(S[1][u], az, D[1][u] * bz);  // y node u, z node b
+          const double wy = fma(S[0][u], az, D[0][u] * bz);  // x node u, z node b
+          const double wz = fma(S[0][u], ay, D[0][u] * by);  // x node u, y node b
+#pragma unroll
+          for (int m = 0; m < 2; m++) {
+            const int q = 9 * m + 3 * u + b;
+            v[q] = fma(cq[0][m], wx, v[q]);
+            v[18 + q] = fma(cq[1][m], wy, v[18 + q]);
+            v[36 + q] = fma(cq[2][m], wz, v[36 + q]);
           }
-          cq[d][0] = (0.0 - ds[d][0]) * qd;
-          cq[d][1] = ((0.0 - ds[d][0]) - ds[d][1]) * qd;
-        }
-#pragma unroll
-        for (int u = 0; u < 3; u++)
-#pragma unroll
-          for (int v = 0; v < 3; v++) {
-            const double wx = fma(A[1][u], s0[2][v], B[1][u] * ds[2][v]);  // y node u, z node v
-            const double wy = fma(A[0][u], s0[2][v], B[0][u] * ds[2][v]);  // x node u, z node v
-            const double wz = fma(A[0][u], s0[1][v], B[0][u] * ds[1][v]);  // x node u, y node v
-#pragma unroll
-            for (int m = 0; m < 2; m++) {
-              const int q = (m * 3 + u) * 3 + v;
-              jx[q] = fma(cq[0][m], wx, jx[q]);
-              jy[q] = fma(cq[1][m], wy, jy[q]);
-              jz[q] = fma(cq[2][m], wz, jz[q]);
-            }
-          }
-      } else {
-        // a particle that changes cell: its window is added after the cell loop
-        const int slot = wave_enqueue(nq_r);
-        if (slot < QW) {
-          const double o[3] = {x, y, z};
-#pragma unroll
-          for (int d = 0; d < 3; d++) {
-            xqd[w][slot][d] = o[d] * d_delx - 5e-1 - cell[d];
-            xqd[w][slot][3 + d] = dh1[d];
-          }
-          xqc[w][slot] = cc | (sc << 7) | ((inc[0] + 1) << 9) | ((inc[1] + 1) << 11) | ((inc[2] + 1) << 13);
-        } else {
-          // beyond the LDS queue: listed for k_deposit3d_overflow, which
-          // reads its new position unwrapped and wraps it after the deposit
-          const int o = atomicAdd(a.nov, 1);
-          a.ovslot[o] = pc;
-          a.ovcell[o] = (int)cidx3(g, i, j, k) | (sc << 28);
-          over = true;
         }
       }
-      // the x wrap, the y-z wraps and the exchange code: particle_x and
-      // particle_yz act on gp after the deposit, which uses nw unwrapped
-      double wx = nw[0], wy = nw[1], wz = nw[2];
-      if (!over) {
-        bool moved;
-        a.code[pc] = wrap3_code<true>(g, wx, wy, wz, j, k, a.err, moved);
-      }
-      a.B.x[pc] = wx;
-      a.B.y[pc] = wy;
-      a.B.z[pc] = wz;
-
     }
-    // reduce the stayers' current over the group, spread the LDS atomics
+    // over the group, spread over its lanes
+    group_reduce<54, GF>(v, lane);
+    // (the places are worked out here: kept over the passes they would spill)
+    int ln = lane;
+    asm volatile("" : "+v"(ln));
+    double* const o = &acc[0][0] + ((lk + 2) * AH + (lj + 2)) * AW + (li + 2);
 #pragma unroll
-    for (int q = 0; q < 54; q++) {
-      double v = q < 18 ? jx[q] : (q < 36 ? jy[q - 18] : jz[q - 36]);
-      static_assert(GF == 8, "the group is one half of a DPP row");
-      v = row8_sum(v);
-      if ((q % GF) == lg && v != 0.0) {
-        const int comp = q / 18, r = q % 18, m = r / 9, u = (r / 3) % 3, b = r % 3;
-        int xo, yo, zo;
-        if (comp == 0) {
-          xo = m; yo = u - 1; zo = b - 1;
-        } else if (comp == 1) {
-          xo = u - 1; yo = m; zo = b - 1;
-        } else {
-          xo = u - 1; yo = b - 1; zo = m;
-        }
-        atomicAdd(&acc[comp][((bz + zo) * AH + (by + yo)) * AW + (bx + xo)], v);
-      }
+    for (int f = 0; f < group_left(54, GF); f++) {
+      const int q = group_index<54, GF>(f, ln);
+      const int c = q / 18, m = q % 18 / 9, u = q % 9 / 3 - 1, b = q % 3 - 1;
+      const int xo = c == 0 ? m : u, yo = c == 0 ? u : (c == 1 ? m : b), zo = c == 2 ? m : b;
+      if (live && q >= 0 && v[f] != 0.0) atomicAdd(o + (c * AN + (zo * AH + yo) * AW + xo), v[f]);
     }
-    }  // the cell
-
-    // the wave's queued particles of the round: the queue was written by this
-    // wave's own lanes, and LDS operations of one wave complete in order
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    const int nq = *nq_r < QW ? *nq_r : QW;
-    for (int q = lane; q < nq; q += 64) {
-      const int e = xqc[w][q];
-      const int qcc = e & 127, s = (e >> 7) & 3;
-      const int inc[3] = {((e >> 9) & 3) - 1, ((e >> 11) & 3) - 1, ((e >> 13) & 3) - 1};
-      const int qbx = qcc % TX + 2, qby = (qcc / TX) % TY + 2, qbz = qcc / (TX * TY) + 2;
-      const double dh0[3] = {xqd[w][q][0], xqd[w][q][1], xqd[w][q][2]};
-      const double dh1[3] = {xqd[w][q][3], xqd[w][q][4], xqd[w][q][5]};
-      deposit3_window_dh(dh0, dh1, inc, spc[s][3], [&](int comp, int xo, int yo, int zo, double v) {
-        atomicAdd(&acc[comp][((qbz + zo) * AH + (qby + yo)) * AW + (qbx + xo)], v);
-      });
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    if (lane == 0) *nq_r = 0;
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
+  if (nq) drain();
   __syncthreads();
   const size_t pl = plane3(g);
   for (int q = tid; q < 3 * AN; q += NT) {
@@ -734,34 +676,6 @@ __global__ __launch_bounds__(p3::NT, 2) void k_push_deposit3d_fast(Push3Args a) 
   }
 }
 
-// The cell-changing particles that did not fit a tile's LDS queue, added to
-// uj with HBM atomics (ghost nodes included; the current boundary folds them).
-__global__ __launch_bounds__(256) void k_deposit3d_overflow(Push3Args a) {
-  const Grid3D& g = a.g;
-  const int n = *a.nov;
-  const size_t pl = plane3(g);
-  for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < n; q += gridDim.x * blockDim.x) {
-    const int pc = a.ovslot[q], pk = a.ovcell[q];
-    const int s = pk >> 28, cix = pk & ((1 << 28) - 1);
-    const int cell[3] = {g.nxgs + cix % g.nx, g.nys + (cix / g.nx) % g.ny, g.nzs + cix / (g.nx * g.ny)};
-    double qs = g.q[0];
-#pragma unroll
-    for (int k = 1; k < WPIC_MAXSP; k++)
-      if (s == k) qs = g.q[k];
-    const double qd = qs * g.delx * g.d_delt;
-    deposit3_window(g, a.A, a.B, a.ap, pc, cell, qd, [&](int comp, int xo, int yo, int zo, double v) {
-      unsafeAtomicAdd(a.uj + pl * comp + fidx3(g, cell[0] + xo, cell[1] + yo, cell[2] + zo), v);
-    });
-    // the wraps and the code the fused kernel left to this deposit
-    double x = a.B.x[pc], y = a.B.y[pc], z = a.B.z[pc];
-    bool moved;
-    a.code[pc] = wrap3_code<true>(g, x, y, z, cell[1], cell[2], a.err, moved);
-    a.B.x[pc] = x;
-    a.B.y[pc] = y;
-    a.B.z[pc] = z;
-  }
-}
-
 static Push3Args push_args(wpic_ctx3d* c) {
   Push3Args a;
   a.g = c->g;
@@ -770,8 +684,6 @@ static Push3Args push_args(wpic_ctx3d* c) {
   a.colbase = c->colbaseA;
   a.cumcnt = c->cumcnt;
   a.ap = c->aperm;
-  a.nov = nullptr;
-  a.ovslot = a.ovcell = nullptr;
   a.uf = c->uf;
   a.uj = c->uj;
   a.pjbuf = c->pjbuf;
@@ -801,22 +713,13 @@ hipError_t launch_deposit3d(wpic_ctx3d* c) {
   return hipGetLastError();
 }
 
-__global__ void k_zero_int3(int* p) { *p = 0; }
-
-// The exchange scratch (R, holes) is free between the sort and the next
-// exchange; the fused kernel lists its queue overflow there.
 hipError_t launch_push_deposit3d(wpic_ctx3d* c) {
   Push3Args a = push_args(c);
-  a.nov = c->nov;
-  a.ovslot = c->R;
-  a.ovcell = c->holes;
   const int nblk = xcd_grid(a.ntx * a.nty * a.ntz);
-  hipLaunchKernelGGL(k_zero_int3, dim3(1), dim3(1), 0, c->st, c->nov);
   if (a.vay)
     hipLaunchKernelGGL(k_push_deposit3d_fast<true>, dim3(nblk), dim3(p3::NT), 0, c->st, a);
   else
     hipLaunchKernelGGL(k_push_deposit3d_fast<false>, dim3(nblk), dim3(p3::NT), 0, c->st, a);
-  hipLaunchKernelGGL(k_deposit3d_overflow, dim3(256), dim3(256), 0, c->st, a);
   return hipGetLastError();
 }
 

@@ -477,19 +477,17 @@ int wpic_create3d(wpic_ctx3d** out, const wpic_params3d* p) {
   const size_t N = (size_t)g.ncap * g.nsp;
   const int nr = g.nsp * g.ncol;
   const size_t pl = plane3(g), nc = (size_t)nx * ny * nz;
-  if (c->mixed) {
-    for (PartsM3* m : {&c->MA, &c->MB}) {
-      if (e == hipSuccess) e = dalloc(&m->ix, N);
-      for (float** q : {&m->ox, &m->oy, &m->oz, &m->ux, &m->uy, &m->uz})
-        if (e == hipSuccess) e = dalloc(q, N);
+  for (int k = 0; k < 2 && e == hipSuccess; k++) {
+    if (c->mixed) {
+      float* r = nullptr;
+      e = dalloc(&r, PARTM3_FLOATS * N);
+      (k ? c->MB : c->MA) = partsm3_at(r);
+    } else {
+      double* r = nullptr;
+      e = dalloc(&r, PART3_DOUBLES * N);
+      (k ? c->B : c->A) = parts3_at(r);
     }
-  } else {
-    double** dp[] = {&c->A.x, &c->A.y, &c->A.z, &c->A.ux, &c->A.uy, &c->A.uz,
-                     &c->B.x, &c->B.y, &c->B.z, &c->B.ux, &c->B.uy, &c->B.uz};
-    for (auto q : dp)
-      if (e == hipSuccess) e = dalloc(q, N);
   }
-  for (int k = 0; k < 2 && e == hipSuccess; k++) e = dalloc(&c->id[k], N);
   int** ip[] = {&c->code, &c->R, &c->holes, &c->mlist, &c->permbuf};
   for (auto q : ip)
     if (e == hipSuccess) e = dalloc(q, N);
@@ -517,7 +515,6 @@ int wpic_create3d(wpic_ctx3d** out, const wpic_params3d* p) {
   if (e == hipSuccess) e = dalloc(&c->part, (size_t)3 * NPB3 * 2);
   if (e == hipSuccess) e = dalloc(&c->scal, 3);
   if (e == hipSuccess) e = dalloc(&c->err, 1);
-  if (e == hipSuccess) e = dalloc(&c->nov, 1);
   if (e == hipSuccess) e = dalloc(&c->red, (size_t)256 * 3);
   if (e == hipSuccess) e = hipMemset(c->err, 0, sizeof(int));
   if (e == hipSuccess) e = hipMemset(c->uf, 0, sizeof(double) * 6 * pl);
@@ -535,8 +532,6 @@ int wpic_create3d(wpic_ctx3d** out, const wpic_params3d* p) {
   c->cb = 1;
   c->cn = 2;
   set_cols(c);
-  c->A.id = c->MA.id = c->id[0];
-  c->B.id = c->MB.id = c->id[1];
   for (int k = 0; k < 3; k++) c->h_cols_ok[k] = false;
   *out = c;
   return 0;
@@ -549,14 +544,12 @@ int wpic_destroy3d(wpic_ctx3d* c) {
     if (t.a) (void)hipEventDestroy(t.a);
     if (t.b) (void)hipEventDestroy(t.b);
   }
-  void* ps[] = {c->A.x,    c->A.y,   c->A.z,      c->A.ux,    c->A.uy,   c->A.uz,    c->B.x,    c->B.y,
-                c->B.z,    c->B.ux,  c->B.uy,     c->B.uz,    c->id[0],  c->id[1],   c->code,   c->R,
-                c->holes,  c->mlist, c->cols[0],  c->cols[1], c->cols[2], c->cumcnt, c->dcnt,   c->dstart,
-                c->colkm,  c->csum,  c->seg,   c->nseg,     c->aosbase, c->uf,     c->df,      c->uj,     c->pjbuf,
-                c->phi,    c->pa,    c->pb,       c->rr,      c->bb,     c->ap,      c->part,   c->scal,
-                c->err,    c->staging, c->gbuf,   c->red,     c->permbuf, c->nov,    c->mom,
-                c->MA.ix,  c->MA.ox, c->MA.oy,    c->MA.oz,   c->MA.ux,  c->MA.uy,  c->MA.uz,
-                c->MB.ix,  c->MB.ox, c->MB.oy,    c->MB.oz,   c->MB.ux,  c->MB.uy,  c->MB.uz};
+  void* ps[] = {c->A.x.p,  c->B.x.p,   c->MA.ix.p,  c->MB.ix.p,  c->code,   c->R,      c->holes,
+                c->mlist,  c->cols[0], c->cols[1],  c->cols[2],  c->cumcnt, c->dcnt,   c->dstart,
+                c->colkm,  c->csum,    c->seg,      c->nseg,     c->aosbase, c->uf,    c->df,
+                c->uj,     c->pjbuf,   c->phi,      c->pa,       c->pb,     c->rr,     c->bb,
+                c->ap,     c->part,    c->scal,     c->err,      c->staging, c->gbuf,  c->red,
+                c->permbuf, c->mom};
   for (void* q : ps)
     if (q) (void)hipFree(q);
   if (c->ev_push) (void)hipEventDestroy(c->ev_push);

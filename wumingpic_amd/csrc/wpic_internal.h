@@ -207,6 +207,48 @@ __host__ __device__ inline void shape3(double dh, double& s0, double& s1, double
   s2 = 0.5 * (0.5 + dh) * (0.5 + dh);
 }
 
+// Two staged cell-centred field components side by side: one 16-byte LDS read
+struct alignas(16) FieldPair {
+  double a, b;
+};
+
+// The correctly rounded square root of x and the correctly rounded reciprocal
+// of that root, as sqrt(x) and 1. / sqrt(x) give them.  The compiler's own
+// sequences scale against overflow and handle zeros and infinities, twice
+// over; for x within 2^-200 .. 2^200 none of that is needed and the
+// reciprocal starts from the root's own iterate instead of a new seed.
+//   y ~ 1/sqrt(x) from the hardware; g ~ sqrt(x) and h ~ 1/(2 sqrt(x)) refined
+//   together by Goldschmidt's iteration, then g corrected twice with the exact
+//   residual x - g g (a fused multiply-add), which rounds it correctly; the
+//   reciprocal of g from 2 h by one Newton step and one correction with the
+//   exact residual 1 - g r (P. Markstein, IBM J. Res. Dev. 34, 111 (1990)).
+__device__ inline void sqrt_and_inverse(double x, double& root, double& inv) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  double e = fma(-h, g, 0.5);
+  g = fma(g, e, g);
+  h = fma(h, e, h);
+  e = fma(-g, g, x);
+  g = fma(e, h, g);
+  e = fma(-g, g, x);
+  g = fma(e, h, g);
+  double r = h + h;
+  e = fma(-g, r, 1.0);
+  r = fma(e, r, r);
+  e = fma(-g, r, 1.0);
+  r = fma(e, r, r);
+  root = g;
+  inv = r;
+  // exponent outside [-200, 200), sign or NaN (one branch for the wave: lanes
+  // that part here cost the caller's live registers a copy each)
+  const bool out = (unsigned)__double2hiint(x) - 0x33700000u >= 0x19000000u;
+  if (__builtin_expect(__any(out), 0)) {
+    const double q = sqrt(x);
+    root = out ? q : g;
+    inv = out ? 1. / q : r;
+  }
+}
+
 // The particles of one cell over all species, as one list: element t is slot
 // beg[s] + t - cum[s] of species s, the last s with cum[s] <= t (species
 // beyond nsp carry cum = INT_MAX).  Kept as named scalars and resolved with

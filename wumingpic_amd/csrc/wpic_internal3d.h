@@ -30,19 +30,71 @@ __host__ __device__ inline size_t cidx3(const Grid3D& g, int i, int j, int k) {
 }
 __host__ __device__ inline size_t plane3(const Grid3D& g) { return (size_t)g.fw * g.fh * g.fd; }
 
-// a particle buffer: the record and its id travel together
+// A particle buffer: 56-byte records (x, y, z, ux, uy, uz, id), the
+// reference's own up(:, ii) layout; the id is raw 64 bits.  A record read out
+// of slot order costs the one or two cache lines it lies in instead of one
+// per field, as in 2D.
 struct Parts3 {
-  double *x, *y, *z, *ux, *uy, *uz;
-  uint64_t* id;
+  Col<double, 7> x, y, z, ux, uy, uz;
+  Col<uint64_t, 7> id;
 };
+constexpr int PART3_DOUBLES = 7;
+inline Parts3 parts3_at(double* r) {
+  return Parts3{{r}, {r + 1}, {r + 2}, {r + 3}, {r + 4}, {r + 5}, {reinterpret_cast<uint64_t*>(r + 6)}};
+}
 
-// mixed-precision particles: x cell index, FP32 in-cell offsets (x - ix,
-// y - j, z - k, all in [0, 1)) and FP32 momenta; 36 B per particle with the id
-struct PartsM3 {
-  int* ix;
-  float *ox, *oy, *oz, *ux, *uy, *uz;
-  uint64_t* id;
+struct Rec3 {
+  double x, y, z, ux, uy, uz;
+  uint64_t id;
 };
+__device__ inline Rec3 load_rec(const Parts3& P, size_t i) {
+  Rec3 r;
+  __builtin_memcpy(&r, P.x.p + PART3_DOUBLES * i, sizeof r);
+  return r;
+}
+__device__ inline void store_rec(const Parts3& P, size_t i, const Rec3& r) {
+  __builtin_memcpy(P.x.p + PART3_DOUBLES * i, &r, sizeof r);
+}
+
+// mixed-precision particles: 36-byte records of x cell index, FP32 in-cell
+// offsets (x - ix, y - j, z - k, all in [0, 1)), FP32 momenta and the id in
+// two words
+struct IdM3 {
+  uint32_t* q;
+  __host__ __device__ operator uint64_t() const { return (uint64_t)q[0] | ((uint64_t)q[1] << 32); }
+  __host__ __device__ void operator=(uint64_t v) const {
+    q[0] = (uint32_t)v;
+    q[1] = (uint32_t)(v >> 32);
+  }
+};
+struct IdColM3 {
+  uint32_t* p;
+  __host__ __device__ IdM3 operator[](size_t i) const { return IdM3{p + 9 * i}; }
+};
+struct PartsM3 {
+  Col<int, 9> ix;
+  Col<float, 9> ox, oy, oz, ux, uy, uz;
+  IdColM3 id;
+};
+constexpr int PARTM3_FLOATS = 9;
+inline PartsM3 partsm3_at(float* r) {
+  return PartsM3{{reinterpret_cast<int*>(r)}, {r + 1}, {r + 2}, {r + 3}, {r + 4}, {r + 5}, {r + 6},
+                 {reinterpret_cast<uint32_t*>(r + 7)}};
+}
+
+struct RecM3 {
+  int ix;
+  float ox, oy, oz, ux, uy, uz;
+  uint32_t id0, id1;
+};
+__device__ inline RecM3 load_rec(const PartsM3& P, size_t i) {
+  RecM3 r;
+  __builtin_memcpy(&r, P.ix.p + PARTM3_FLOATS * i, sizeof r);
+  return r;
+}
+__device__ inline void store_rec(const PartsM3& P, size_t i, const RecM3& r) {
+  __builtin_memcpy(P.ix.p + PARTM3_FLOATS * i, &r, sizeof r);
+}
 
 // Exchange direction of a particle leaving column (j, k) for (j+dj, k+dk):
 // dir = (dk+1)*3 + (dj+1); DIR_STAY = 4.  The exchange code of a particle is
@@ -115,8 +167,6 @@ struct wpic_ctx3d {
   wpic::PartsM3 MA, MB;
   int* aperm;    // A's slot -> record in A's buffer, or null
   int* permbuf;  // [N] the sort's permutation
-  int* nov;      // [1] overflow count of the fused push+deposit
-  uint64_t* id[2];  // the two id buffers (A's and B's)
   int *code, *R, *holes, *mlist;  // [N]
   int* cols[3];                   // column structures: base [nsp*ncol] then np2 [nsp*ncol]
   int ca, cb, cn;                 // which column structure belongs to A, B, the exchange
