@@ -106,16 +106,19 @@ __global__ void k_adj_field1(Grid2D g, const double* __restrict__ lamF, double* 
 
 // warm start and |b|^2 partials for the transposed solves (the CG kernels of
 // the forward then run unchanged on b and phi)
-__global__ __launch_bounds__(256) void k_adj_cg_init(Grid2D g, double* phi, const double* b, double* part,
-                                                     int parity) {
+__global__ __launch_bounds__(256) void k_adj_cg_init(Grid2D g, double* phi, const double* b, double* r, double* pold,
+                                                     double* part, int nb, int parity) {
   __shared__ double sh[4];
   const int n = g.nx * g.ny;
   double s[3] = {0.0, 0.0, 0.0};
-  for (int k = blockIdx.x * 256 + threadIdx.x; k < n; k += NPB * 256) {
+  for (int k = blockIdx.x * 256 + threadIdx.x; k < n; k += nb * 256) {
 #pragma unroll
     for (int l = 0; l < 3; l++) {
-      phi[(size_t)l * n + k] = 0.0;
-      const double v = b[(size_t)l * n + k];
+      const size_t q = (size_t)l * n + k;
+      const double v = b[q];
+      phi[q] = 0.0;
+      r[q] = v;
+      if (parity) pold[q] = v;
       s[l] = s[l] + v * v;
     }
   }
@@ -127,7 +130,11 @@ __global__ __launch_bounds__(256) void k_adj_cg_init(Grid2D g, double* phi, cons
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     if (lane == 0) sh[w] = v;
     __syncthreads();
-    if (threadIdx.x == 0) part[((size_t)l * NPB + blockIdx.x) * 2] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
+    if (threadIdx.x == 0) {
+      const double t = (sh[0] + sh[1]) + (sh[2] + sh[3]);
+      part[(l * 3 + 0) * NPB + blockIdx.x] = t;  // r.r
+      part[(l * 3 + 2) * NPB + blockIdx.x] = t;  // b.b
+    }
     __syncthreads();
   }
 }
@@ -331,6 +338,8 @@ __global__ __launch_bounds__(256, 2) void k_adj_particles(AdjPArgs a) {
         }
         F[cm] = f;
       }
+      // (combined here, not where a later block uses them)
+      asm volatile("" : "+v"(F[0]), "+v"(F[1]), "+v"(F[2]), "+v"(F[3]), "+v"(F[4]), "+v"(F[5]));
       const double B[3] = {F[0], F[1], F[2]}, E[3] = {F[3], F[4], F[5]};
       double uvm[3];
 #pragma unroll
@@ -645,7 +654,8 @@ hipError_t launch_adj_unsort(wpic_ctx* c, const int* rows, const int* perm, cons
 
 hipError_t launch_adj_field1(wpic_ctx* c, const double* lamF, double* lamF2, double* lamJ) {
   hipLaunchKernelGGL(k_adj_field1, dim3(cells_grid(c->g)), dim3(256), 0, c->st, c->g, lamF, lamF2, c->bb, lamJ);
-  hipLaunchKernelGGL(k_adj_cg_init, dim3(NPB), dim3(256), 0, c->st, c->g, c->phi, c->bb, c->part,
+  const int nb = cg_blocks(c->g);
+  hipLaunchKernelGGL(k_adj_cg_init, dim3(nb), dim3(256), 0, c->st, c->g, c->phi, c->bb, c->rr, c->pa, c->part, nb,
                      c->mode == WPIC_MODE_PARITY ? 1 : 0);
   return hipGetLastError();
 }

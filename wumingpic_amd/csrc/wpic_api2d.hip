@@ -153,33 +153,41 @@ int ensure_pjbuf(wpic_ctx* c) {
   return 0;
 }
 
-// field__fdtd_i after the deposit: current BCs, RHS, CG, E, BCs, update
+// The CG's iterations, launched a batch at a time; the three components stop
+// on their own device flags (an iteration past convergence changes nothing),
+// and the host polls once per batch.  The first batch is the last solve's
+// count, so a step whose count does not grow polls once.
 int cg_loop_impl(wpic_ctx* c) {
-  // iterations are launched a batch at a time; the three components stop on
-  // their own device flags (an iteration past convergence changes nothing),
-  // the host polls once per batch.  The first batch is the last solve's
-  // count plus one, so a step whose count does not grow polls once.
+  const bool parity = c->mode == WPIC_MODE_PARITY;
   const int NB = 4;
-  int it = 0;
-  struct {
-    CgScal s[3];
-    int err;
-  } h;
-  int nb = c->cg_hint > 0 ? c->cg_hint + 1 : NB;
+  int it = 0, nb = c->cg_hint > 0 ? c->cg_hint : NB;
+  CgPoll h;
   for (;;) {
-    for (int b = 0; b < nb && it < 100; b++, it++) HIPCHK(launch_cg_iter(c, it));
+    for (int b = 0; b < nb && it < 100; b++, it++) HIPCHK(launch_cg_iter(c, it, b == nb - 1 || it == 99));
     nb = NB;
-    HIPCHK(hipMemcpyAsync(h.s, c->scal, sizeof(h.s), hipMemcpyDeviceToHost, c->st));
-    HIPCHK(hipMemcpyAsync(&h.err, c->err, sizeof(int), hipMemcpyDeviceToHost, c->st));
-    HIPCHK(hipStreamSynchronize(c->st));
+    if (parity) {
+      CgScal s[3];
+      HIPCHK(hipMemcpyAsync(s, c->scal, sizeof(s), hipMemcpyDeviceToHost, c->st));
+      HIPCHK(hipMemcpyAsync(&h.err, c->err, sizeof(int), hipMemcpyDeviceToHost, c->st));
+      HIPCHK(hipStreamSynchronize(c->st));
+      for (int l = 0; l < 3; l++) {
+        h.more[l] = s[l].active;
+        h.ite[l] = s[l].ite;
+      }
+    } else {
+      HIPCHK(hipEventSynchronize(c->ev_poll));
+      std::memcpy(&h, c->poll, sizeof(h));
+    }
     if (h.err) return check_err(c);
-    if (!h.s[0].active && !h.s[1].active && !h.s[2].active) break;
-    if (it >= 100) return set_error(WPIC_ECG, "********** stop at cgm after ite_max **********");
+    const bool stop = !h.more[0] && !h.more[1] && !h.more[2];
+    if ((it >= 100 && !stop) || h.ite[0] >= 100 || h.ite[1] >= 100 || h.ite[2] >= 100)
+      return set_error(WPIC_ECG, "********** stop at cgm after ite_max **********");
+    if (stop) break;
   }
   c->cg_hint = 0;
   for (int l = 0; l < 3; l++) {
-    c->cg_iters[l] = h.s[l].ite;
-    if (h.s[l].ite > c->cg_hint) c->cg_hint = h.s[l].ite;
+    c->cg_iters[l] = h.ite[l];
+    if (h.ite[l] > c->cg_hint) c->cg_hint = h.ite[l];
   }
   return 0;
 }
@@ -193,7 +201,11 @@ int field_after_deposit(wpic_ctx* c) {
     HIPCHK(launch_cg_init(c));
     int rc = cg_loop_impl(c);
     if (rc) return rc;
-    HIPCHK(launch_cg_store(c));
+    if (walls(c->g)) HIPCHK(launch_cg_store(c));
+  }
+  if (!walls(c->g)) {
+    HIPCHK(launch_field_end_periodic(c));
+    return 0;
   }
   HIPCHK(launch_dfield_bc(c));
   HIPCHK(launch_e_update(c));
@@ -441,8 +453,10 @@ int wpic_create2d(wpic_ctx** out, const wpic_params2d* p) {
   double** cg[] = {&c->phi, &c->pa, &c->pb, &c->rr, &c->bb, &c->ap};
   for (auto q : cg)
     if (e == hipSuccess) e = dalloc(q, 3 * nc);
-  if (e == hipSuccess) e = dalloc(&c->part, (size_t)3 * NPB * 2);
-  if (e == hipSuccess) e = dalloc(&c->scal, 3);
+  if (e == hipSuccess) e = dalloc(&c->part, (size_t)3 * 3 * NPB);
+  if (e == hipSuccess) e = dalloc(&c->scal, 6);
+  if (e == hipSuccess) e = hipHostMalloc((void**)&c->poll, sizeof(CgPoll), hipHostMallocCoherent);
+  if (e == hipSuccess) e = hipEventCreateWithFlags(&c->ev_poll, hipEventDisableTiming);
   if (e == hipSuccess) e = dalloc(&c->err, 1);
   if (e == hipSuccess) e = dalloc(&c->red, (size_t)256 * 3);
   if (e == hipSuccess) e = hipMemset(c->err, 0, sizeof(int));
@@ -482,6 +496,8 @@ int wpic_destroy(wpic_ctx* c) {
     if (q) (void)hipFree(q);
   if (c->ev_push) (void)hipEventDestroy(c->ev_push);
   if (c->ev_sort) (void)hipEventDestroy(c->ev_sort);
+  if (c->ev_poll) (void)hipEventDestroy(c->ev_poll);
+  if (c->poll) (void)hipHostFree(c->poll);
   if (c->st2) (void)hipStreamDestroy(c->st2);
   if (c->st) (void)hipStreamDestroy(c->st);
   delete c;

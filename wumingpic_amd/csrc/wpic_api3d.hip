@@ -169,28 +169,41 @@ int field_after_deposit3(wpic_ctx3d* c) {
   {
     Timed3 tc(c, "cg");
     HIPCHK(launch_cg_init3d(c));
+    // a batch of iterations at a time, the first as many as the last solve
+    // took: the host polls once per batch
+    const bool parity = c->mode == WPIC_MODE_PARITY;
     const int NB = 4;
-    int it = 0;
-    struct {
-      CgScal s[3];
-    } h;
-    int herr = 0;
+    int it = 0, nb = c->cg_hint > 0 ? c->cg_hint : NB;
+    CgPoll h;
     for (;;) {
-      for (int b = 0; b < NB && it < 100; b++, it++) HIPCHK(launch_cg_iter3d(c, it));
-      HIPCHK(hipMemcpyAsync(h.s, c->scal, sizeof(h.s), hipMemcpyDeviceToHost, c->st));
-      HIPCHK(hipMemcpyAsync(&herr, c->err, sizeof(int), hipMemcpyDeviceToHost, c->st));
-      HIPCHK(hipStreamSynchronize(c->st));
-      if (herr) return check_err3(c);
-      if (!h.s[0].active && !h.s[1].active && !h.s[2].active) break;
-      if (it >= 100) return set_error(WPIC_ECG, "********** stop at cgm after ite_max **********");
+      for (int b = 0; b < nb && it < 100; b++, it++) HIPCHK(launch_cg_iter3d(c, it, b == nb - 1 || it == 99));
+      nb = NB;
+      if (parity) {
+        CgScal s[3];
+        HIPCHK(hipMemcpyAsync(s, c->scal, sizeof(s), hipMemcpyDeviceToHost, c->st));
+        HIPCHK(hipMemcpyAsync(&h.err, c->err, sizeof(int), hipMemcpyDeviceToHost, c->st));
+        HIPCHK(hipStreamSynchronize(c->st));
+        for (int l = 0; l < 3; l++) {
+          h.more[l] = s[l].active;
+          h.ite[l] = s[l].ite;
+        }
+      } else {
+        HIPCHK(hipEventSynchronize(c->ev_poll));
+        std::memcpy(&h, c->poll, sizeof(h));
+      }
+      if (h.err) return check_err3(c);
+      const bool stop = !h.more[0] && !h.more[1] && !h.more[2];
+      if ((it >= 100 && !stop) || h.ite[0] >= 100 || h.ite[1] >= 100 || h.ite[2] >= 100)
+        return set_error(WPIC_ECG, "********** stop at cgm after ite_max **********");
+      if (stop) break;
     }
-    for (int l = 0; l < 3; l++) c->cg_iters[l] = h.s[l].ite;
-    HIPCHK(launch_cg_store3d(c));
+    c->cg_hint = 0;
+    for (int l = 0; l < 3; l++) {
+      c->cg_iters[l] = h.ite[l];
+      if (h.ite[l] > c->cg_hint) c->cg_hint = h.ite[l];
+    }
   }
-  HIPCHK(launch_dfield_bc3d(c));
-  HIPCHK(launch_e_update3d(c));
-  HIPCHK(launch_dfield_bc3d(c));
-  HIPCHK(launch_uf_add3d(c));
+  HIPCHK(launch_field_end3d(c));
   return 0;
 }
 
@@ -512,8 +525,10 @@ int wpic_create3d(wpic_ctx3d** out, const wpic_params3d* p) {
   double** cg[] = {&c->phi, &c->pa, &c->pb, &c->rr, &c->bb, &c->ap};
   for (auto q : cg)
     if (e == hipSuccess) e = dalloc(q, 3 * nc);
-  if (e == hipSuccess) e = dalloc(&c->part, (size_t)3 * NPB3 * 2);
-  if (e == hipSuccess) e = dalloc(&c->scal, 3);
+  if (e == hipSuccess) e = dalloc(&c->part, (size_t)3 * 3 * NPB3);
+  if (e == hipSuccess) e = dalloc(&c->scal, 6);
+  if (e == hipSuccess) e = hipHostMalloc((void**)&c->poll, sizeof(CgPoll), hipHostMallocCoherent);
+  if (e == hipSuccess) e = hipEventCreateWithFlags(&c->ev_poll, hipEventDisableTiming);
   if (e == hipSuccess) e = dalloc(&c->err, 1);
   if (e == hipSuccess) e = dalloc(&c->red, (size_t)256 * 3);
   if (e == hipSuccess) e = hipMemset(c->err, 0, sizeof(int));
@@ -554,6 +569,8 @@ int wpic_destroy3d(wpic_ctx3d* c) {
     if (q) (void)hipFree(q);
   if (c->ev_push) (void)hipEventDestroy(c->ev_push);
   if (c->ev_sort) (void)hipEventDestroy(c->ev_sort);
+  if (c->ev_poll) (void)hipEventDestroy(c->ev_poll);
+  if (c->poll) (void)hipHostFree(c->poll);
   if (c->st2) (void)hipStreamDestroy(c->st2);
   if (c->st) (void)hipStreamDestroy(c->st);
   delete c;

@@ -315,6 +315,17 @@ __device__ inline T row16_sum(T v) {
   return v;
 }
 
+// Sum over the 64 lanes of a wholly active wave, the same bits in every lane.
+__device__ inline double wave_sum(double v) {
+  v = row16_sum(v);
+  double r[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++)
+    r[q] = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 16 * q),
+                            __builtin_amdgcn_readlane(__double2loint(v), 16 * q));
+  return (r[0] + r[1]) + (r[2] + r[3]);
+}
+
 // Sum over the 8 lanes of a half DPP row, every lane of the half receiving
 // it: quad permutes for the partners 1 and 2 apart, then the half-row mirror
 // (lane l and 7 - l), which pairs each quad with the other.
@@ -472,6 +483,12 @@ struct CgScal {
   int ite, active;
 };
 
+// how a fast solve stands after an iteration, written by the device into the
+// host's pinned memory: components that go on, iterations done, error bits
+struct CgPoll {
+  int more[3], ite[3], err;
+};
+
 struct TimerRec {
   std::string name;
   hipEvent_t a, b;
@@ -528,10 +545,11 @@ struct wpic_ctx {
 
   // CG: interior vectors per component
   double *phi, *pa, *pb, *rr, *bb, *ap;  // [3][nx*ny]
-  double* part;                          // block partial sums [3][NPB][2]
-  wpic::CgScal* scal;                    // [3]
+  double* part;                          // block partial sums [3][3][NPB]
+  wpic::CgScal* scal;                    // [2][3]
   int* err;                              // device error bits
-  int* hflags;                           // pinned host mirror: err, active[3], ite[3]
+  wpic::CgPoll* poll;                    // pinned host memory
+  hipEvent_t ev_poll;                    // recorded after the iteration that writes it
   int cg_iters[3];
   int cg_hint;  // the largest iteration count of the last solve (the first batch's size)
 
@@ -553,7 +571,27 @@ struct wpic_ctx {
 
 namespace wpic {
 
-constexpr int NPB = 256;  // fixed number of partial-sum blocks in CG reductions
+// partial-sum blocks of a CG component: one per 256 cells, at most NPB (the
+// number, and so the order of the sums, depends on the grid alone)
+constexpr int NPB = 1024;
+inline int cg_blocks(const Grid2D& g) {
+  const int n = (g.nx * g.ny + 255) / 256;
+  return n < NPB ? n : NPB;
+}
+// Work units of an iteration's kernels: 64 columns of `len` rows for each wave,
+// len so that a grid gives some 2,048 units (a wave that marches more rows
+// reads fewer of its neighbours')
+struct Strips2 {
+  int ntx, len, units;
+};
+__host__ __device__ inline Strips2 strips2(const Grid2D& g) {
+  Strips2 s;
+  s.ntx = (g.nx + 63) / 64;
+  int len = (int)((long long)s.ntx * g.ny / 2048);
+  s.len = len < 1 ? 1 : (len > 16 ? 16 : len);
+  s.units = s.ntx * ((g.ny + s.len - 1) / s.len);
+  return s;
+}
 
 int set_error(int code, const std::string& msg);
 int hip_fail(hipError_t e, const char* what);
@@ -567,7 +605,8 @@ hipError_t launch_zero(wpic_ctx* c, double* p, size_t n);
 hipError_t launch_curre_bc(wpic_ctx* c);
 hipError_t launch_dfield_bc(wpic_ctx* c);
 hipError_t launch_cg_init(wpic_ctx* c);
-hipError_t launch_cg_iter(wpic_ctx* c, int it_in_batch);
+hipError_t launch_cg_iter(wpic_ctx* c, int it, bool poll);
+hipError_t launch_field_end_periodic(wpic_ctx* c);
 hipError_t launch_cg_store(wpic_ctx* c);
 hipError_t launch_e_update(wpic_ctx* c);
 hipError_t launch_uf_add(wpic_ctx* c);

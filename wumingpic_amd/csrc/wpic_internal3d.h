@@ -190,8 +190,11 @@ struct wpic_ctx3d {
   double* pjbuf;         // parity deposit blocks [nx*ny*nz][300] (lazy)
 
   double *phi, *pa, *pb, *rr, *bb, *ap;  // CG vectors [3][nx*ny*nz]
-  double* part;
-  wpic::CgScal* scal;
+  double* part;              // block partial sums [3][3][NPB3]
+  wpic::CgScal* scal;        // [2][3]
+  wpic::CgPoll* poll;        // pinned host memory
+  hipEvent_t ev_poll;        // recorded after the iteration that writes it
+  int cg_hint;               // the largest iteration count of the last solve (the first batch's size)
   int* err;
   int cg_iters[3];
 
@@ -226,12 +229,9 @@ hipError_t launch_gather_pj3d(wpic_ctx3d* c);
 // fields
 hipError_t launch_fill3d(wpic_ctx3d* c, double* p, size_t n, double v);
 hipError_t launch_curre_bc3d(wpic_ctx3d* c);
-hipError_t launch_dfield_bc3d(wpic_ctx3d* c);
 hipError_t launch_cg_init3d(wpic_ctx3d* c);
-hipError_t launch_cg_iter3d(wpic_ctx3d* c, int it);
-hipError_t launch_cg_store3d(wpic_ctx3d* c);
-hipError_t launch_e_update3d(wpic_ctx3d* c);
-hipError_t launch_uf_add3d(wpic_ctx3d* c);
+hipError_t launch_cg_iter3d(wpic_ctx3d* c, int it, bool poll);
+hipError_t launch_field_end3d(wpic_ctx3d* c);
 hipError_t launch_energy3d(wpic_ctx3d* c, double* dout, int sp = -1);
 hipError_t launch_ic_weibel3d(wpic_ctx3d* c, unsigned long long seed, int n0, const double* sd, double t_ani);
 hipError_t launch_gauss3d(wpic_ctx3d* c, double* G, double* rho);
