@@ -172,6 +172,66 @@ __global__ __launch_bounds__(SB) void k_colscan3d(Sort3Args a, int wrap) {
   }
 }
 
+// The same counts and mover lists for the fused fast sort, which needs neither
+// the holes nor the lists in slot order (the codes are written): a leaver takes
+// its rank in its direction from an LDS counter, only leavers cost more than
+// their code's read, and up to LQ of them wait in LDS for the directions'
+// starts.  Bound by the read of the codes; at 256^3, 16 ppc a species, next to
+// the field solve 1.6 ms, where the two passes with nine ballots for every 64
+// codes take 2.1.
+__global__ __launch_bounds__(SB) void k_colscan3d_fast(Sort3Args a) {
+  constexpr int SF = 8, LQ = 1024;
+  __shared__ int cnt[9], start[9], nl;
+  __shared__ int lslot[LQ], lrank[LQ];  // slot, rank << 4 | direction
+  const Grid3D& g = a.g;
+  const int rw = blockIdx.x;
+  const int base = a.colbaseB[rw], n = a.np2B[rw];
+  const int tid = threadIdx.x;
+  if (tid < 9) cnt[tid] = 0;
+  if (tid == 0) nl = 0;
+  __syncthreads();
+  for (int k0 = 0; k0 < n; k0 += SB * SF) {
+    int v[SF];
+#pragma unroll
+    for (int u = 0; u < SF; u++) {
+      const int q = k0 + u * SB + tid;
+      v[u] = q < n ? a.code[base + q] : DIR_STAY;
+    }
+#pragma unroll
+    for (int u = 0; u < SF; u++) {
+      const int dir = v[u] & 15;
+      if (dir == DIR_STAY || dir > 8) continue;
+      const int rank = atomicAdd(&cnt[dir], 1), e = wave_enqueue(&nl);
+      if (e < LQ) {
+        lslot[e] = k0 + u * SB + tid;
+        lrank[e] = rank << 4 | dir;
+      }
+    }
+  }
+  __syncthreads();
+  if (tid == 0) {
+    int acc = 0;
+    for (int d = 0; d < 9; d++) {
+      start[d] = acc;
+      a.dstart[rw * 9 + d] = acc;
+      a.dcnt[rw * 9 + d] = cnt[d];
+      acc += cnt[d];
+    }
+    a.dcnt[rw * 9 + DIR_STAY] = n - acc;
+    a.colkm[rw * 2] = acc;  // leavers
+  }
+  __syncthreads();
+  if (nl <= LQ) {
+    for (int e = tid; e < nl; e += SB) a.mlist[base + start[lrank[e] & 15] + (lrank[e] >> 4)] = base + lslot[e];
+    return;
+  }
+  // more leavers than wait in LDS: read the codes again, start counts up
+  for (int q = tid; q < n; q += SB) {
+    const int dir = a.code[base + q] & 15;
+    if (dir != DIR_STAY && dir <= 8) a.mlist[base + atomicAdd(&start[dir], 1)] = base + q;
+  }
+}
+
 // arrivals m of every column, new length L = np2 - leavers + m, and its base:
 // one workgroup per 1024 columns of a species takes the exclusive prefix of L
 // within its columns (written as colbaseN for now) and its total; a single
@@ -497,13 +557,22 @@ __global__ __launch_bounds__(SB) void k_colsort3d(Sort3Args a, int nbits) {
 // permutation.  Each cell receives the particles particle_yz and sort__bucket
 // put there (np2 and cumcnt are the reference's), in an order of its own, so
 // only the summation order of the deposit changes.
+//
+// A wave whose share fits SR stayers and AR arrivals a lane keeps them in
+// registers: one pass reads a code, takes the particle's rank among the wave's
+// particles of its cell from the LDS counter, and after the scan writes the
+// permutation at the cell's start plus the rank.  A longer column (more than
+// 5,120 particles, or 1,024 arrivals) is read twice.
+// What held it back was the chain of waits: one thread looked up the eight
+// segments one after another, and every chunk was loaded, counted and waited
+// for twice.  At 256^3, 16 ppc a species, next to the field solve: 9.0 -> 2.2
+// ms; 160x144x128 1.4 -> 0.39 ms.
 __global__ __launch_bounds__(SB) void k_colsort3d_fast(Sort3Args a) {
   extern __shared__ int hist[];  // [SB/64][nx]
   __shared__ int wsum[SB / 64];
   __shared__ int carry;
   __shared__ int scnt[8], sptr[8];
-  __shared__ int nsg;
-  constexpr int SF = 8, NW = SB / 64;
+  constexpr int SF = 8, SR = 20, AR = 4, NW = SB / 64;
   const Grid3D& g = a.g;
   const int nx = g.nx;
   const int rw = blockIdx.x;
@@ -511,16 +580,19 @@ __global__ __launch_bounds__(SB) void k_colsort3d_fast(Sort3Args a) {
   const int base = a.colbaseB[rw], n = a.np2B[rw];
   const int L = a.np2N[rw], nb = a.colbaseN[rw];
   const int m = a.colkm[rw * 2 + 1];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const unsigned ntot = (unsigned)(g.ncap * g.nsp);
-  if (tid == 0) {
-    nsg = a.nseg[col];
-    for (int e = 0; e < nsg; e++) {
-      const int sg = a.seg[col * 8 + e];
+  const int nseg = a.nseg[col];
+  if (tid < 8) {
+    int cnt = 0, ptr = 0;
+    if (tid < nseg) {
+      const int sg = a.seg[col * 8 + tid];
       const int src = s * g.ncol + (sg >> 4), d = sg & 15;
-      scnt[e] = a.dcnt[src * 9 + d];
-      sptr[e] = a.colbaseB[src] + a.dstart[src * 9 + d];
+      cnt = a.dcnt[src * 9 + d];
+      ptr = a.colbaseB[src] + a.dstart[src * 9 + d];
     }
+    scnt[tid] = cnt;
+    sptr[tid] = ptr;
   }
   for (int q = tid; q < NW * nx; q += SB) hist[q] = 0;
   __syncthreads();
@@ -529,84 +601,24 @@ __global__ __launch_bounds__(SB) void k_colsort3d_fast(Sort3Args a) {
   const int alo = (int)(((long long)m * w) / NW), ahi = (int)(((long long)m * (w + 1)) / NW);
   const int nsl = hi - lo;  // chunk index space: stayer slots then arrivals
   const int tot = nsl + (ahi - alo);
-  // the segments in registers: arrival t of segment q (first arrival sb[q])
-  // is list entry sp[q] + t; an empty tail of segments starts at infinity
-  int sb[8], sp[8];
-  {
-    const int nseg = nsg;
-    int acc = 0;
+  // arrival t of segment q (first arrival sb) is list entry sptr[q] + t - sb
+  auto list_entry = [&](int t) {
+    int sb = 0, d = sptr[0];
 #pragma unroll
-    for (int q = 0; q < 8; q++) {
-      const bool in = q < nseg;
-      const int cnt = in ? scnt[q] : 0;
-      sb[q] = in ? acc : 0x7fffffff;
-      sp[q] = in ? sptr[q] - acc : 0;
-      acc += cnt;
+    for (int q = 1; q < 8; q++) {
+      sb += scnt[q - 1];
+      if (q < nseg && t >= sb) d = sptr[q] - sb;
     }
-  }
+    return d + t;
+  };
   int* hw = hist + w * nx;
   int* cc = a.cumcnt + (size_t)rw * (nx + 1);
   bool bad = false;
-  for (int pass = 0; pass < 2; pass++) {
-    for (int e0 = 0; e0 < tot; e0 += 64 * SF) {
-      // a stayer slot's code (direction and key in one word), or an
-      // arrival's list entry (its source slot); every load of the chunk is
-      // issued before the first is used
-      int v[SF];
-#pragma unroll
-      for (int u = 0; u < SF; u++) {
-        const int e = e0 + u * 64 + lane;
-        const int t = alo + (e - nsl);
-        int d = sp[0];
-#pragma unroll
-        for (int q = 1; q < 8; q++) d = t >= sb[q] ? sp[q] : d;
-        const int* ptr = e < nsl ? a.code + (base + lo + e) : (e < tot ? a.mlist + (d + t) : a.code);
-        v[u] = *ptr;
-      }
-      int src[SF];
-#pragma unroll
-      for (int u = 0; u < SF; u++) {
-        const int e = e0 + u * 64 + lane;
-        const bool arr = e >= nsl && e < tot;
-        const bool okarr = arr && (unsigned)v[u] < ntot;
-        bad |= arr && !okarr;
-        src[u] = e < nsl ? (((v[u] & 15) == DIR_STAY) ? base + lo + e : -1) : (okarr ? v[u] : -1);
-      }
-      // an arrival's code (the stayers already hold theirs)
-      int c2[SF];
-#pragma unroll
-      for (int u = 0; u < SF; u++) {
-        const int e = e0 + u * 64 + lane;
-        c2[u] = a.code[(e >= nsl && src[u] >= 0) ? src[u] : 0];
-      }
-      int key[SF];
-#pragma unroll
-      for (int u = 0; u < SF; u++) {
-        const int e = e0 + u * 64 + lane;
-        key[u] = src[u] < 0 ? 0 : ((e < nsl ? v[u] : c2[u]) >> CODE_SHIFT3);
-      }
-      // one LDS atomic per particle: lanes of a key meet on its counter and
-      // the LDS serves them one after another (the order within a cell is
-      // the fast modes' own)
-      if (pass == 0) {
-#pragma unroll
-        for (int u = 0; u < SF; u++)
-          if (src[u] >= 0) atomicAdd(&hw[key[u]], 1);
-      } else {
-        int pos[SF];
-#pragma unroll
-        for (int u = 0; u < SF; u++) pos[u] = src[u] >= 0 ? atomicAdd(&hw[key[u]], 1) : 0;
-#pragma unroll
-        for (int u = 0; u < SF; u++) {
-          const bool ok = src[u] >= 0 && pos[u] < L;
-          bad |= src[u] >= 0 && !ok;
-          if (ok) a.perm[nb + pos[u]] = src[u];
-        }
-      }
-    }
+
+  // exclusive scan over keys of the column totals -> cumcnt; hist becomes the
+  // waves' first slots of each cell
+  auto scan = [&]() {
     __syncthreads();
-    if (pass == 1) break;
-    // exclusive scan over keys of the column totals -> cumcnt; per-wave cursors
     if (tid == 0) carry = 0;
     __syncthreads();
     for (int k0 = 0; k0 < nx; k0 += SB) {
@@ -640,6 +652,90 @@ __global__ __launch_bounds__(SB) void k_colsort3d_fast(Sort3Args a) {
     }
     if (tid == 0) cc[nx] = L;
     __syncthreads();
+  };
+
+  if ((n + NW - 1) / NW <= 64 * SR && (m + NW - 1) / NW <= 64 * AR) {  // the same for all waves
+    int key[SR + AR], src[AR], rank[SR + AR];
+#pragma unroll
+    for (int u = 0; u < SR; u++) key[u] = u * 64 + lane < nsl ? a.code[base + lo + u * 64 + lane] : 0;
+#pragma unroll
+    for (int u = 0; u < AR; u++) {
+      src[u] = -1;
+      key[SR + u] = 0;
+      const int t = alo + u * 64 + lane;
+      if (alo + u * 64 < ahi && t < ahi) {
+        src[u] = a.mlist[list_entry(t)];
+        const bool ok = (unsigned)src[u] < ntot;
+        bad |= !ok;
+        if (!ok) src[u] = -1;
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < AR; u++)
+      if (src[u] >= 0) key[SR + u] = a.code[src[u]];
+    // ranks; a key of -1 is no entry
+#pragma unroll
+    for (int u = 0; u < SR + AR; u++) {
+      const bool in = u < SR ? u * 64 + lane < nsl && (key[u] & 15) == DIR_STAY : src[u < SR ? 0 : u - SR] >= 0;
+      key[u] = in ? key[u] >> CODE_SHIFT3 : -1;
+      rank[u] = 0;
+      if (in) rank[u] = atomicAdd(&hw[key[u]], 1);
+    }
+    scan();
+#pragma unroll
+    for (int u = 0; u < SR + AR; u++) {
+      const int pos = hw[key[u] >= 0 ? key[u] : 0] + rank[u];
+      const bool ok = key[u] >= 0 && pos < L;
+      bad |= key[u] >= 0 && !ok;
+      if (ok) a.perm[nb + pos] = u < SR ? base + lo + u * 64 + lane : src[u < SR ? 0 : u - SR];
+    }
+    if (bad) atomicOr(a.err, ERR_ROW);
+    return;
+  }
+
+  for (int pass = 0; pass < 2; pass++) {
+    for (int e0 = 0; e0 < tot; e0 += 64 * SF) {
+      // a stayer slot's code (direction and key in one word), or an
+      // arrival's list entry (its source slot); every load of the chunk is
+      // issued before the first is used
+      int v[SF];
+#pragma unroll
+      for (int u = 0; u < SF; u++) {
+        const int e = e0 + u * 64 + lane;
+        const int* ptr =
+            e < nsl ? a.code + (base + lo + e) : (e < tot ? a.mlist + list_entry(alo + (e - nsl)) : a.code);
+        v[u] = *ptr;
+      }
+      int src[SF];
+#pragma unroll
+      for (int u = 0; u < SF; u++) {
+        const int e = e0 + u * 64 + lane;
+        const bool arr = e >= nsl && e < tot;
+        const bool okarr = arr && (unsigned)v[u] < ntot;
+        bad |= arr && !okarr;
+        src[u] = e < nsl ? (((v[u] & 15) == DIR_STAY) ? base + lo + e : -1) : (okarr ? v[u] : -1);
+      }
+      // an arrival's code (the stayers already hold theirs)
+      int c2[SF];
+#pragma unroll
+      for (int u = 0; u < SF; u++) {
+        const int e = e0 + u * 64 + lane;
+        c2[u] = a.code[(e >= nsl && src[u] >= 0) ? src[u] : 0];
+      }
+      // one LDS atomic per particle: lanes of a key meet on its counter and
+      // the LDS serves them one after another (the order within a cell is
+      // the fast modes' own)
+#pragma unroll
+      for (int u = 0; u < SF; u++) {
+        const int e = e0 + u * 64 + lane;
+        if (src[u] < 0) continue;
+        const int pos = atomicAdd(&hw[(e < nsl ? v[u] : c2[u]) >> CODE_SHIFT3], 1);
+        if (pass == 0) continue;
+        bad |= pos >= L;
+        if (pos < L) a.perm[nb + pos] = src[u];
+      }
+    }
+    if (pass == 0) scan();
   }
   if (bad) atomicOr(a.err, ERR_ROW);
 }
@@ -695,6 +791,12 @@ hipError_t launch_wrapx3d(wpic_ctx3d* c) {
 // wrap = 0: the codes come from the mixed-precision push (cell wrap done)
 hipError_t launch_colscan3d(wpic_ctx3d* c, int wrap) {
   hipLaunchKernelGGL(k_colscan3d, ncols(c), dim3(SB), 0, c->st, sort3_args(c), wrap);
+  return hipGetLastError();
+}
+
+// the fused fast sort's lists alone, from the codes the push wrote
+hipError_t launch_colscan3d_fast(wpic_ctx3d* c) {
+  hipLaunchKernelGGL(k_colscan3d_fast, ncols(c), dim3(SB), 0, c->st, sort3_args(c));
   return hipGetLastError();
 }
 

@@ -267,7 +267,10 @@ int push_deposit3(wpic_ctx3d* c) {
 // sort (k_colsort3d_fast builds each new column from them)
 int exchange3(wpic_ctx3d* c, bool lists_only = false) {
   Timed3 t(c, "exchange");
-  HIPCHK(launch_colscan3d(c, c->b_coded ? 0 : 1));
+  if (lists_only && c->b_coded)
+    HIPCHK(launch_colscan3d_fast(c));
+  else
+    HIPCHK(launch_colscan3d(c, c->b_coded ? 0 : 1));
   HIPCHK(launch_colcount3d(c));
   if (!lists_only) HIPCHK(launch_colbuild3d(c));
   c->h_cols_ok[c->cn] = false;

@@ -238,6 +238,7 @@ hipError_t launch_gauss3d(wpic_ctx3d* c, double* G, double* rho);
 // particles
 hipError_t launch_wrapx3d(wpic_ctx3d* c);
 hipError_t launch_colscan3d(wpic_ctx3d* c, int wrap = 1);
+hipError_t launch_colscan3d_fast(wpic_ctx3d* c);
 hipError_t launch_colcount3d(wpic_ctx3d* c);
 hipError_t launch_colbuild3d(wpic_ctx3d* c);
 hipError_t launch_colsort3d(wpic_ctx3d* c);
