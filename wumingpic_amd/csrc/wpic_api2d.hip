@@ -498,6 +498,7 @@ int wpic_destroy(wpic_ctx* c) {
   if (c->ev_sort) (void)hipEventDestroy(c->ev_sort);
   if (c->ev_poll) (void)hipEventDestroy(c->ev_poll);
   if (c->poll) (void)hipHostFree(c->poll);
+  ring_free(c->ring);
   if (c->st2) (void)hipStreamDestroy(c->st2);
   if (c->st) (void)hipStreamDestroy(c->st);
   delete c;
@@ -680,8 +681,7 @@ static int download_planes(wpic_ctx* c, const double* planes, double* out, int n
   int rc = ensure_staging(c, n);
   if (rc) return rc;
   HIPCHK(launch_planes_to_aos(c, planes, c->staging, ncomp));
-  HIPCHK(hipMemcpyAsync(out, c->staging, sizeof(double) * n, hipMemcpyDeviceToHost, c->st));
-  HIPCHK(hipStreamSynchronize(c->st));
+  HIPCHK(copy_to_host(c->ring, c->device, c->st, out, c->staging, sizeof(double) * n));
   return 0;
 }
 
@@ -1293,8 +1293,7 @@ int wpic_download_mom2d(wpic_ctx* c, double* mom) {
   int rc = ensure_mom(c);
   if (rc) return rc;
   const size_t n = (size_t)7 * (c->g.nx + 2) * (c->g.ny + 2) * c->g.nsp;
-  HIPCHK(hipMemcpyAsync(mom, c->mom, sizeof(double) * n, hipMemcpyDeviceToHost, c->st));
-  HIPCHK(hipStreamSynchronize(c->st));
+  HIPCHK(copy_to_host(c->ring, c->device, c->st, mom, c->mom, sizeof(double) * n));
   return 0;
 }
 

@@ -391,8 +391,7 @@ int download_planes3(wpic_ctx3d* c, const double* planes, double* out, int ncomp
   int rc = ensure_staging3(c, n);
   if (rc) return rc;
   HIPCHK(launch_planes_to_aos3d(c, planes, c->staging, ncomp));
-  HIPCHK(hipMemcpyAsync(out, c->staging, sizeof(double) * n, hipMemcpyDeviceToHost, c->st));
-  HIPCHK(hipStreamSynchronize(c->st));
+  HIPCHK(copy_to_host(c->ring, c->device, c->st, out, c->staging, sizeof(double) * n));
   return 0;
 }
 
@@ -574,6 +573,7 @@ int wpic_destroy3d(wpic_ctx3d* c) {
   if (c->ev_sort) (void)hipEventDestroy(c->ev_sort);
   if (c->ev_poll) (void)hipEventDestroy(c->ev_poll);
   if (c->poll) (void)hipHostFree(c->poll);
+  ring_free(c->ring);
   if (c->st2) (void)hipStreamDestroy(c->st2);
   if (c->st) (void)hipStreamDestroy(c->st);
   delete c;
@@ -1064,8 +1064,7 @@ int wpic_download_mom3d(wpic_ctx3d* c, double* mom) {
   if (!c || !mom) return set_error(WPIC_EINVAL, "null argument");
   int rc = ensure_mom3(c);
   if (rc) return rc;
-  HIPCHK(hipMemcpyAsync(mom, c->mom, sizeof(double) * mom3_size(c->g), hipMemcpyDeviceToHost, c->st));
-  HIPCHK(hipStreamSynchronize(c->st));
+  HIPCHK(copy_to_host(c->ring, c->device, c->st, mom, c->mom, sizeof(double) * mom3_size(c->g)));
   return 0;
 }
 

@@ -489,6 +489,18 @@ struct CgPoll {
   int more[3], ite[3], err;
 };
 
+// A context's pinned slots for large copies to the host (wpic_copy.hip), made
+// by the first such copy and given back with the context.
+struct HostRing {
+  static constexpr int NSLOT = 12;
+  char* buf = nullptr;
+  hipEvent_t ev[NSLOT] = {};
+};
+// `bytes` from device memory to the caller's array, in stream order; done on
+// return
+hipError_t copy_to_host(HostRing& ring, int device, hipStream_t st, void* dst, const void* src, size_t bytes);
+void ring_free(HostRing& ring);
+
 struct TimerRec {
   std::string name;
   hipEvent_t a, b;
@@ -553,6 +565,7 @@ struct wpic_ctx {
   int cg_iters[3];
   int cg_hint;  // the largest iteration count of the last solve (the first batch's size)
 
+  wpic::HostRing ring;
   double* staging;  // transfer staging (lazy)
   size_t staging_n;
   long long* aosbase;  // [nsp*ny] row starts in a compact AoS transfer buffer

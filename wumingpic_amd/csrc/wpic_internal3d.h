@@ -198,6 +198,7 @@ struct wpic_ctx3d {
   int* err;
   int cg_iters[3];
 
+  wpic::HostRing ring;
   double* staging;
   size_t staging_n;
   long long* aosbase;  // [nsp*ncol]
