@@ -250,26 +250,12 @@ __global__ void k_ic_beams(IcArgs a) {
   const double th = electron ? a.uth_e : a.uth_i;
   double ux = th * n0;
   if (electron) ux += (sl & 1) ? -a.udrift : a.udrift;
-  if (MIXED) {
-    a.M.ix[d] = i;
-    a.M.ox[d] = to_offset(x - i);
-    a.M.oy[d] = to_offset(y - j);
-    a.M.ux[d] = (float)ux;
-    a.M.uy[d] = (float)(th * n1);
-    a.M.uz[d] = (float)(th * n2);
-  } else {
-    a.A.x[d] = x;
-    a.A.y[d] = y;
-    a.A.ux[d] = ux;
-    a.A.uy[d] = th * n1;
-    a.A.uz[d] = th * n2;
-  }
   // id = -(pid), pid counted row by row from 1 (app.f90:455-470)
-  const long long pid = k + 1;
+  const uint64_t id = (uint64_t)(-(long long)(k + 1));
   if (MIXED)
-    a.M.id[d] = (uint64_t)(-pid);
+    store_rec(a.M, d, RecM{i, to_offset(x - i), to_offset(y - j), (float)ux, (float)(th * n1), (float)(th * n2), id});
   else
-    a.A.id[d] = (uint64_t)(-pid);
+    store_rec(a.A, d, Rec{x, y, ux, th * n1, th * n2, id});
 }
 
 static IcArgs ic_args(wpic_ctx* c, unsigned long long seed, int n_ppc, double udrift, double uth_e,

@@ -1,5 +1,5 @@
 // k_misc3d.hip -- 3D layout conversion at the boundary (reference AoS of
-// ndim = 7 doubles <-> device SoA), the seeded initial state and diagnostics.
+// ndim = 7 doubles <-> the device's records), the seeded initial state and diagnostics.
 #include "wpic_internal3d.h"
 
 namespace wpic {
@@ -12,41 +12,26 @@ struct Xfer3Args {
   const long long* aosbase;  // [nsp*ncol] start of each column in the AoS buffer
 };
 
-__global__ void k_aos_to_soa3(Xfer3Args a, const double* __restrict__ aos) {
+// The records have the reference's own layout: a column is a copy (in) or, seen
+// through a permutation, a gather of records (out), a double at a time.
+__global__ void k_records3_in(Xfer3Args a, const uint64_t* __restrict__ aos) {
   const int rw = blockIdx.x;
-  const int base = a.colbase[rw], n = a.np2[rw];
-  const double* src = aos + a.aosbase[rw] * 7;
-  for (int q = threadIdx.x; q < n; q += blockDim.x) {
-    const double* s = src + (size_t)q * 7;
-    const int d = base + q;
-    a.P.x[d] = s[0];
-    a.P.y[d] = s[1];
-    a.P.z[d] = s[2];
-    a.P.ux[d] = s[3];
-    a.P.uy[d] = s[4];
-    a.P.uz[d] = s[5];
-    uint64_t b;
-    __builtin_memcpy(&b, &s[6], 8);
-    a.P.id[d] = b;
-  }
+  const size_t n = (size_t)a.np2[rw] * 7;
+  const uint64_t* src = aos + a.aosbase[rw] * 7;
+  uint64_t* dst = reinterpret_cast<uint64_t*>(a.P.x.p) + (size_t)a.colbase[rw] * 7;
+  for (size_t e = threadIdx.x; e < n; e += blockDim.x) dst[e] = src[e];
 }
 
-__global__ void k_soa_to_aos3(Xfer3Args a, double* __restrict__ aos) {
+__global__ void k_records3_out(Xfer3Args a, uint64_t* __restrict__ aos) {
   const int rw = blockIdx.x;
-  const int base = a.colbase[rw], n = a.np2[rw];
-  double* dst = aos + a.aosbase[rw] * 7;
-  for (int q = threadIdx.x; q < n; q += blockDim.x) {
-    int s = a.R ? a.R[base + q] : base + q;
+  const int base = a.colbase[rw];
+  const unsigned n = (unsigned)a.np2[rw] * 7u;
+  uint64_t* dst = aos + a.aosbase[rw] * 7;
+  for (unsigned e = threadIdx.x; e < n; e += blockDim.x) {
+    const unsigned q = e / 7u;
+    int s = a.R ? a.R[base + (int)q] : base + (int)q;
     if ((unsigned)s >= (unsigned)(a.g.ncap * a.g.nsp)) s = 0;
-    double* d = dst + (size_t)q * 7;
-    d[0] = a.P.x[s];
-    d[1] = a.P.y[s];
-    d[2] = a.P.z[s];
-    d[3] = a.P.ux[s];
-    d[4] = a.P.uy[s];
-    d[5] = a.P.uz[s];
-    const uint64_t b = a.P.id[s];
-    __builtin_memcpy(&d[6], &b, 8);
+    dst[e] = reinterpret_cast<const uint64_t*>(a.P.x.p)[(size_t)s * 7 + (e - 7u * q)];
   }
 }
 
@@ -86,7 +71,8 @@ hipError_t launch_up_to_soa3d(wpic_ctx3d* c, const double* aos, long long n, int
   a.np2 = which == 0 ? c->np2A : c->np2B;
   a.R = nullptr;
   a.aosbase = c->aosbase;
-  hipLaunchKernelGGL(k_aos_to_soa3, dim3((unsigned)(c->g.nsp * c->g.ncol)), dim3(256), 0, c->st, a, aos);
+  hipLaunchKernelGGL(k_records3_in, dim3((unsigned)(c->g.nsp * c->g.ncol)), dim3(256), 0, c->st, a,
+                     reinterpret_cast<const uint64_t*>(aos));
   return hipGetLastError();
 }
 
@@ -108,7 +94,8 @@ hipError_t launch_soa_to_aos3d(wpic_ctx3d* c, double* aos, int which) {
     a.R = nullptr;
   }
   a.aosbase = c->aosbase;
-  hipLaunchKernelGGL(k_soa_to_aos3, dim3((unsigned)(c->g.nsp * c->g.ncol)), dim3(256), 0, c->st, a, aos);
+  hipLaunchKernelGGL(k_records3_out, dim3((unsigned)(c->g.nsp * c->g.ncol)), dim3(256), 0, c->st, a,
+                     reinterpret_cast<uint64_t*>(aos));
   return hipGetLastError();
 }
 
@@ -250,22 +237,11 @@ __global__ void k_ic_beams3(Ic3Args a) {
   double ux = th * n0;
   if (electron) ux += (sl & 1) ? -a.udrift : a.udrift;
   if (MIXED) {
-    a.M.ix[d] = i;
-    a.M.ox[d] = to_offset(x - i);
-    a.M.oy[d] = to_offset(y - j);
-    a.M.oz[d] = to_offset(z - k);
-    a.M.ux[d] = (float)ux;
-    a.M.uy[d] = (float)(th * n1);
-    a.M.uz[d] = (float)(th * n2);
-    a.M.id[d] = (uint64_t)(-(q + 1));
+    const uint64_t id = (uint64_t)(-(q + 1));
+    store_rec(a.M, d, RecM3{i, to_offset(x - i), to_offset(y - j), to_offset(z - k), (float)ux, (float)(th * n1),
+                            (float)(th * n2), (uint32_t)id, (uint32_t)(id >> 32)});
   } else {
-    a.A.x[d] = x;
-    a.A.y[d] = y;
-    a.A.z[d] = z;
-    a.A.ux[d] = ux;
-    a.A.uy[d] = th * n1;
-    a.A.uz[d] = th * n2;
-    a.A.id[d] = (uint64_t)(-(q + 1));
+    store_rec(a.A, d, Rec3{x, y, z, ux, th * n1, th * n2, (uint64_t)(-(q + 1))});
   }
 }
 
