@@ -5,9 +5,10 @@
 // mom(7, nxgs-1:nxge+1, nys-1:nye+1, nsp) is kept in the reference's own
 // layout (the seven moments of a node contiguous), so transfers are plain
 // copies.  Three deposits:
-//   k_mom_tile<KICK>  fast: one workgroup per tile of cells accumulates the
-//                     tile's nodes (one-node halo) in LDS and adds them to
-//                     HBM once per node and species; with KICK it applies
+//   k_mom_tile<KICK>  fast: one workgroup per tile of cells sums a cell's
+//                     particles in registers, the tile's nodes (one-node
+//                     halo) in LDS, and adds those to HBM once per node and
+//                     species; with KICK it applies
 //                     mom_calc__accl's half-step kick on the fly (the fused
 //                     accl + nvt of the app's output sequence) and never
 //                     writes gp;
@@ -95,27 +96,22 @@ __global__ __launch_bounds__(NT) void k_mom_accl(MomArgs a) {
 // cell its slot belongs to (gp not sorted by cell) is added to HBM directly.
 // ---------------------------------------------------------------------------
 constexpr int MTW = TX + 2, MTH = TY + 2;
-#ifndef MOM_G
-#define MOM_G 8
-#endif
-
-// the seven moments of a particle rotated by r (out[q] = m[(q + r) % 7]),
-// r in 0..6, with three static conditional rotations
-__device__ inline void rotate7(double (&m)[7], int r) {
-  double t[7];
-#pragma unroll
-  for (int q = 0; q < 7; q++) t[q] = (r & 1) ? m[(q + 1) % 7] : m[q];
-#pragma unroll
-  for (int q = 0; q < 7; q++) m[q] = (r & 2) ? t[(q + 2) % 7] : t[q];
-#pragma unroll
-  for (int q = 0; q < 7; q++) t[q] = (r & 4) ? m[(q + 4) % 7] : m[q];
-#pragma unroll
-  for (int q = 0; q < 7; q++) m[q] = t[q];
-}
-
+// A particle of cell (i, j) adds to two of the nodes i-1, i, i+1 per axis, so a
+// cell's particles meet on 9 nodes: every lane sums those 9 x 7 values for the
+// particles it handles, the 8 lanes of the cell add up by halving exchanges
+// and each adds 8 of the 63 sums to the LDS tile.  Up to KP passes kick their
+// particles and leave dx, dy and the moments in registers, then the sums are
+// formed from those (next to the gather's reads in flight they would not fit).
+// A gp particle that left its cell is added to the tile by itself, or to HBM
+// when its node lies off it.
+//
+// What bounds it (1024x1024, 2 species of 64 ppc, with the kick): VALU issue,
+// half of it the kick, in 3.4 ms; the reads alone take 1.5.  28 LDS atomics a
+// particle, on planes rotated by the lane, took 3.8.
 template <bool KICK>
-__global__ __launch_bounds__(NT) void k_mom_tile(MomArgs a) {
-  constexpr int G = MOM_G, NGRP = NT / G;  // lanes per cell, cells in flight
+__global__ __launch_bounds__(NT, 2) void k_mom_tile(MomArgs a) {
+  constexpr int G = 8, KP = 4, RX = 64 / G;
+  static_assert(NT / 64 == TY, "one wave per tile row");
   __shared__ FieldPair sf[KICK ? 3 : 1][SFW * SFH];
   __shared__ double mt[7][MTW * MTH];
   const Grid2D& g = a.g;
@@ -124,87 +120,134 @@ __global__ __launch_bounds__(NT) void k_mom_tile(MomArgs a) {
   if (tile >= ntiles) return;
   const int i0 = g.nxgs + (tile % a.ntx) * TX;
   const int j0 = g.nys + (tile / a.ntx) * TY;
-  const int ncx = min(TX, g.nxge + 1 - i0), ncy = min(TY, g.nye + 1 - j0);
+  const int ncx = min(TX, g.nxge + 1 - i0);
   const int tid = threadIdx.x;
   if constexpr (KICK) stage_fields(g, a.uf, sf, i0, j0);
-  const double hdelt = g.delt * 0.5, d_delx = g.d_delx, c = g.c;
-  const int grp = tid / G, lg = tid % G;
-  // The lanes of a group work on one cell (and neighbouring groups on
-  // neighbouring cells), so their particles' nodes coincide; each lane walks
-  // the seven moment planes in an order rotated by its lane index, so that
-  // lanes meeting on a node at the same instruction mostly add to different
-  // planes.
-  const int rot = tid % 7;
+  const double hdelt = g.delt * 0.5, c = g.c;
+  const bool unit_c = c * c == 1.0;
+  const int lane = tid & 63, lg = lane % G;
+  const int lj = __builtin_amdgcn_readfirstlane(tid >> 6), j = j0 + lj;
 
   for (int s = 0; s < g.nsp; s++) {
     for (int k = tid; k < 7 * MTW * MTH; k += NT) (&mt[0][0])[k] = 0.0;
     __syncthreads();
-    for (int cc = grp; cc < TX * TY; cc += NGRP) {
-      const int li = cc % TX, lj = cc / TX;
-      if (li >= ncx || lj >= ncy) continue;  // uniform within a group
-      const int i = i0 + li, j = j0 + lj;
-      const int rw = s * g.ny + (j - g.nys);
-      const int* cr = a.cumcnt + (size_t)rw * (g.nx + 1);
-      const int base = a.rowbaseA[rw];
-      const int pe = base + cr[i - g.nxgs + 1];
-      for (int pi = base + cr[i - g.nxgs] + lg; pi < pe; pi += G) {
-        double x, y, ux, uy, uz;
-        if constexpr (KICK) {
-          const int ia = a.ap ? a.ap[pi] : pi;
-          x = a.A.x[ia];
-          y = a.A.y[ia];
-          double nxp, nyp, gmv;
-          boris_push(sf, li, lj, i, j, hdelt, c, true, a.fac1[s], a.txxx[s], a.fac2[s], x, y, a.A.ux[ia],
-                     a.A.uy[ia], a.A.uz[ia], nxp, nyp, ux, uy, uz, gmv);
-        } else {
-          x = a.B.x[pi];
-          y = a.B.y[pi];
-          ux = a.B.ux[pi];
-          uy = a.B.uy[pi];
-          uz = a.B.uz[pi];
-        }
-        const int ih = (int)(x * d_delx - 0.5), jh = (int)(y * d_delx - 0.5);
-        if (ih < g.nxgs - 1 || ih > g.nxge || jh < j - 1 || jh > j) {
-          atomicOr(a.err, ERR_DOMAIN);
-          continue;
-        }
-        const double dx = x * d_delx - 0.5 - ih, dxm = 1. - dx;
-        const double dy = y * d_delx - 0.5 - jh, dym = 1. - dy;
-        MomTerms m;
-        m.set(ux, uy, uz, c);
-        const int lx = ih - (i0 - 1), ly = jh - (j0 - 1);
-        if (lx < 0 || lx > ncx) {
-          // a gp particle whose node lies off this tile (gp not sorted by
-          // cell): straight to HBM
-          double* p00 = a.mom + midx(g, ih, jh, s);
-          double* p01 = a.mom + midx(g, ih, jh + 1, s);
+    const int rw = s * g.ny + (j - g.nys);
+    for (int l0 = 0; l0 < ncx && j <= g.nye; l0 += RX) {
+      const int li = l0 + lane / G, i = i0 + li;
+      int pe = 0, t = lg;
+      if (i <= g.nxge) {  // uniform within a group
+        const int* cr = a.cumcnt + (size_t)rw * (g.nx + 1) + (i - g.nxgs);
+        const int base = a.rowbaseA[rw];
+        t = base + cr[0] + lg;
+        pe = base + cr[1];
+      }
+      // (a cell's surplus lanes kick a particle at rest at its centre)
+      Rec pr = {i + 0.5, j + 0.5, 0.0, 0.0, 0.0, 0};
+      int ia_n = t + G;
+      if (KICK && a.ap) ia_n = t + G < pe ? a.ap[t + G] : 0;
+      if (t < pe) pr = KICK ? load_rec(a.A, a.ap ? a.ap[t] : t) : load_rec(a.B, t);
+      while (__any(t < pe)) {
+        double q[KP][8];  // dx, dy and the six moments u/gamma, u^2/gamma of the last KP passes, the latest first
+        int at[KP];       // node of dx, dy: bit 0 x, bit 1 y (0: i-1, j-1); -1: nothing to add
 #pragma unroll
-          for (int k = 0; k < 7; k++) {
-            unsafeAtomicAdd(p00 + k, m.term(k, dxm, dym));
-            unsafeAtomicAdd(p00 + 7 + k, m.term(k, dx, dym));
-            unsafeAtomicAdd(p01 + k, m.term(k, dxm, dy));
-            unsafeAtomicAdd(p01 + 7 + k, m.term(k, dx, dy));
+        for (int h = 0; h < KP; h++) {
+          at[h] = -1;
+#pragma unroll
+          for (int k = 0; k < 8; k++) q[h][k] = 0.0;
+        }
+        for (int h = 0; h < KP && __any(t < pe); h++, t += G) {
+          const Rec p = pr;
+          if (t + G < pe) pr = KICK ? load_rec(a.A, ia_n) : load_rec(a.B, t + G);
+          if (KICK) {
+            ia_n = t + 2 * G;
+            if (a.ap) ia_n = t + 2 * G < pe ? a.ap[t + 2 * G] : 0;
           }
-          continue;
-        }
-        double mv[7] = {1.0,
-                        m.u[0] * m.gam,
-                        m.u[1] * m.gam,
-                        m.u[2] * m.gam,
-                        m.u[0] * m.u[0] * m.gam,
-                        m.u[1] * m.u[1] * m.gam,
-                        m.u[2] * m.u[2] * m.gam};
-        rotate7(mv, rot);
-        const double w00 = dxm * dym, w10 = dx * dym, w01 = dxm * dy, w11 = dx * dy;
-        double* node = &mt[0][ly * MTW + lx];
+          double u[3] = {p.ux, p.uy, p.uz};
+          if constexpr (KICK) {
+            double nxp, nyp, gmv;
+            boris_push(sf, li, lj, i, j, hdelt, c, true, a.fac1[s], a.txxx[s], a.fac2[s], p.x, p.y, p.ux, p.uy, p.uz,
+                       nxp, nyp, u[0], u[1], u[2], gmv);
+          }
+          const int ih = (int)(p.x - 0.5), jh = (int)(p.y - 0.5);
+          const double u2 = +u[0] * u[0] + u[1] * u[1] + u[2] * u[2];
+          double root, gam;
+          sqrt_and_inverse(1.0 + (unit_c ? u2 : u2 / (c * c)), root, gam);
 #pragma unroll
-        for (int q = 0; q < 7; q++) {
-          const int plane = q + rot < 7 ? q + rot : q + rot - 7;
-          double* p = node + plane * (MTW * MTH);
-          atomicAdd(p, mv[q] * w00);
-          atomicAdd(p + 1, mv[q] * w10);
-          atomicAdd(p + MTW, mv[q] * w01);
-          atomicAdd(p + MTW + 1, mv[q] * w11);
+          for (int r = KP - 1; r > 0; r--) {
+            at[r] = at[r - 1];
+#pragma unroll
+            for (int k = 0; k < 8; k++) q[r][k] = q[r - 1][k];
+          }
+          const double dx = p.x - 0.5 - ih, dxm = 1. - dx, dy = p.y - 0.5 - jh, dym = 1. - dy;
+          double m[7] = {1.0};
+#pragma unroll
+          for (int d = 0; d < 3; d++) {
+            m[1 + d] = u[d] * gam;
+            m[4 + d] = u[d] * u[d] * gam;
+          }
+          const bool act = t < pe, in_cell = (unsigned)(ih - i + 1) < 2u && (unsigned)(jh - j + 1) < 2u;
+          const bool add = act && in_cell;
+          at[0] = add ? (ih - i + 1) | (jh - j + 1) << 1 : -1;
+          q[0][0] = dx;
+          q[0][1] = dy;
+#pragma unroll
+          for (int k = 1; k < 7; k++) q[0][1 + k] = add ? m[k] : 0.0;
+          if (act && !in_cell) {
+            if (ih < g.nxgs - 1 || ih > g.nxge || jh < j - 1 || jh > j) {
+              atomicOr(a.err, ERR_DOMAIN);
+            } else {
+              const int lx = ih - (i0 - 1), ly = jh - (j0 - 1);
+              const bool tiled = lx >= 0 && lx <= ncx;
+              double* const node = &mt[0][0] + (tiled ? ly * MTW + lx : 0);
+              double* const far = a.mom + midx(g, ih, jh, s);
+              const size_t up = (size_t)7 * (g.nx + 2);
+#pragma unroll
+              for (int k = 0; k < 7; k++) {
+                const double v[4] = {m[k] * (dxm * dym), m[k] * (dx * dym), m[k] * (dxm * dy), m[k] * (dx * dy)};
+                if (tiled) {
+                  double* const o = node + k * (MTW * MTH);
+                  atomicAdd(o, v[0]);
+                  atomicAdd(o + 1, v[1]);
+                  atomicAdd(o + MTW, v[2]);
+                  atomicAdd(o + MTW + 1, v[3]);
+                } else {
+                  unsafeAtomicAdd(far + k, v[0]);
+                  unsafeAtomicAdd(far + 7 + k, v[1]);
+                  unsafeAtomicAdd(far + up + k, v[2]);
+                  unsafeAtomicAdd(far + up + 7 + k, v[3]);
+                }
+              }
+            }
+          }
+        }
+        double v[63];  // [moment][y node][x node]
+#pragma unroll
+        for (int k = 0; k < 63; k++) v[k] = 0.0;
+#pragma unroll
+        for (int h = 0; h < KP; h++) {
+          if (!__any(at[h] >= 0)) continue;
+          const bool xr = at[h] & 1, yr = at[h] & 2;
+          const bool add = at[h] >= 0;
+          const double dx = add ? q[h][0] : 0.0, dxm = (add ? 1.0 : 0.0) - dx;
+          const double dy = add ? q[h][1] : 0.0, dym = 1. - dy;
+          const double wx[3] = {xr ? 0.0 : dxm, xr ? dxm : dx, xr ? dx : 0.0};
+          const double wy[3] = {yr ? 0.0 : dym, yr ? dym : dy, yr ? dy : 0.0};
+#pragma unroll
+          for (int e = 0; e < 9; e++) {
+            const double w = wx[e % 3] * wy[e / 3];
+            v[e] += w;
+#pragma unroll
+            for (int k = 1; k < 7; k++) v[9 * k + e] = fma(q[h][1 + k], w, v[9 * k + e]);
+          }
+        }
+        group_reduce<63, G>(v, lane);
+        int ln = lane;
+        asm volatile("" : "+v"(ln));  // (the places worked out here, not kept over the passes)
+#pragma unroll
+        for (int f = 0; f < group_left(63, G); f++) {
+          const int e = group_index<63, G>(f, ln);
+          if (i <= g.nxge && e >= 0 && v[f] != 0.0)
+            atomicAdd(&mt[0][0] + ((e / 9) * (MTW * MTH) + (lj + e % 9 / 3) * MTW + li + e % 3), v[f]);
         }
       }
     }
