@@ -3,7 +3,7 @@
 // 2d/proj/reconnection/boundary_reconnection.f90:61-99) at one rank.
 //
 // Particles of species s live in rows j = nys..nye, each row a contiguous
-// segment of the species' structure-of-arrays block.  The reference's in-row
+// segment of the species' block of records.  The reference's in-row
 // order after boundary_periodic__particle_y (leavers' slots refilled first by
 // arriving particles, then from the tail) followed by its stable bucket sort
 // is reproduced exactly, but computed in parallel:
