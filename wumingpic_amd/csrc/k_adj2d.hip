@@ -209,11 +209,15 @@ __device__ inline void spread5(const double a[3], int inc, double o[5]) {
   o[3] = l ? 0.0 : (r ? a[1] : a[2]);
   o[4] = r ? a[2] : 0.0;
 }
-// its transpose: the three values of five that spread5 fills
-__device__ inline void pick3(const double o[5], int inc, double a[3]) {
+// its transpose: the three values of five that spread5 fills (from scalars that
+// the compiler cannot see through: it would index an array in scratch)
+__device__ inline void pick3(const double v[5], int inc, double a[3]) {
   const bool l = inc < 0, r = inc > 0;
-#pragma unroll
-  for (int k = 0; k < 3; k++) a[k] = l ? o[k] : (r ? o[k + 2] : o[k + 1]);
+  double o0 = v[0], o1 = v[1], o2 = v[2], o3 = v[3], o4 = v[4];
+  asm volatile("" : "+v"(o0), "+v"(o1), "+v"(o2), "+v"(o3), "+v"(o4));
+  a[0] = l ? o0 : (r ? o2 : o1);
+  a[1] = l ? o1 : (r ? o3 : o2);
+  a[2] = l ? o2 : (r ? o4 : o3);
 }
 
 // One workgroup per tile of cells, as in the push: the tile's cell-centred
@@ -227,8 +231,10 @@ __device__ inline void pick3(const double o[5], int inc, double a[3]) {
 // per particle with every field, current and atomic in HBM took 6.57 ms at
 // 256x256, 16 ppc (54 field stencils, read twice, 65 current reads and 54
 // atomics a particle, and arrays indexed by the cell step in scratch); this
-// takes 0.255 ms.  At 1 wave a SIMD, without its 200 bytes of spills, it takes
-// 3 % of a whole backward pass longer.
+// took 0.255 ms with 224 bytes of scratch a thread.  Now 72 bytes (the node
+// table in LDS, lamB loaded where it is used, pick3 without an array): a pass of
+// 40 steps back 37.5 -> 35.5 ms.  At 1 wave a SIMD, without spills, it takes 3 %
+// of a whole backward pass longer.
 __global__ __launch_bounds__(256, 2) void k_adj_particles(AdjPArgs a) {
   constexpr int TX = 32, TY = 4, NT = 256, G = 8;
   constexpr int SFW = TX + 2, SFH = TY + 2, ACW = TX + 4, ACH = TY + 4;
@@ -273,17 +279,17 @@ __global__ __launch_bounds__(256, 2) void k_adj_particles(AdjPArgs a) {
 
   const double delt = g.delt, c2 = g.c * g.c;
   const size_t N = a.N;
-  const int w = tid >> 6, lane = tid & 63, lg = lane % G;
-  const int lj = w, j = j0 + lj;
-  // where this lane's sums of two components' 18 terms go in lt: component
-  // (0 or 1) and the node's offset from the cell's lower left neighbour
+  const int lj = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, lg = lane % G;
+  const int j = j0 + lj;
+  // where a lane's sums of two components' 18 terms go in lt, from the cell's
+  // lower left neighbour
   constexpr int NRES = group_left(18, G);
-  int node[NRES];
-#pragma unroll
-  for (int f = 0; f < NRES; f++) {
-    const int q = group_index<18, G>(f, lane);
-    node[f] = q < 0 ? -1 : (q / 9) * (SFW * SFH) + (q % 9 / 3) * SFW + q % 3;
+  __shared__ int node[NRES][G];
+  if (tid < NRES * G) {
+    const int q = group_index<18, G>(tid / G, tid % G);
+    node[tid / G][tid % G] = q < 0 ? -1 : (q / 9) * (SFW * SFH) + (q % 9 / 3) * SFW + q % 3;
   }
+  __syncthreads();
   for (int l0 = 0; l0 < a.tw; l0 += 64 / G) {
     const int li = l0 + lane / G, i = i0 + li;
     const bool live = i <= g.nxge && j <= g.nye;  // uniform within a group
@@ -316,10 +322,6 @@ __global__ __launch_bounds__(256, 2) void k_adj_particles(AdjPArgs a) {
       double G_xn = 0.0, G_yn = 0.0, G_g[3] = {0.0, 0.0, 0.0};
       if (act) {
         P = load_rec(a.P, p);
-        G_xn = a.lamB[p];
-        G_yn = a.lamB[N + p];
-#pragma unroll
-        for (int d = 0; d < 3; d++) G_g[d] = a.lamB[(2 + d) * N + p];
       }
       const double x = P.x, y = P.y, u[3] = {P.ux, P.uy, P.uz};
       const double fac1 = spc[s][0], txxx = spc[s][1], fac2 = spc[s][2], q = spc[s][3], qk = spc[s][4];
@@ -379,6 +381,13 @@ __global__ __launch_bounds__(256, 2) void k_adj_particles(AdjPArgs a) {
         dsy[m] -= s0y[m];
       }
       const double qvz = q * (gv[2] * gmv);
+      if (act) {
+        G_xn = a.lamB[p];
+        G_yn = a.lamB[N + p];
+#pragma unroll
+        for (int d = 0; d < 3; d++) G_g[d] = a.lamB[(2 + d) * N + p];
+      }
+      // (the phases one after another: interleaved, their values do not fit)
       // ---- reverse: deposit ----
       double G_dsx[5], G_dsy[5], G_s0x[5], G_s0y[5];
       {
@@ -546,8 +555,10 @@ __global__ __launch_bounds__(256, 2) void k_adj_particles(AdjPArgs a) {
         for (int k = 0; k < 18; k++) v[k] = G_F[cp + k / 9] * sx[k % 3] * sy[k % 9 / 3];
         group_reduce<18, G>(v, lane);
 #pragma unroll
-        for (int f = 0; f < NRES; f++)
-          if (live && node[f] >= 0) atomicAdd(&lt[cp][0] + (node[f] + so), v[f]);
+        for (int f = 0; f < NRES; f++) {
+          const int n = node[f][lg];
+          if (live && n >= 0) atomicAdd(&lt[cp][0] + (n + so), v[f]);
+        }
       }
     }
   }
