@@ -67,7 +67,7 @@ hipError_t launch_planes_to_aos(wpic_ctx* c, const double* planes, double* aos, 
 
 // which: 0 = A rows, 1 = B rows (through R when the exchange is pending),
 // 2 = B rows in B's own order.  aosbase lives in the staging tail.
-hipError_t launch_up_to_soa(wpic_ctx* c, const double* aos, long long n, int which) {
+hipError_t launch_records_in(wpic_ctx* c, const double* aos, long long n, int which) {
   (void)n;
   XferArgs a;
   a.g = c->g;
@@ -81,7 +81,7 @@ hipError_t launch_up_to_soa(wpic_ctx* c, const double* aos, long long n, int whi
   return hipGetLastError();
 }
 
-hipError_t launch_soa_to_aos(wpic_ctx* c, double* aos, int which) {
+hipError_t launch_records_out(wpic_ctx* c, double* aos, int which) {
   XferArgs a;
   a.g = c->g;
   a.P = which == 0 ? c->A : c->B;

@@ -62,7 +62,7 @@ hipError_t launch_planes_to_aos3d(wpic_ctx3d* c, const double* planes, double* a
 }
 
 // which: 0 = A columns, 1 = B seen through R (exchange pending), 2 = B columns
-hipError_t launch_up_to_soa3d(wpic_ctx3d* c, const double* aos, long long n, int which) {
+hipError_t launch_records_in3d(wpic_ctx3d* c, const double* aos, long long n, int which) {
   (void)n;
   Xfer3Args a;
   a.g = c->g;
@@ -76,7 +76,7 @@ hipError_t launch_up_to_soa3d(wpic_ctx3d* c, const double* aos, long long n, int
   return hipGetLastError();
 }
 
-hipError_t launch_soa_to_aos3d(wpic_ctx3d* c, double* aos, int which) {
+hipError_t launch_records_out3d(wpic_ctx3d* c, double* aos, int which) {
   Xfer3Args a;
   a.g = c->g;
   a.P = which == 0 ? c->A : c->B;

@@ -249,9 +249,10 @@ __device__ inline void tile_origin_m(const Grid3D& g, int tile, int ntx, int nty
 }
 
 // Its structure is that of k_push_deposit3d_fast.  What bounds it (256^3, 2
-// species of 16 ppc, 537 M particles): VALU issue and 43 GB of traffic in 20.3
-// ms, where one pass with the sums kept, one array per field, single LDS reads
-// and per-round queues took 28.5.  KP = 3, 4, 5, 6: 22.0, 21.4, 20.4, 20.4 ms.
+// species of 16 ppc, 537 M particles): VALU issue, 85 % of the SIMD cycles at 3
+// waves; 53 GB of traffic (43 algorithmic) in 20.3 ms.  One pass with the sums
+// kept, one array per field, single LDS reads and per-round queues took 28.5.
+// KP = 3, 4, 5, 6: 22.0, 21.4, 20.4, 20.4 ms.
 __global__ __launch_bounds__(m3::NT, 3) void k_push_deposit_mixed3d(Mix3Args a) {
 #pragma clang fp contract(fast)
   using namespace m3;

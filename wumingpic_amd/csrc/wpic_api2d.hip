@@ -565,7 +565,7 @@ static int upload_rows(wpic_ctx* c, int which, const double* up, const int* np2,
   if (c->mixed)
     HIPCHK(launch_up_to_mixed(c, c->staging));
   else
-    HIPCHK(launch_up_to_soa(c, c->staging, total, kind));
+    HIPCHK(launch_records_in(c, c->staging, total, kind));
   HIPCHK(hipStreamSynchronize(c->st));
   c->h_rows[which] = hrows;
   c->h_rows_ok[which] = true;
@@ -591,7 +591,7 @@ static int download_rows(wpic_ctx* c, int which, int kind, double* up, int* np2,
   if (c->mixed)
     HIPCHK(launch_mixed_to_aos(c, c->staging));
   else
-    HIPCHK(launch_soa_to_aos(c, c->staging, kind));
+    HIPCHK(launch_records_out(c, c->staging, kind));
   std::vector<double> h((size_t)total * 6);
   HIPCHK(hipMemcpyAsync(h.data(), c->staging, sizeof(double) * h.size(), hipMemcpyDeviceToHost, c->st));
   HIPCHK(hipStreamSynchronize(c->st));

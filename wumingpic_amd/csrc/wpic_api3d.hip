@@ -350,7 +350,7 @@ int upload_cols(wpic_ctx3d* c, int which, const double* up, const int* np2, int 
   if (kind == 3)
     HIPCHK(launch_up_to_mixed3d(c, c->staging));
   else
-    HIPCHK(launch_up_to_soa3d(c, c->staging, total, kind));
+    HIPCHK(launch_records_in3d(c, c->staging, total, kind));
   HIPCHK(hipStreamSynchronize(c->st));
   c->h_cols[which] = hcols;
   c->h_cols_ok[which] = true;
@@ -375,7 +375,7 @@ int download_cols(wpic_ctx3d* c, int which, int kind, double* up, int* np2, int 
   if (kind == 3)
     HIPCHK(launch_mixed_to_aos3d(c, c->staging));
   else
-    HIPCHK(launch_soa_to_aos3d(c, c->staging, kind));
+    HIPCHK(launch_records_out3d(c, c->staging, kind));
   std::vector<double> h((size_t)total * 7);
   HIPCHK(hipMemcpyAsync(h.data(), c->staging, sizeof(double) * h.size(), hipMemcpyDeviceToHost, c->st));
   HIPCHK(hipStreamSynchronize(c->st));

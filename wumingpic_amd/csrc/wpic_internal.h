@@ -298,7 +298,6 @@ constexpr int DPP_QUAD_XOR1 = 0xB1;  // quad_perm [1, 0, 3, 2]
 constexpr int DPP_QUAD_XOR2 = 0x4E;  // quad_perm [2, 3, 0, 1]
 constexpr int DPP_ROW_ROR4 = 0x124;
 constexpr int DPP_ROW_ROR8 = 0x128;
-constexpr int DPP_ROW_BCAST15 = 0x142;  // lane 15 of each row to the next row's lanes
 template <class T>
 __device__ inline T row16_sum(T v) {
   if constexpr (sizeof(T) == 8) {
@@ -326,23 +325,7 @@ __device__ inline double wave_sum(double v) {
   return (r[0] + r[1]) + (r[2] + r[3]);
 }
 
-// Sum over the 8 lanes of a half DPP row, every lane of the half receiving
-// it: quad permutes for the partners 1 and 2 apart, then the half-row mirror
-// (lane l and 7 - l), which pairs each quad with the other.
-constexpr int DPP_ROW_HALF_MIRROR = 0x141;
-template <class T>
-__device__ inline T row8_sum(T v) {
-  if constexpr (sizeof(T) == 8) {
-    v += dpp_f64<DPP_QUAD_XOR1>(v);
-    v += dpp_f64<DPP_QUAD_XOR2>(v);
-    v += dpp_f64<DPP_ROW_HALF_MIRROR>(v);
-  } else {
-    v += dpp_f32<DPP_QUAD_XOR1>(v);
-    v += dpp_f32<DPP_QUAD_XOR2>(v);
-    v += dpp_f32<DPP_ROW_HALF_MIRROR>(v);
-  }
-  return v;
-}
+constexpr int DPP_ROW_HALF_MIRROR = 0x141;  // lane l and 7 - l of each half row
 
 // Sums over the G lanes of a group (4, half a DPP row or a whole one) of N
 // values at once, each sum left in one lane.  Every step halves both the
@@ -639,8 +622,8 @@ hipError_t launch_rowbuild(wpic_ctx* c);
 hipError_t launch_rowsort(wpic_ctx* c);
 hipError_t launch_rowsort_fast(wpic_ctx* c);
 // transfers and initial state
-hipError_t launch_up_to_soa(wpic_ctx* c, const double* aos, long long n, int which);
-hipError_t launch_soa_to_aos(wpic_ctx* c, double* aos, int which);
+hipError_t launch_records_in(wpic_ctx* c, const double* aos, long long n, int which);
+hipError_t launch_records_out(wpic_ctx* c, double* aos, int which);
 hipError_t launch_planes_from_aos(wpic_ctx* c, const double* aos, double* planes, int ncomp);
 hipError_t launch_planes_to_aos(wpic_ctx* c, const double* planes, double* aos, int ncomp);
 hipError_t launch_ic_beams(wpic_ctx* c, unsigned long long seed, int n_ppc, double udrift, double uth_e,

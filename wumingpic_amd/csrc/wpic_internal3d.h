@@ -246,8 +246,8 @@ hipError_t launch_colsort3d(wpic_ctx3d* c);
 hipError_t launch_colsort3d_fast(wpic_ctx3d* c);
 hipError_t launch_codes_identity3d(wpic_ctx3d* c);
 // transfers and initial state
-hipError_t launch_up_to_soa3d(wpic_ctx3d* c, const double* aos, long long n, int which);
-hipError_t launch_soa_to_aos3d(wpic_ctx3d* c, double* aos, int which);
+hipError_t launch_records_in3d(wpic_ctx3d* c, const double* aos, long long n, int which);
+hipError_t launch_records_out3d(wpic_ctx3d* c, double* aos, int which);
 hipError_t launch_planes_from_aos3d(wpic_ctx3d* c, const double* aos, double* planes, int ncomp);
 hipError_t launch_planes_to_aos3d(wpic_ctx3d* c, const double* planes, double* aos, int ncomp);
 hipError_t launch_ic_beams3d(wpic_ctx3d* c, unsigned long long seed, int n_ppc, double udrift, double uth_e,
