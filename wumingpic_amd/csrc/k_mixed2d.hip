@@ -490,11 +490,12 @@ __global__ __launch_bounds__(mx::NT, 3) void k_push_deposit_mixed(MixArgs a) {
         if (nq >= 64) drain();
       }
     }
-    // the stayers' 21 sums over the group, spread over its lanes
+    // the stayers' 21 sums over the group, spread over its lanes (a cell without
+    // particles adds nothing: its fields may be any, and 0 * NaN is not 0)
     group_reduce<21, G>(v, lane);
 #pragma unroll
     for (int f = 0; f < NRES; f++)
-      if (live && node[f] >= 0 && v[f] != 0.0f) atomicAdd(&acc[0][0] + (node[f] + li), (double)v[f]);
+      if (tot > 0 && node[f] >= 0 && v[f] != 0.0f) atomicAdd(&acc[0][0] + (node[f] + li), (double)v[f]);
   }
   if (nq) drain();
 

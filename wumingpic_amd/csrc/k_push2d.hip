@@ -648,7 +648,8 @@ __global__ __launch_bounds__(NT, 2) void k_push_deposit_fast(PushArgs a) {
       }
     }
     if constexpr (DEPOSITS) {
-    // the stayers' 21 sums over the group, spread over its lanes
+    // the stayers' 21 sums over the group, spread over its lanes (a cell without
+    // particles adds nothing: its fields may be any, and 0 * NaN is not 0)
     double v[21];
 #pragma unroll
     for (int u = 0; u < 3; u++) {
@@ -663,7 +664,7 @@ __global__ __launch_bounds__(NT, 2) void k_push_deposit_fast(PushArgs a) {
     group_reduce<21, G>(v, lane);
 #pragma unroll
     for (int f = 0; f < NRES; f++)
-      if (live && node[f] >= 0 && v[f] != 0.0) atomicAdd(&acc[0][0] + (node[f] + li), v[f]);
+      if (tot > 0 && node[f] >= 0 && v[f] != 0.0) atomicAdd(&acc[0][0] + (node[f] + li), v[f]);
     }
   }
   if constexpr (DEPOSITS) {

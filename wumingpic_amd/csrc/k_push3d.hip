@@ -648,7 +648,8 @@ __global__ __launch_bounds__(p3::NT, 2) void k_push_deposit3d_fast(Push3Args a) 
         }
       }
     }
-    // over the group, spread over its lanes
+    // over the group, spread over its lanes (a cell without particles adds
+    // nothing: its fields may be any, and 0 * NaN is not 0)
     group_reduce<54, GF>(v, lane);
     // (the places are worked out here: kept over the passes they would spill)
     int ln = lane;
@@ -659,7 +660,7 @@ __global__ __launch_bounds__(p3::NT, 2) void k_push_deposit3d_fast(Push3Args a) 
       const int q = group_index<54, GF>(f, ln);
       const int c = q / 18, m = q % 18 / 9, u = q % 9 / 3 - 1, b = q % 3 - 1;
       const int xo = c == 0 ? m : u, yo = c == 0 ? u : (c == 1 ? m : b), zo = c == 2 ? m : b;
-      if (live && q >= 0 && v[f] != 0.0) atomicAdd(o + (c * AN + (zo * AH + yo) * AW + xo), v[f]);
+      if (tot > 0 && q >= 0 && v[f] != 0.0) atomicAdd(o + (c * AN + (zo * AH + yo) * AW + xo), v[f]);
     }
     }
   }
