@@ -222,6 +222,9 @@ struct alignas(16) FieldPair {
 //   residual x - g g (a fused multiply-add), which rounds it correctly; the
 //   reciprocal of g from 2 h by one Newton step and one correction with the
 //   exact residual 1 - g r (P. Markstein, IBM J. Res. Dev. 34, 111 (1990)).
+// That last correction rounds wrongly for one significand of the root, all ones
+// (its reciprocal lies just above the middle of two doubles): such roots, told
+// by their lower word, take the compiler's sequences as well.
 __device__ inline void sqrt_and_inverse(double x, double& root, double& inv) {
   const double y = __builtin_amdgcn_rsq(x);
   double g = x * y, h = 0.5 * y;
@@ -239,9 +242,10 @@ __device__ inline void sqrt_and_inverse(double x, double& root, double& inv) {
   r = fma(e, r, r);
   root = g;
   inv = r;
-  // exponent outside [-200, 200), sign or NaN (one branch for the wave: lanes
-  // that part here cost the caller's live registers a copy each)
-  const bool out = (unsigned)__double2hiint(x) - 0x33700000u >= 0x19000000u;
+  // exponent outside [-200, 200), sign or NaN, or the root's all ones (one branch
+  // for the wave: lanes that part here cost the caller's live registers a copy
+  // each)
+  const bool out = ((unsigned)__double2hiint(x) - 0x33700000u >= 0x19000000u) | (__double2loint(g) == -1);
   if (__builtin_expect(__any(out), 0)) {
     const double q = sqrt(x);
     root = out ? q : g;
