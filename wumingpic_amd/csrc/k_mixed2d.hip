@@ -78,21 +78,24 @@ __device__ inline float rcpf(float x) { return __builtin_amdgcn_rcpf(x); }
 __device__ inline float rsqf(float x) { return __builtin_amdgcn_rsqf(x); }
 
 // The 4-node window [lo, lo + 3] (of the 5 nodes -2..2) of one axis that holds
-// every non-zero s0 and ds of a particle with |inc| <= 1: S0 and DS on it
+// every non-zero s0 and ds: S0 and DS on it, the new shape with the reference's
+// weights, |inc| moved by one node and 1 - |inc| unmoved, as in the FP64 kernel
 __device__ inline void window_f(float o, float f, int inc, float S0[4], float DS[4], int& lo) {
   float t0, t1, t2, u0, u1, u2;
   shape3f(o - 0.5f, t0, t1, t2);
   shape3f(f - 0.5f, u0, u1, u2);
-  const bool left = inc < 0, right = inc > 0;
+  const bool left = inc < 0;
   lo = left ? 0 : 1;
+  const float far = (float)abs(inc), near = 1.0f - far;
+  const float p = left ? far : near, q = left ? near : far;
   S0[0] = left ? 0.0f : t0;
   S0[1] = left ? t0 : t1;
   S0[2] = left ? t1 : t2;
   S0[3] = left ? t2 : 0.0f;
-  DS[0] = (right ? 0.0f : u0) - S0[0];
-  DS[1] = (right ? u0 : u1) - S0[1];
-  DS[2] = (right ? u1 : u2) - S0[2];
-  DS[3] = (right ? u2 : 0.0f) - S0[3];
+  DS[0] = p * u0 - S0[0];
+  DS[1] = p * u1 + q * u0 - S0[1];
+  DS[2] = p * u2 + q * u1 - S0[2];
+  DS[3] = q * u2 - S0[3];
 }
 
 // The fields of a cell side by side, so that the gather's 54 values come in 18

@@ -295,10 +295,13 @@ __device__ inline void deposit2_full(double (*acc)[ACW * ACH], int li, int lj, c
   }
 }
 
-// The same current of a particle with |inc| <= 1 (any particle where no wall
-// reflects it): the 4-node window [lo, lo + 3] of the 5 nodes -2..2 per axis,
-// lo = 0 for a step to the left and 1 otherwise, holds every non-zero s0 and
-// ds, so the block is 12 + 12 + 16 values instead of 65.
+// The same current on the 4-node window [lo, lo + 3] of the 5 nodes -2..2 per
+// axis, lo = 0 for a step to the left and 1 otherwise, which holds every
+// non-zero s0 and ds: 12 + 12 + 16 values instead of 65.  The new shape at its
+// nodes carries the reference's weights (field.f90:244-266), |inc| moved by one
+// node and 1 - |inc| unmoved: a plain shift for a step of one cell (where the
+// products are exact), and what the reference does where a particle near c
+// rounds across two faces (c delt = delx allows that in x).
 __device__ inline void shapes_window(double old, double nw, int cell, double S0[4], double DS[4], int& lo) {
   double t0, t1, t2, u0, u1, u2;
   shape3(old - 0.5 - cell, t0, t1, t2);
@@ -306,17 +309,18 @@ __device__ inline void shapes_window(double old, double nw, int cell, double S0[
   shape3(nw - 0.5 - c2, u0, u1, u2);
   const bool left = inc < 0;
   lo = left ? 0 : 1;
-  // old shape on window nodes 1..3 (left) or 0..2; new one on 0..2 (left),
-  // 1..3 (right) or 0..2 (unmoved along this axis)
+  const double far = (double)abs(inc), near = 1.0 - far;
+  const double p = left ? far : near, q = left ? near : far;
+  // old shape on window nodes 1..3 (left) or 0..2; of the new one p on 0..2 and
+  // q on 1..3
   S0[0] = left ? 0.0 : t0;
   S0[1] = left ? t0 : t1;
   S0[2] = left ? t1 : t2;
   S0[3] = left ? t2 : 0.0;
-  const bool right = inc > 0;
-  DS[0] = (right ? 0.0 : u0) - S0[0];
-  DS[1] = (right ? u0 : u1) - S0[1];
-  DS[2] = (right ? u1 : u2) - S0[2];
-  DS[3] = (right ? u2 : 0.0) - S0[3];
+  DS[0] = p * u0 - S0[0];
+  DS[1] = p * u1 + q * u0 - S0[1];
+  DS[2] = p * u2 + q * u1 - S0[2];
+  DS[3] = q * u2 - S0[3];
 }
 
 __device__ inline void deposit2_window(double (*acc)[ACW * ACH], int li, int lj, int i, int j, double x, double y,

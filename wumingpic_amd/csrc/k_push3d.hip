@@ -317,10 +317,12 @@ __global__ __launch_bounds__(256) void k_gather_pj3d(Grid3D g, const double* __r
 // (x - 0.5 - cell per axis, field.f90:253-266) and its cell increments, added
 // to the LDS tile: o is the tile's Jx at the particle's cell.  The 4-node
 // window [lo, lo + 3] of the 5 nodes -2..2 per axis, lo = 0 for a step to the
-// left and 1 otherwise, holds every non-zero s0 and ds when |inc| <= 1.  An
-// axis along which the particle keeps its cell has nothing on its fourth node
-// and only rounding on its third face, so a step along one axis costs 75
-// atomics and one along all three 144.
+// left and 1 otherwise, holds every non-zero s0 and ds; the new shape carries
+// the reference's weights there, |inc| moved by one node and 1 - |inc| unmoved
+// (a plain shift for a step of one cell; a particle near c may round across two
+// faces in x).  An axis along which the particle keeps its cell has nothing on
+// its fourth node and only rounding on its third face, so a step along one axis
+// costs 75 atomics and one along all three 144.
 __device__ inline void deposit3_window(double* o, const double dh0[3], const double dh1[3], const int inc[3],
                                        double qd) {
   using namespace p3;
@@ -332,17 +334,19 @@ __device__ inline void deposit3_window(double* o, const double dh0[3], const dou
     double t0, t1, t2, u0, u1, u2;
     shape3(dh0[d], t0, t1, t2);
     shape3(dh1[d], u0, u1, u2);
-    const bool left = inc[d] < 0, right = inc[d] > 0;
-    mv[d] = left || right;
+    const bool left = inc[d] < 0;
+    mv[d] = inc[d] != 0;
+    const double far = (double)abs(inc[d]), near = 1.0 - far;
+    const double p = left ? far : near, q = left ? near : far;
     o += (left ? -2 : -1) * (d == 0 ? 1 : (d == 1 ? SY : SZ));  // window node 0 of the axis
     S[d][0] = left ? 0.0 : t0;
     S[d][1] = left ? t0 : t1;
     S[d][2] = left ? t1 : t2;
     S[d][3] = left ? t2 : 0.0;
-    D[d][0] = (right ? 0.0 : u0) - S[d][0];
-    D[d][1] = (right ? u0 : u1) - S[d][1];
-    D[d][2] = (right ? u1 : u2) - S[d][2];
-    D[d][3] = (right ? u2 : 0.0) - S[d][3];
+    D[d][0] = p * u0 - S[d][0];
+    D[d][1] = p * u1 + q * u0 - S[d][1];
+    D[d][2] = p * u2 + q * u1 - S[d][2];
+    D[d][3] = q * u2 - S[d][3];
     double run = 0.0;
 #pragma unroll
     for (int m = 0; m < 3; m++) {
@@ -437,7 +441,7 @@ __global__ __launch_bounds__(p3::NT, 2) void k_push_deposit3d_fast(Push3Args a) 
   __shared__ double acc[3][AN];
   __shared__ double spc[WPIC_MAXSP][4];  // fac1, txxx, fac2, q delx / delt
   // the waves' queued particles: old and new shape arguments per axis, and
-  // cell in the tile | species << 7 | (inc + 1) per axis << 9, 11, 13
+  // cell in the tile | species << 7 | (inc + 4) per axis << 9, 12, 15
   __shared__ double xqd[NW][6][QW];
   __shared__ int xqc[NW][QW];
   const Grid3D& g = a.g;
@@ -479,7 +483,7 @@ __global__ __launch_bounds__(p3::NT, 2) void k_push_deposit3d_fast(Push3Args a) 
     if (q < nq) {
       const int e = xqc[w][q];
       const int cc = e & 127, s = (e >> 7) & 3;
-      const int inc[3] = {((e >> 9) & 3) - 1, ((e >> 11) & 3) - 1, ((e >> 13) & 3) - 1};
+      const int inc[3] = {((e >> 9) & 7) - 4, ((e >> 12) & 7) - 4, ((e >> 15) & 7) - 4};
       const double dh0[3] = {xqd[w][0][q], xqd[w][1][q], xqd[w][2][q]};
       const double dh1[3] = {xqd[w][3][q], xqd[w][4][q], xqd[w][5][q]};
       deposit3_window(&acc[0][((cc / (TX * TY) + 2) * AH + (cc / TX % TY + 2)) * AW + (cc % TX + 2)], dh0, dh1, inc,
@@ -600,8 +604,8 @@ __global__ __launch_bounds__(p3::NT, 2) void k_push_deposit3d_fast(Push3Args a) 
                                                                __builtin_amdgcn_mbcnt_lo((uint32_t)mm, 0));
 #pragma unroll
           for (int d = 0; d < 6; d++) xqd[w][d][slot] = pd[0][d];
-          xqc[w][slot] = ((lk * TY + lj) * TX + li) | (s << 7) | (((i2 - i + 1) & 3) << 9) |
-                         (((j2 - j + 1) & 3) << 11) | (((k2 - k + 1) & 3) << 13);
+          xqc[w][slot] = ((lk * TY + lj) * TX + li) | (s << 7) | (((i2 - i + 4) & 7) << 9) |
+                         (((j2 - j + 4) & 7) << 12) | (((k2 - k + 4) & 7) << 15);
         }
         nq += __popcll(mm);
         if (nq >= 64) drain();
