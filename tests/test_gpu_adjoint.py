@@ -68,3 +68,25 @@ def test_adjoint_called_from_fortran_matches_the_harness():
     wb.backward()
     assert abs(wb_f - float(wb.detach())) <= 1e-12 * abs(wb_f)
     assert np.allclose(g_f, t.grad.numpy(), rtol=1e-9, atol=0)
+
+
+def test_a_run_recorded_after_a_backward_pass_starts_from_the_state_it_left():
+    """include/wpic_adj.h: the context then holds the end of the first segment; recording again frees
+    the record that its particles were read through. Rounding alone (the order of the current's
+    atomics) parts it from a context stepped there: 1e-9 of the largest value after 4 steps."""
+    from wumingpic_amd.adjoint import WeibelCase, make_sim
+    case = WeibelCase(nx=32, ny=32, n_ppc=8, nsteps=6, every=3)
+    with make_sim(case, 0.5, 0.1, 1e-3) as sim, make_sim(case, 0.5, 0.1, 1e-3) as ref:
+        sim.adj_forward(case.nsteps, case.every)
+        sim.adj_backward(1.0)
+        ref.step(case.every)
+        wb, wb_ref = sim.adj_forward(4, 2), ref.adj_forward(4, 2)
+        assert abs(wb - wb_ref) <= 1e-9 * abs(wb_ref)
+        assert np.abs(sim.download_fields() - ref.download_fields()).max() <= 1e-9 * np.abs(ref.download_fields()).max()
+        for s in (sim, ref):
+            s.adj_backward(1.0)
+        lam, lam_ref = (s.adj_download(2 * 8 * 32)[1] for s in (sim, ref))
+        assert np.abs(lam - lam_ref).max() <= 1e-9 * np.abs(lam_ref).max()
+        sim.step(1)
+        ref.step(1)
+        assert np.abs(sim.download_fields() - ref.download_fields()).max() <= 1e-9 * np.abs(ref.download_fields()).max()

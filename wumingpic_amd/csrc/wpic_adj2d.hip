@@ -41,6 +41,10 @@ namespace wpic {
 void adj_free(wpic_ctx* c) {
   AdjState* a = c->adj;
   if (!a) return;
+  // after a replay A is read through the record's permutation of its last step:
+  // that buffer becomes the context's own, which goes in its place
+  for (auto& p : a->st_perm)
+    if (p && p == c->aperm) std::swap(p, c->permbuf);
   auto fr = [](void* p) {
     if (p) (void)hipFree(p);
   };
@@ -140,6 +144,8 @@ int alloc_adj(wpic_ctx* c, int nsteps, int every) {
     e = dal(&a.st_part[t], PART_DOUBLES * a.N);
     if (e == hipSuccess) e = dal(&a.st_uf[t], 6 * a.pl);
     if (e == hipSuccess) e = dal(&a.st_perm[t], a.N);
+    // (as the context's own: every entry is a slot, whether a sort wrote it or not)
+    if (e == hipSuccess) e = hipMemsetAsync(a.st_perm[t], 0, sizeof(int) * a.N, c->st);
     if (e == hipSuccess) e = dal(&a.st_cumcnt[t], (size_t)a.ncc);
   }
   for (int t = 0; t <= K && e == hipSuccess; t++) e = dal(&a.st_rows[t], (size_t)2 * a.nr);
