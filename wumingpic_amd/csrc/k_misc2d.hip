@@ -21,10 +21,10 @@ struct XferArgs {
 // (raw 64-bit words: a record is the reference's own six)
 __global__ void k_records_in(XferArgs a, const uint64_t* __restrict__ aos) {
   const int rw = blockIdx.x;
-  const int base = a.rowbase[rw], n = a.np2[rw];
+  const size_t n = (size_t)a.np2[rw] * PART_DOUBLES;
   const uint64_t* src = aos + a.aosbase[rw] * PART_DOUBLES;
-  uint64_t* dst = reinterpret_cast<uint64_t*>(a.P.x.p) + (size_t)base * PART_DOUBLES;
-  for (int k = threadIdx.x; k < n * PART_DOUBLES; k += blockDim.x) dst[k] = src[k];
+  uint64_t* dst = reinterpret_cast<uint64_t*>(a.P.x.p) + (size_t)a.rowbase[rw] * PART_DOUBLES;
+  for (size_t e = threadIdx.x; e < n; e += blockDim.x) dst[e] = src[e];
 }
 
 __global__ void k_records_out(XferArgs a, uint64_t* __restrict__ aos) {

@@ -25,13 +25,13 @@ __global__ void k_records3_in(Xfer3Args a, const uint64_t* __restrict__ aos) {
 __global__ void k_records3_out(Xfer3Args a, uint64_t* __restrict__ aos) {
   const int rw = blockIdx.x;
   const int base = a.colbase[rw];
-  const unsigned n = (unsigned)a.np2[rw] * 7u;
+  const size_t n = (size_t)a.np2[rw] * 7;
   uint64_t* dst = aos + a.aosbase[rw] * 7;
-  for (unsigned e = threadIdx.x; e < n; e += blockDim.x) {
-    const unsigned q = e / 7u;
-    int s = a.R ? a.R[base + (int)q] : base + (int)q;
+  for (size_t e = threadIdx.x; e < n; e += blockDim.x) {
+    const int q = (int)(e / 7);
+    int s = a.R ? a.R[base + q] : base + q;
     if ((unsigned)s >= (unsigned)(a.g.ncap * a.g.nsp)) s = 0;
-    dst[e] = reinterpret_cast<const uint64_t*>(a.P.x.p)[(size_t)s * 7 + (e - 7u * q)];
+    dst[e] = reinterpret_cast<const uint64_t*>(a.P.x.p)[(size_t)s * 7 + (e - (size_t)7 * q)];
   }
 }
 
