@@ -147,9 +147,11 @@ int check_err(wpic_ctx* c) {
   return 0;
 }
 
-int ensure_pjbuf(wpic_ctx* c) {
-  if (c->pjbuf) return 0;
-  HIPCHK(dalloc(&c->pjbuf, (size_t)c->g.nx * c->g.ny * 65));
+// what the parity mode alone uses
+int ensure_parity(wpic_ctx* c) {
+  const size_t nc = (size_t)c->g.nx * c->g.ny;
+  if (!c->pjbuf) HIPCHK(dalloc(&c->pjbuf, nc * 65));
+  if (!c->ap) HIPCHK(dalloc(&c->ap, nc * 3));
   return 0;
 }
 
@@ -226,7 +228,7 @@ int deposit(wpic_ctx* c, bool push) {
   }
   const bool parity = c->mode == WPIC_MODE_PARITY;
   if (parity) {
-    int rc = ensure_pjbuf(c);
+    int rc = ensure_parity(c);
     if (rc) return rc;
   } else {
     HIPCHK(launch_zero(c, c->uj, (size_t)3 * c->g.fw * c->g.fh));
@@ -450,7 +452,7 @@ int wpic_create2d(wpic_ctx** out, const wpic_params2d* p) {
   if (e == hipSuccess) e = dalloc(&c->uf, 6 * pl);
   if (e == hipSuccess) e = dalloc(&c->df, 6 * pl);
   if (e == hipSuccess) e = dalloc(&c->uj, 3 * pl);
-  double** cg[] = {&c->phi, &c->pa, &c->pb, &c->rr, &c->bb, &c->ap};
+  double** cg[] = {&c->phi, &c->pa, &c->pb, &c->rr, &c->bb};
   for (auto q : cg)
     if (e == hipSuccess) e = dalloc(q, 3 * nc);
   if (e == hipSuccess) e = dalloc(&c->part, (size_t)3 * 3 * NPB);

@@ -157,9 +157,12 @@ void segment_table(const Grid3D& g, std::vector<int>& seg, std::vector<int>& nse
     }
 }
 
-int ensure_pjbuf3(wpic_ctx3d* c) {
-  if (c->pjbuf) return 0;
-  HIPCHK(dalloc(&c->pjbuf, (size_t)c->g.nx * c->g.ny * c->g.nz * 300));
+// what the parity mode alone uses
+int ensure_parity3(wpic_ctx3d* c) {
+  const size_t nc = (size_t)c->g.nx * c->g.ny * c->g.nz;
+  if (!c->pjbuf) HIPCHK(dalloc(&c->pjbuf, nc * 300));
+  if (!c->bb) HIPCHK(dalloc(&c->bb, nc * 3));
+  if (!c->ap) HIPCHK(dalloc(&c->ap, nc * 3));
   return 0;
 }
 
@@ -210,7 +213,7 @@ int field_after_deposit3(wpic_ctx3d* c) {
 int deposit3(wpic_ctx3d* c) {
   const bool parity = c->mode == WPIC_MODE_PARITY;
   if (parity) {
-    int rc = ensure_pjbuf3(c);
+    int rc = ensure_parity3(c);
     if (rc) return rc;
   } else {
     HIPCHK(launch_fill3d(c, c->uj, 3 * plane3(c->g), 0.0));
@@ -524,7 +527,7 @@ int wpic_create3d(wpic_ctx3d** out, const wpic_params3d* p) {
   if (e == hipSuccess) e = dalloc(&c->uf, 6 * pl);
   if (e == hipSuccess) e = dalloc(&c->df, 6 * pl);
   if (e == hipSuccess) e = dalloc(&c->uj, 3 * pl);
-  double** cg[] = {&c->phi, &c->pa, &c->pb, &c->rr, &c->bb, &c->ap};
+  double** cg[] = {&c->phi, &c->pa, &c->pb, &c->rr};
   for (auto q : cg)
     if (e == hipSuccess) e = dalloc(q, 3 * nc);
   if (e == hipSuccess) e = dalloc(&c->part, (size_t)3 * 3 * NPB3);

@@ -543,7 +543,8 @@ struct wpic_ctx {
   double* pjbuf;  // parity-mode per-cell current blocks [nx*ny][65]
 
   // CG: interior vectors per component
-  double *phi, *pa, *pb, *rr, *bb, *ap;  // [3][nx*ny]
+  double *phi, *pa, *pb, *rr;            // [3][nx*ny]
+  double *bb, *ap;                       // [3][nx*ny] b (parity mode, adjoint) and A p (parity mode, lazy)
   double* part;                          // block partial sums [3][3][NPB]
   wpic::CgScal* scal;                    // [2][3]
   int* err;                              // device error bits

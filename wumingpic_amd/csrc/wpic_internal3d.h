@@ -189,7 +189,8 @@ struct wpic_ctx3d {
   double *uf, *df, *uj;  // 6, 6, 3 components of (nx+4)(ny+4)(nz+4)
   double* pjbuf;         // parity deposit blocks [nx*ny*nz][300] (lazy)
 
-  double *phi, *pa, *pb, *rr, *bb, *ap;  // CG vectors [3][nx*ny*nz]
+  double *phi, *pa, *pb, *rr;  // CG vectors [3][nx*ny*nz]
+  double *bb, *ap;             // b and A p, parity mode (lazy)
   double* part;              // block partial sums [3][3][NPB3]
   wpic::CgScal* scal;        // [2][3]
   wpic::CgPoll* poll;        // pinned host memory
