@@ -90,3 +90,17 @@ def test_a_run_recorded_after_a_backward_pass_starts_from_the_state_it_left():
         sim.step(1)
         ref.step(1)
         assert np.abs(sim.download_fields() - ref.download_fields()).max() <= 1e-9 * np.abs(ref.download_fields()).max()
+
+
+@pytest.mark.parametrize("nx, ny", [(37, 30), (250, 131), (250, 259)], ids=["8 columns", "16 columns", "32 columns"])
+def test_adjoint_gradients_on_ragged_tiles(nx, ny):
+    """the particle kernel's tile widths, each with a last tile that is not full in x and in y"""
+    from wumingpic_amd.adjoint import WeibelCase, WeibelMagneticEnergy
+    print(nx, ny, flush=True)
+    case = WeibelCase(nx=nx, ny=ny, n_ppc=4, nsteps=6, every=4)
+    theta = [0.5, 0.1, 1e-3]
+    t = torch.tensor(theta, dtype=torch.float64, requires_grad=True)
+    WeibelMagneticEnergy.apply(t, case).backward()
+    grad, fd = t.grad.numpy(), _fd(case, theta)
+    rel = np.abs(grad - fd) / np.abs(fd)
+    assert (rel <= 1e-3).all(), (grad, fd, rel)

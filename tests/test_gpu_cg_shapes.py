@@ -62,3 +62,33 @@ def test_field_solve_3d(nx, ny, nz):
     print(nx, ny, nz, flush=True)
     sim = Pic3D(nx, ny, nz, list(p.q)[:2], list(p.r)[:2], delt=0.5, mode=MODE_FAST, capacity=nx * ny * nz)
     _check(sim, po.Oracle3D(p), p, up, cc, np2, uf)
+
+
+@pytest.mark.parametrize("n", [(64, 66000), (1056, 520, 3)], ids=["4125 strips", "2145 tiles"])
+def test_field_solve_with_more_work_units_than_blocks(n):
+    """each block (2D: wave) takes several units; no particles, so the fields alone drive the solve.
+    The oracle adds 4.2e6 terms one after another, about sqrt(4.2e6) 1e-16 off per dot product and
+    some ten iterations of two: 1e-11 of the largest value."""
+    from wumingpic_amd import MODE_FAST
+    from wumingpic_amd.pic2d import Pic2D
+    from wumingpic_amd.pic3d import Pic3D
+    rng = np.random.default_rng(5)
+    q, r = S.weibel_consts(1)
+    print(n, flush=True)
+    if len(n) == 2:
+        p = po.make_params(*n, np_cap=1, delt=0.5, q=q, r=r)
+        o, (up, gp, _, cc, np2) = po.Oracle2D(p), po.alloc_state(p)
+        uf = np.asfortranarray(S.periodic_fill_fields(p, S.random_fields(p, rng, scale=0.02)))
+    else:
+        p = po.make_params3d(*n, np_cap=1, delt=0.5, q=q, r=r)
+        o, (up, gp, _, cc, np2) = po.Oracle3D(p), po.alloc_state3d(p)
+        uf = S3.periodic_fill_fields3d(p, S3.random_fields3d(p, rng, scale=0.02))
+    with (Pic2D if len(n) == 2 else Pic3D)(*n, list(q), list(r), delt=0.5, mode=MODE_FAST, capacity=1) as sim:
+        sim.upload_up(up, np2, cc)
+        sim.upload_fields(uf)
+        for _ in range(2):
+            sim.particle_solv()
+            assert tuple(sim.field_fdtd_i()) == tuple(o.field_fdtd_i(uf, up, gp, cc))
+            got = sim.download_dfield()
+            assert np.abs(got - o.df).max() <= 1e-11 * np.abs(o.df).max()
+            assert np.abs(sim.download_fields() - uf).max() <= 1e-11 * np.abs(uf).max()
