@@ -200,7 +200,9 @@ struct AdjPArgs {
   int ntx, nty, tw;
 };
 
-// (a, b, c) at nodes 0..4 of five, shifted from 1..3 by inc in {-1, 0, 1}
+// (a, b, c) at nodes 0..4 of five, shifted from 1..3 by inc in {-1, 0, 1} (a
+// step over two faces, which only rounding makes, at c delt = delx, has no
+// derivative and counts as one)
 __device__ inline void spread5(const double a[3], int inc, double o[5]) {
   const bool l = inc < 0, r = inc > 0;
   o[0] = l ? a[0] : 0.0;

@@ -312,11 +312,6 @@ __global__ void k_cg_parity_b(CgArgs a) {
 // loads what `node(q, p, ap, words)` needs of its own, ap being f4 p - the sum
 // of the four neighbours.  `scal()` runs after the first loads are on their
 // way, by all of the block, and says whether to go on.
-template <int CTRL>
-__device__ inline double lane_shift(double v) {
-  return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, false),
-                          __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, false));
-}
 template <class Load, class Val, class Pre, class Node, class Scal>
 __device__ inline void march2(const Grid2D& g, int nb, int l, Load load, Val val, Pre pre, Node node, Scal scal) {
   constexpr int WAVE_SHL1 = 0x130, WAVE_SHR1 = 0x138;  // from the lane above, below
@@ -364,7 +359,7 @@ __device__ inline void march2(const Grid2D& g, int nb, int l, Load load, Val val
         if (bw) hw = load(at(iw, j + 1));
         if (be) he = load(at(ie, j + 1));
       }
-      double pW = lane_shift<WAVE_SHR1>(pC), pE = lane_shift<WAVE_SHL1>(pC);
+      double pW = dpp_f64<WAVE_SHR1>(pC), pE = dpp_f64<WAVE_SHL1>(pC);
       if (bw) pW = signed_val(sw, hwv);
       if (be) pE = signed_val(se, hev);
       if (act) node(cidx(g, i, j), pC, -pB - pW + f4 * pC - pE - pT, mine);

@@ -367,9 +367,10 @@ __device__ inline void march3(const Grid3D& g, int nb, double (*sm)[SM3], Load l
 // 2D: every block of k_cg3_a adds the partial sums of r.r, every block of
 // k_cg3_b those of p.ap, in the same order; k_cg3_b forms ap again from p.
 //
-// What bounds it at 256^3: 3.2 GB an iteration through march3 in about 0.9 ms
-// (3.5 TB/s where a plain copy reaches 4.8); on small grids the launches, as in
-// 2D.  A whole solve of 8 iterations with its right-hand side, next to the sort
+// What bounds it at 256^3: traffic, 4.6 GB an iteration in 0.86 ms (5.3 TB/s, a
+// part of it from the cache behind L2) where the arrays themselves are 3.2 GB:
+// a 32-column tile reads whole lines for its one-column halos.  On small grids
+// the launches, as in 2D.  A whole solve of 8 iterations with its right-hand side, next to the sort
 // on the other stream: 67x45x38 365 -> 212 us, 64^3 430 -> 286, 160x144x128
 // 2.19 -> 1.69 ms, 256^3 11.8 -> 8.5.  Without the loads ahead of the level in
 // work and with two barriers a level the new form was no faster than the old.

@@ -167,8 +167,8 @@ __device__ inline Mix3Push mixed_push3(const Mix3Const& mc, const Field4M* fa, c
 }
 
 // Current of one particle that changes cell, added to the FP64 tile with the
-// window of k_push_deposit3d_fast (|inc| <= 1): o is the tile's Jx at the
-// particle's cell.
+// window of k_push_deposit3d_fast (|inc| <= 1; a longer step is reported): o is
+// the tile's Jx at the particle's cell.
 __device__ inline void deposit3_window_m(double* o, const float dh0[3], const float dh1[3], const int inc[3],
                                          float qd) {
 #pragma clang fp contract(fast)

@@ -104,7 +104,7 @@ __global__ __launch_bounds__(p3::NT) void k_mom_accl3d(Mom3Args a) {
       for (int pi = base + cr[i - g.nxgs] + lg; pi < pend; pi += G) {
         const int ia = a.ap ? a.ap[pi] : pi;
         const double x = a.A.x[ia], y = a.A.y[ia], z = a.A.z[ia];
-        double nxp, nyp, nzp, g4, g5, g6, sh[9];
+        double nxp, nyp, nzp, g4, g5, g6;
         boris_push3(sf, so, i, j, k, hdelt, g.c, a.fac1[s], a.txxx[s], a.fac2[s], x, y, z, a.A.ux[ia],
                     a.A.uy[ia], a.A.uz[ia], nxp, nyp, nzp, g4, g5, g6);
         a.B.x[pi] = x;
@@ -187,7 +187,7 @@ __global__ __launch_bounds__(p3::NT) void k_mom3d_tile(Mom3Args a) {
           x = a.A.x[ia];
           y = a.A.y[ia];
           z = a.A.z[ia];
-          double nxp, nyp, nzp, sh[9];
+          double nxp, nyp, nzp;
           boris_push3(sf, so, i, j, k, hdelt, c, a.fac1[s], a.txxx[s], a.fac2[s], x, y, z, a.A.ux[ia],
                       a.A.uy[ia], a.A.uz[ia], nxp, nyp, nzp, ux, uy, uz);
         } else {

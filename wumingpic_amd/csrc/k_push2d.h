@@ -99,8 +99,10 @@ __device__ inline void gather6(const FieldPair (*sf)[SFW * SFH], int li, int lj,
 // fields gathered from the tile's staged cell-centred values.  Shared by the
 // parity and fast kernels, so both produce bit-identical gp.  gmv returns the
 // 1/gamma of the move.
-__device__ inline void boris_push(const FieldPair (*sf)[SFW * SFH], int li, int lj, int i, int j, double delt, double c, bool unit_c, double fac1, double txxx, double fac2, double x, double y, double ux, double uy, double uz, double& nxp, double& nyp,
-                                  double& g3, double& g4, double& g5, double& gmv) {
+__device__ inline void boris_push(const FieldPair (*sf)[SFW * SFH], int li, int lj, int i, int j, double delt,
+                                  double c, bool unit_c, double fac1, double txxx, double fac2, double x, double y,
+                                  double ux, double uy, double uz, double& nxp, double& nyp, double& g3, double& g4,
+                                  double& g5, double& gmv) {
   double fl[6];
   gather6(sf, li, lj, i, j, x, y, fl);
   const double bpx = fl[0], bpy = fl[1], bpz = fl[2], epx = fl[3], epy = fl[4], epz = fl[5];
@@ -132,9 +134,9 @@ __device__ inline void boris_push(const FieldPair (*sf)[SFW * SFH], int li, int 
 // gather, u' = u + fac2 E + (fac1/gam) u x B, tau = fac1 B / c, the new gamma
 // from sigma and u'.tau, then the implicit rotation; the move uses that gamma.
 // Same arguments as boris_push (txxx unused).
-__device__ inline void vay_push(const FieldPair (*sf)[SFW * SFH], int li, int lj, int i, int j, double delt, double c, double fac1, double fac2, double x, double y, double ux,
-                                double uy, double uz, double& nxp, double& nyp, double& g3, double& g4, double& g5,
-                                double& gmv) {
+__device__ inline void vay_push(const FieldPair (*sf)[SFW * SFH], int li, int lj, int i, int j, double delt, double c,
+                                double fac1, double fac2, double x, double y, double ux, double uy, double uz,
+                                double& nxp, double& nyp, double& g3, double& g4, double& g5, double& gmv) {
   double fl[6];
   gather6(sf, li, lj, i, j, x, y, fl);
   const double bpx = fl[0], bpy = fl[1], bpz = fl[2], epx = fl[3], epy = fl[4], epz = fl[5];
