@@ -33,6 +33,7 @@ struct AdjState {
   double *lamA = nullptr, *lamA2 = nullptr, *lamB = nullptr;
   double *lamF = nullptr, *lamF2 = nullptr, *lamJ = nullptr, *lamT = nullptr;
   double* red = nullptr;
+  char* mem = nullptr;  // all of the above
   bool recorded = false, done = false;
 };
 
@@ -42,25 +43,14 @@ void adj_free(wpic_ctx* c) {
   AdjState* a = c->adj;
   if (!a) return;
   // after a replay A is read through the record's permutation of its last step:
-  // that buffer becomes the context's own, which goes in its place
-  for (auto& p : a->st_perm)
-    if (p && p == c->aperm) std::swap(p, c->permbuf);
-  auto fr = [](void* p) {
-    if (p) (void)hipFree(p);
-  };
-  for (auto p : a->ck_part) fr(p);
-  for (auto p : a->ck_uf) fr(p);
-  for (auto p : a->ck_df) fr(p);
-  for (auto p : a->ck_rows) fr(p);
-  for (auto p : a->ck_cumcnt) fr(p);
-  for (auto p : a->st_part) fr(p);
-  for (auto p : a->st_uf) fr(p);
-  for (auto p : a->st_rows) fr(p);
-  for (auto p : a->st_perm) fr(p);
-  for (auto p : a->st_cumcnt) fr(p);
-  for (void* p : {(void*)a->lamA, (void*)a->lamA2, (void*)a->lamB, (void*)a->lamF, (void*)a->lamF2, (void*)a->lamJ,
-                  (void*)a->lamT, (void*)a->red})
-    fr(p);
+  // it moves to the context's own buffer
+  for (int* p : a->st_perm)
+    if (p && p == c->aperm) {
+      (void)hipMemcpyAsync(c->permbuf, p, sizeof(int) * a->N, hipMemcpyDeviceToDevice, c->st);
+      c->aperm = c->permbuf;
+    }
+  (void)hipStreamSynchronize(c->st);
+  if (a->mem) (void)hipFree(a->mem);
   delete a;
   c->adj = nullptr;
 }
@@ -69,10 +59,40 @@ void adj_free(wpic_ctx* c) {
 
 namespace {
 
-template <class T>
-hipError_t dal(T** p, size_t n) {
-  *p = nullptr;
-  return hipMalloc((void**)p, (n ? n : 1) * sizeof(T));
+// hands out the parts of one allocation; without one it adds up what they need
+struct Carve {
+  char* base;
+  size_t used = 0;
+  template <class T>
+  void operator()(T*& p, size_t n) {
+    p = base ? reinterpret_cast<T*>(base + used) : nullptr;
+    used += (n * sizeof(T) + 255) & ~size_t(255);
+  }
+};
+
+// The recorded run is one allocation: a pass makes and frees it, and while the
+// driver still clears memory that was freed before, a free waits for it, 5.7 or
+// 7.5 ms at a time.  As 119 allocations a pass took, 55x52, 20 ppc, 23 steps, 23
+// ms or, then, 75; 256x256, 16 ppc, 40 steps 70 ms or 167 to 384.  As one it
+// takes 16, and 51 or, when passes free their 5.2 GB faster than the driver
+// clears them, 155 to 163.
+size_t carve_record(AdjState& a, char* base) {
+  Carve m{base};
+  for (auto& p : a.ck_part) m(p, PART_DOUBLES * a.N);
+  for (auto& p : a.ck_uf) m(p, 6 * a.pl);
+  for (auto& p : a.ck_df) m(p, 6 * a.pl);
+  for (auto& p : a.ck_rows) m(p, (size_t)2 * a.nr);
+  for (auto& p : a.ck_cumcnt) m(p, (size_t)a.ncc);
+  for (auto& p : a.st_part) m(p, PART_DOUBLES * a.N);
+  for (auto& p : a.st_uf) m(p, 6 * a.pl);
+  for (auto& p : a.st_perm) m(p, a.N);
+  for (auto& p : a.st_cumcnt) m(p, (size_t)a.ncc);
+  for (auto& p : a.st_rows) m(p, (size_t)2 * a.nr);
+  for (double** p : {&a.lamA, &a.lamA2, &a.lamB}) m(*p, 5 * a.N);
+  for (double** p : {&a.lamF, &a.lamF2, &a.lamT}) m(*p, 6 * a.nc);
+  m(a.lamJ, 3 * a.nc);
+  m(a.red, (size_t)256 * 3);
+  return m.used;
 }
 
 int copy_d(wpic_ctx* c, void* dst, const void* src, size_t bytes) {
@@ -121,40 +141,26 @@ int alloc_adj(wpic_ctx* c, int nsteps, int every) {
   a.ncc = a.nr * (g.nx + 1);
   a.pl = (size_t)g.fw * g.fh;
   a.nc = (size_t)g.nx * g.ny;
-  hipError_t e = hipSuccess;
   a.ck_part.assign(a.nseg, nullptr);
   a.ck_uf.assign(a.nseg, nullptr);
   a.ck_df.assign(a.nseg, nullptr);
   a.ck_rows.assign(a.nseg, nullptr);
   a.ck_cumcnt.assign(a.nseg, nullptr);
-  for (int s = 0; s < a.nseg && e == hipSuccess; s++) {
-    e = dal(&a.ck_part[s], PART_DOUBLES * a.N);
-    if (e == hipSuccess) e = dal(&a.ck_uf[s], 6 * a.pl);
-    if (e == hipSuccess) e = dal(&a.ck_df[s], 6 * a.pl);
-    if (e == hipSuccess) e = dal(&a.ck_rows[s], (size_t)2 * a.nr);
-    if (e == hipSuccess) e = dal(&a.ck_cumcnt[s], (size_t)a.ncc);
-  }
   const int K = every < nsteps ? every : nsteps;
   a.st_part.assign(K, nullptr);
   a.st_uf.assign(K, nullptr);
   a.st_perm.assign(K, nullptr);
   a.st_cumcnt.assign(K, nullptr);
   a.st_rows.assign(K + 1, nullptr);
-  for (int t = 0; t < K && e == hipSuccess; t++) {
-    e = dal(&a.st_part[t], PART_DOUBLES * a.N);
-    if (e == hipSuccess) e = dal(&a.st_uf[t], 6 * a.pl);
-    if (e == hipSuccess) e = dal(&a.st_perm[t], a.N);
+  hipError_t e = hipMalloc((void**)&a.mem, carve_record(a, nullptr));
+  if (e != hipSuccess) {
+    a.mem = nullptr;
+  } else {
+    carve_record(a, a.mem);
     // (as the context's own: every entry is a slot, whether a sort wrote it or not)
-    if (e == hipSuccess) e = hipMemsetAsync(a.st_perm[t], 0, sizeof(int) * a.N, c->st);
-    if (e == hipSuccess) e = dal(&a.st_cumcnt[t], (size_t)a.ncc);
+    for (int* p : a.st_perm)
+      if (e == hipSuccess) e = hipMemsetAsync(p, 0, sizeof(int) * a.N, c->st);
   }
-  for (int t = 0; t <= K && e == hipSuccess; t++) e = dal(&a.st_rows[t], (size_t)2 * a.nr);
-  for (double** p : {&a.lamA, &a.lamA2, &a.lamB})
-    if (e == hipSuccess) e = dal(p, 5 * a.N);
-  for (double** p : {&a.lamF, &a.lamF2, &a.lamT})
-    if (e == hipSuccess) e = dal(p, 6 * a.nc);
-  if (e == hipSuccess) e = dal(&a.lamJ, 3 * a.nc);
-  if (e == hipSuccess) e = dal(&a.red, (size_t)256 * 3);
   if (e != hipSuccess) {
     adj_free(c);
     return set_error(WPIC_EMEM, std::string("device memory for the recorded run: ") + hipGetErrorString(e));
