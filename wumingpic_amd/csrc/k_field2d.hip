@@ -254,52 +254,56 @@ __device__ inline void tell_host(const CgArgs& a, int l, int more, int ite) {
   if (l == 0) __hip_atomic_store(&a.poll->err, *a.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// Parity mode's scalars, from serial sums over the interior in (j, i) order.
-__device__ inline double serial_dot(const double* x, const double* y, int n) {
-  double s = 0.0;
-  for (int k = 0; k < n; k++) s = s + x[k] * y[k];
-  return s;
-}
+// Parity mode's scalars, from serial sums over the interior in (j, i) order,
+// one wave a component.
 
 // sum_g = |b|^2, eps = sqrt(sum_g)*err (field.f90:351-364), sumr_g; enter the
 // loop iff sqrt(sumr_g) > eps and sum_g > eps (:383-387)
-__global__ void k_cg_parity0(CgArgs a) {
+__global__ __launch_bounds__(64) void k_cg_parity0(CgArgs a) {
   const int l = blockIdx.x, n = a.g.nx * a.g.ny;
   const double *b = a.b + (size_t)l * n, *r = a.r + (size_t)l * n;
+  const double bb = serial_dot(b, b, n), rr = serial_dot(r, r, n);
+  if (threadIdx.x) return;
   CgScal& c = a.sc[l];
-  c.sum_g = serial_dot(b, b, n);
+  c.sum_g = bb;
   c.eps = sqrt(c.sum_g) * a.g.cg_err;
-  c.sumr_g = serial_dot(r, r, n);
+  c.sumr_g = rr;
   c.ite = 0;
   c.bv = 0.0;
   c.active = (sqrt(c.sumr_g) > c.eps) && (c.sum_g > c.eps);
 }
 
 // av = sumr_g / sum2_g (:409-415); sum_g = sqrt(sumr_g) (:426)
-__global__ void k_cg_parity_a(CgArgs a) {
+__global__ __launch_bounds__(64) void k_cg_parity_a(CgArgs a) {
   const int l = blockIdx.x, n = a.g.nx * a.g.ny;
   CgScal& c = a.sc[l];
   if (!c.active) return;
   const double *r = a.r + (size_t)l * n, *p = a.pnew + (size_t)l * n, *ap = a.ap + (size_t)l * n;
-  c.sumr_g = serial_dot(r, r, n);
-  c.sum2_g = serial_dot(p, ap, n);
+  const double rr = serial_dot(r, r, n), pap = serial_dot(p, ap, n);
+  if (threadIdx.x) return;
+  c.sumr_g = rr;
+  c.sum2_g = pap;
   c.av = c.sumr_g / c.sum2_g;
   c.ite = c.ite + 1;
   c.sum_g = sqrt(c.sumr_g);
 }
 
 // ite >= ite_max stops (:427-430); bv = sum1/sumr_g (:441-442); loop test
-__global__ void k_cg_parity_b(CgArgs a) {
+__global__ __launch_bounds__(64) void k_cg_parity_b(CgArgs a) {
   const int l = blockIdx.x, n = a.g.nx * a.g.ny;
   CgScal& c = a.sc[l];
   if (!c.active) return;
   if (c.ite >= 100) {
-    atomicOr(a.err, ERR_CG);
-    c.active = 0;
+    if (threadIdx.x == 0) {
+      atomicOr(a.err, ERR_CG);
+      c.active = 0;
+    }
     return;
   }
   const double* r = a.r + (size_t)l * n;
-  c.bv = serial_dot(r, r, n) / c.sumr_g;
+  const double rr = serial_dot(r, r, n);
+  if (threadIdx.x) return;
+  c.bv = rr / c.sumr_g;
   c.active = c.sum_g > c.eps;
 }
 
@@ -653,7 +657,7 @@ hipError_t launch_cg_init(wpic_ctx* c) {
   CgArgs a = cg_args(c);
   if (c->mode == WPIC_MODE_PARITY) {
     hipLaunchKernelGGL(k_cg_init<true>, dim3(a.nb0, 3), dim3(256), 0, c->st, a);
-    hipLaunchKernelGGL(k_cg_parity0, dim3(3), dim3(1), 0, c->st, a);
+    hipLaunchKernelGGL(k_cg_parity0, dim3(3), dim3(64), 0, c->st, a);
   } else {
     hipLaunchKernelGGL(k_cg_init<false>, dim3(a.nb0, 3), dim3(256), 0, c->st, a);
   }
@@ -664,7 +668,7 @@ hipError_t launch_cg_init(wpic_ctx* c) {
 // adjoint's transposed solves)
 hipError_t launch_cg_start(wpic_ctx* c) {
   CgArgs a = cg_args(c);
-  if (c->mode == WPIC_MODE_PARITY) hipLaunchKernelGGL(k_cg_parity0, dim3(3), dim3(1), 0, c->st, a);
+  if (c->mode == WPIC_MODE_PARITY) hipLaunchKernelGGL(k_cg_parity0, dim3(3), dim3(64), 0, c->st, a);
   return hipGetLastError();
 }
 
@@ -678,9 +682,9 @@ hipError_t launch_cg_iter(wpic_ctx* c, int it, bool poll) {
   const dim3 grid(a.nb, 3);
   if (c->mode == WPIC_MODE_PARITY) {
     hipLaunchKernelGGL(k_cg_a<true>, grid, dim3(256), 0, c->st, a);
-    hipLaunchKernelGGL(k_cg_parity_a, dim3(3), dim3(1), 0, c->st, a);
+    hipLaunchKernelGGL(k_cg_parity_a, dim3(3), dim3(64), 0, c->st, a);
     hipLaunchKernelGGL(k_cg_b<true>, grid, dim3(256), 0, c->st, a);
-    hipLaunchKernelGGL(k_cg_parity_b, dim3(3), dim3(1), 0, c->st, a);
+    hipLaunchKernelGGL(k_cg_parity_b, dim3(3), dim3(64), 0, c->st, a);
     return hipGetLastError();
   }
   a.sc = c->scal + 3 * (it & 1);

@@ -137,12 +137,6 @@ __device__ inline void decode3(const Grid3D& g, size_t q, int& i, int& j, int& k
   k = g.nzs + (int)(row / ny);
 }
 
-__device__ inline double serial_dot3(const double* x, const double* y, size_t n) {
-  double s = 0.0;
-  for (size_t k = 0; k < n; k++) s = s + x[k] * y[k];
-  return s;
-}
-
 // One block's sum of its threads' values, kept as partial sum `slot` of
 // component l.
 enum { S_RR = 0, S_PAP = 1, S_BB = 2 };  // r.r, p.ap, b.b
@@ -223,46 +217,54 @@ __global__ __launch_bounds__(256) void k_cg3_init(Cg3Args a) {
   }
 }
 
-// Parity mode's scalars, from serial sums: sum_g = |b|^2, eps =
+// Parity mode's scalars, from serial sums, one wave a component: sum_g = |b|^2, eps =
 // sqrt(sum_g)*err (field.f90:454-456), sumr_g, the loop's first test
-__global__ void k_cg3_parity0(Cg3Args a) {
+__global__ __launch_bounds__(64) void k_cg3_parity0(Cg3Args a) {
   const int l = blockIdx.x;
   const size_t n = (size_t)a.g.nx * a.g.ny * a.g.nz;
   const double *b = a.b + (size_t)l * n, *r = a.r + (size_t)l * n;
+  const double bb = serial_dot(b, b, n), rr = serial_dot(r, r, n);
+  if (threadIdx.x) return;
   CgScal& c = a.sc[l];
-  c.sum_g = serial_dot3(b, b, n);
+  c.sum_g = bb;
   c.eps = sqrt(c.sum_g) * a.g.cg_err;
-  c.sumr_g = serial_dot3(r, r, n);
+  c.sumr_g = rr;
   c.ite = 0;
   c.bv = 0.0;
   c.active = (sqrt(c.sumr_g) > c.eps) && (c.sum_g > c.eps);
 }
 
-__global__ void k_cg3_parity_a(Cg3Args a) {
+__global__ __launch_bounds__(64) void k_cg3_parity_a(Cg3Args a) {
   const int l = blockIdx.x;
   CgScal& c = a.sc[l];
   if (!c.active) return;
   const size_t n = (size_t)a.g.nx * a.g.ny * a.g.nz;
   const double *r = a.r + (size_t)l * n, *p = a.pnew + (size_t)l * n, *ap = a.ap + (size_t)l * n;
-  c.sumr_g = serial_dot3(r, r, n);
-  c.sum2_g = serial_dot3(p, ap, n);
+  const double rr = serial_dot(r, r, n), pap = serial_dot(p, ap, n);
+  if (threadIdx.x) return;
+  c.sumr_g = rr;
+  c.sum2_g = pap;
   c.av = c.sumr_g / c.sum2_g;
   c.ite = c.ite + 1;
   c.sum_g = sqrt(c.sumr_g);
 }
 
-__global__ void k_cg3_parity_b(Cg3Args a) {
+__global__ __launch_bounds__(64) void k_cg3_parity_b(Cg3Args a) {
   const int l = blockIdx.x;
   CgScal& c = a.sc[l];
   if (!c.active) return;
   if (c.ite >= 100) {
-    atomicOr(a.err, ERR_CG);
-    c.active = 0;
+    if (threadIdx.x == 0) {
+      atomicOr(a.err, ERR_CG);
+      c.active = 0;
+    }
     return;
   }
   const size_t n = (size_t)a.g.nx * a.g.ny * a.g.nz;
   const double* r = a.r + (size_t)l * n;
-  c.bv = serial_dot3(r, r, n) / c.sumr_g;
+  const double rr = serial_dot(r, r, n);
+  if (threadIdx.x) return;
+  c.bv = rr / c.sumr_g;
   c.active = c.sum_g > c.eps;
 }
 
@@ -581,7 +583,7 @@ hipError_t launch_cg_init3d(wpic_ctx3d* c) {
   Cg3Args a = cg3_args(c);
   if (c->mode == WPIC_MODE_PARITY) {
     hipLaunchKernelGGL(k_cg3_init<true>, dim3(a.nb0), dim3(256), 0, c->st, a);
-    hipLaunchKernelGGL(k_cg3_parity0, dim3(3), dim3(1), 0, c->st, a);
+    hipLaunchKernelGGL(k_cg3_parity0, dim3(3), dim3(64), 0, c->st, a);
   } else {
     hipLaunchKernelGGL(k_cg3_init<false>, dim3(a.nb0), dim3(256), 0, c->st, a);
   }
@@ -597,9 +599,9 @@ hipError_t launch_cg_iter3d(wpic_ctx3d* c, int it, bool poll) {
   const dim3 grid(a.nb, 3);
   if (c->mode == WPIC_MODE_PARITY) {
     hipLaunchKernelGGL(k_cg3_a<true>, grid, dim3(256), 0, c->st, a);
-    hipLaunchKernelGGL(k_cg3_parity_a, dim3(3), dim3(1), 0, c->st, a);
+    hipLaunchKernelGGL(k_cg3_parity_a, dim3(3), dim3(64), 0, c->st, a);
     hipLaunchKernelGGL(k_cg3_b<true>, grid, dim3(256), 0, c->st, a);
-    hipLaunchKernelGGL(k_cg3_parity_b, dim3(3), dim3(1), 0, c->st, a);
+    hipLaunchKernelGGL(k_cg3_parity_b, dim3(3), dim3(64), 0, c->st, a);
     return hipGetLastError();
   }
   a.sc = c->scal + 3 * (it & 1);
