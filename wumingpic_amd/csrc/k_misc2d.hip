@@ -668,11 +668,17 @@ __global__ __launch_bounds__(256) void k_energy(Grid2D g, Parts A, PartsM M, con
   for (int rw = blockIdx.x; rw < nrow; rw += gridDim.x) {
     const int s = rw / g.ny;
     const int base = rowbase[rw], n = np2[rw];
+#pragma unroll 4
     for (int k = threadIdx.x; k < n; k += 256) {
       const int p = ap ? ap[base + k] : base + k;
-      const double ux = MIXED ? (double)M.ux[p] : A.ux[p];
-      const double uy = MIXED ? (double)M.uy[p] : A.uy[p];
-      const double uz = MIXED ? (double)M.uz[p] : A.uz[p];
+      double ux, uy, uz;
+      if constexpr (MIXED) {
+        const RecM r = load_rec(M, p);
+        ux = r.ux, uy = r.uy, uz = r.uz;
+      } else {
+        const Rec r = load_rec(A, p);
+        ux = r.ux, uy = r.uy, uz = r.uz;
+      }
       const double u2 = ux * ux + uy * uy + uz * uz;
       const double gam = sqrt(1 + u2 / (g.c * g.c));
       kin = kin + g.r[s] * (gam - 1);

@@ -341,11 +341,17 @@ __global__ __launch_bounds__(256) void k_energy3(Grid3D g, Parts3 A, PartsM3 M, 
     const int s = rw / g.ncol;
     if (sp >= 0 && s != sp) continue;  // one species' kinetic energy
     const int base = colbase[rw], n = np2[rw];
+#pragma unroll 4
     for (int q = threadIdx.x; q < n; q += 256) {
       const int p = ap ? ap[base + q] : base + q;
-      const double ux = MIXED ? (double)M.ux[p] : A.ux[p];
-      const double uy = MIXED ? (double)M.uy[p] : A.uy[p];
-      const double uz = MIXED ? (double)M.uz[p] : A.uz[p];
+      double ux, uy, uz;
+      if constexpr (MIXED) {
+        const RecM3 r = load_rec(M, p);
+        ux = r.ux, uy = r.uy, uz = r.uz;
+      } else {
+        const Rec3 r = load_rec(A, p);
+        ux = r.ux, uy = r.uy, uz = r.uz;
+      }
       const double u2 = ux * ux + uy * uy + uz * uz;
       kin = kin + g.r[s] * (sqrt(1 + u2 / (g.c * g.c)) - 1);
     }

@@ -333,8 +333,9 @@ __device__ inline double wave_sum(double v) {
 // active wave, the same bits in every lane: the lanes read and multiply 64
 // elements at a time, the next 256 on their way, and the products are added one
 // after another.  (Past the end they are +0, which changes no sum that began as
-// +0.)  Read by the adding lane itself, an element costs its share of a memory wait: 65 ns
-// where this takes 10 (a parity step at 256x256, 16 ppc: 89 -> 15 ms).
+// +0.)  Read by the adding lane itself, an element costs its share of a memory
+// wait: 65 ns where this takes 10 (a parity step at 256x256, 16 ppc: 89 -> 15
+// ms).
 __device__ inline double serial_dot(const double* x, const double* y, size_t n) {
   constexpr int U = 4;
   const size_t lane = threadIdx.x & 63;
