@@ -321,9 +321,12 @@ __global__ __launch_bounds__(NT) void k_mom_parity(MomArgs a, int aligned) {
       pb = cr[lo - g.nxgs];
       pe = cr[hi + 1 - g.nxgs];
     }
+    Rec next{};  // (the next record on its way while one is added)
+    if (pb < pe) next = load_rec(a.B, base + pb);
     for (int p = pb; p < pe; p++) {
-      const int pi = base + p;
-      const double x = a.B.x[pi], y = a.B.y[pi];
+      const Rec r = next;
+      if (p + 1 < pe) next = load_rec(a.B, base + p + 1);
+      const double x = r.x, y = r.y;
       const int ih = (int)(x * g.d_delx - 0.5), jh = (int)(y * g.d_delx - 0.5);
       if (ih < g.nxgs - 1 || ih > g.nxge || jh < j - 1 || jh > j) {
         atomicOr(a.err, ERR_DOMAIN);
@@ -344,7 +347,7 @@ __global__ __launch_bounds__(NT) void k_mom_parity(MomArgs a, int aligned) {
       else
         continue;
       MomTerms t;
-      t.set(a.B.ux[pi], a.B.uy[pi], a.B.uz[pi], g.c);
+      t.set(r.ux, r.uy, r.uz, g.c);
 #pragma unroll
       for (int k = 0; k < 7; k++) acc[k] = acc[k] + t.term(k, wx, wy);
     }

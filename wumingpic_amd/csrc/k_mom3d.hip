@@ -103,17 +103,11 @@ __global__ __launch_bounds__(p3::NT) void k_mom_accl3d(Mom3Args a) {
       const int pend = base + cr[i - g.nxgs + 1];
       for (int pi = base + cr[i - g.nxgs] + lg; pi < pend; pi += G) {
         const int ia = a.ap ? a.ap[pi] : pi;
-        const double x = a.A.x[ia], y = a.A.y[ia], z = a.A.z[ia];
+        const Rec3 p = load_rec(a.A, ia);
         double nxp, nyp, nzp, g4, g5, g6;
-        boris_push3(sf, so, i, j, k, hdelt, g.c, a.fac1[s], a.txxx[s], a.fac2[s], x, y, z, a.A.ux[ia],
-                    a.A.uy[ia], a.A.uz[ia], nxp, nyp, nzp, g4, g5, g6);
-        a.B.x[pi] = x;
-        a.B.y[pi] = y;
-        a.B.z[pi] = z;
-        a.B.ux[pi] = g4;
-        a.B.uy[pi] = g5;
-        a.B.uz[pi] = g6;
-        a.B.id[pi] = a.A.id[ia];
+        boris_push3(sf, so, i, j, k, hdelt, g.c, a.fac1[s], a.txxx[s], a.fac2[s], p.x, p.y, p.z, p.ux, p.uy, p.uz, nxp,
+                    nyp, nzp, g4, g5, g6);
+        store_rec(a.B, pi, Rec3{p.x, p.y, p.z, g4, g5, g6, p.id});
       }
     }
   }
@@ -183,20 +177,14 @@ __global__ __launch_bounds__(p3::NT) void k_mom3d_tile(Mom3Args a) {
       for (int pi = base + cr[i - g.nxgs] + lg; pi < pe; pi += GM) {
         double x, y, z, ux, uy, uz;
         if constexpr (KICK) {
-          const int ia = a.ap ? a.ap[pi] : pi;
-          x = a.A.x[ia];
-          y = a.A.y[ia];
-          z = a.A.z[ia];
+          const Rec3 p = load_rec(a.A, a.ap ? a.ap[pi] : pi);
+          x = p.x, y = p.y, z = p.z;
           double nxp, nyp, nzp;
-          boris_push3(sf, so, i, j, k, hdelt, c, a.fac1[s], a.txxx[s], a.fac2[s], x, y, z, a.A.ux[ia],
-                      a.A.uy[ia], a.A.uz[ia], nxp, nyp, nzp, ux, uy, uz);
+          boris_push3(sf, so, i, j, k, hdelt, c, a.fac1[s], a.txxx[s], a.fac2[s], x, y, z, p.ux, p.uy, p.uz, nxp, nyp,
+                      nzp, ux, uy, uz);
         } else {
-          x = a.B.x[pi];
-          y = a.B.y[pi];
-          z = a.B.z[pi];
-          ux = a.B.ux[pi];
-          uy = a.B.uy[pi];
-          uz = a.B.uz[pi];
+          const Rec3 p = load_rec(a.B, pi);
+          x = p.x, y = p.y, z = p.z, ux = p.ux, uy = p.uy, uz = p.uz;
         }
         Cic3 w;
         w.set(g, x, y, z);
@@ -306,10 +294,13 @@ __global__ __launch_bounds__(p3::NT) void k_mom3d_parity(Mom3Args a, int aligned
         pb = cr[max(g.nxgs, n - 1) - g.nxgs];
         pe = cr[min(g.nxge, n + 1) + 1 - g.nxgs];
       }
+      Rec3 next{};  // (the next record on its way while one is added)
+      if (pb < pe) next = load_rec(a.B, base + pb);
       for (int p = pb; p < pe; p++) {
-        const int pi = base + p;
+        const Rec3 r = next;
+        if (p + 1 < pe) next = load_rec(a.B, base + p + 1);
         Cic3 w;
-        w.set(g, a.B.x[pi], a.B.y[pi], a.B.z[pi]);
+        w.set(g, r.x, r.y, r.z);
         if (!w.ok(g, j, k)) {
           atomicOr(a.err, ERR_DOMAIN);
           continue;
@@ -317,7 +308,7 @@ __global__ __launch_bounds__(p3::NT) void k_mom3d_parity(Mom3Args a, int aligned
         const int ox = n - w.ih, oy = m - w.jh, oz = l - w.kh;
         if (ox < 0 || ox > 1 || oy < 0 || oy > 1 || oz < 0 || oz > 1) continue;
         Mom3Terms tm;
-        tm.set(a.B.ux[pi], a.B.uy[pi], a.B.uz[pi], g.c);
+        tm.set(r.ux, r.uy, r.uz, g.c);
         const double wx = w.w(0, ox), wy = w.w(1, oy), wz = w.w(2, oz);
 #pragma unroll
         for (int q = 0; q < 7; q++) acc[q] = acc[q] + tm.term(q, wx, wy, wz);
