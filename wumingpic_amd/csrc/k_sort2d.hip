@@ -41,18 +41,17 @@ __global__ __launch_bounds__(SB) void k_wrapx(SortArgs a, int inj) {
   const int base = a.rowbaseB[rw], n = a.np2B[rw];
   for (int k = threadIdx.x; k < n; k += SB) {
     const int p = base + k;
-    double x = a.B.x[p];
+    const Rec r = load_rec(a.B, p);
     if (walls(g)) {
-      double ux = a.B.ux[p], uy = a.B.uy[p], uz = a.B.uz[p];
+      Rec q = r;
       if (inj)
-        reflect_x<WPIC_BC_SHOCK, true>(g, x, ux, uy, uz);
+        reflect_x<WPIC_BC_SHOCK, true>(g, q.x, q.ux, q.uy, q.uz);
       else
-        reflect_x<WPIC_BC_SHOCK, false>(g, x, ux, uy, uz);
-      a.B.x[p] = x;
-      a.B.ux[p] = ux;
-      a.B.uy[p] = uy;
-      a.B.uz[p] = uz;
+        reflect_x<WPIC_BC_SHOCK, false>(g, q.x, q.ux, q.uy, q.uz);
+      // (only a reflected record is written: every reflection turns uy's sign)
+      if (__double_as_longlong(q.uy) != __double_as_longlong(r.uy)) store_rec(a.B, p, q);
     } else {
+      const double x = r.x;
       const int ipos = cell_of(x);
       if (ipos < g.nxgs)
         a.B.x[p] = rd_add(x, g.spanx);
