@@ -316,15 +316,12 @@ __global__ void k_ic_weibel(IcWeibelArgs a) {
   const long long d = s * g.ncap + k;
   const int j = g.nys + r;
   const int np2 = (int)rowlen;
-  a.A.x[d] = (g.nxgs + (g.nxge - g.nxgs + 1) * (ii - 0.5) / np2) * g.delx;
-  a.A.y[d] = (j + u01(rkey(a.seed, 3, r, 0, ii))) * g.delx;
+  const double x = (g.nxgs + (g.nxge - g.nxgs + 1) * (ii - 0.5) / np2) * g.delx;
+  const double y = (j + u01(rkey(a.seed, 3, r, 0, ii))) * g.delx;
   double n0, n1, n2, n3;
   normal2(rkey(a.seed, 20 + 4 * s, r, 0, ii), rkey(a.seed, 21 + 4 * s, r, 0, ii), n0, n1);
   normal2(rkey(a.seed, 22 + 4 * s, r, 0, ii), rkey(a.seed, 23 + 4 * s, r, 0, ii), n2, n3);
-  a.A.ux[d] = a.sd[s] * n0;
-  a.A.uy[d] = a.sd[s] * n1;
-  a.A.uz[d] = a.t_ani * a.sd[s] * n2;
-  a.A.id[d] = (uint64_t)(-(k + 1));
+  store_rec(a.A, d, Rec{x, y, a.sd[s] * n0, a.sd[s] * n1, a.t_ani * a.sd[s] * n2, (uint64_t)(-(k + 1))});
 }
 
 // 2d/proj/reconnection/app.f90:373-452: the Harris sheet with the X-point
@@ -373,12 +370,7 @@ __global__ void k_ic_harris(IcHarrisArgs a) {
     normal2(rkey(a.seed, 30 + 4 * s, r, 0, ii), rkey(a.seed, 31 + 4 * s, r, 0, ii), n0, n1);
     normal2(rkey(a.seed, 32 + 4 * s, r, 0, ii), rkey(a.seed, 33 + 4 * s, r, 0, ii), n2, n3);
     const long long d = s * g.ncap + t;
-    a.B.x[d] = x;
-    a.B.y[d] = y;
-    a.B.ux[d] = a.sd[s] * n0;
-    a.B.uy[d] = a.sd[s] * n1;
-    a.B.uz[d] = a.sd[s] * n2 + a.f[s] * jz / den;
-    a.B.id[d] = (uint64_t)(-(t + 1));
+    store_rec(a.B, d, Rec{x, y, a.sd[s] * n0, a.sd[s] * n1, a.sd[s] * n2 + a.f[s] * jz / den, (uint64_t)(-(t + 1))});
   }
 }
 
@@ -475,15 +467,10 @@ __global__ void k_ic_shock(IcShockArgs a) {
     const double gamp = sqrt(1 + (ux * ux + uy * uy + uz * uz) / (c * c));
     ux = gam1 * (ux + v1 * gamp);
     const long long d = s * g.ncap + t;
-    a.B.x[d] = x;
-    a.B.y[d] = y;
-    a.B.ux[d] = ux;
-    a.B.uy[d] = uy;
-    a.B.uz[d] = uz;
     // set_particle_ids (app.f90:500-524): the id is -pid, made positive
     // (a tracer written by io__orb) for x in [xrs, xre] = [450, 500]
     const bool tracer = x >= 450.0 && x <= 500.0;
-    a.B.id[d] = tracer ? (uint64_t)(t + 1) : (uint64_t)(-(t + 1));
+    store_rec(a.B, d, Rec{x, y, ux, uy, uz, tracer ? (uint64_t)(t + 1) : (uint64_t)(-(t + 1))});
   }
 }
 
@@ -581,12 +568,7 @@ __global__ __launch_bounds__(256) void k_inject(InjArgs a) {
     const double gam1 = 1 / sqrt(1 - (v1 / c) * (v1 / c));
     const double gamp = sqrt(1 + (ux * ux + uy * uy + uz * uz) / (c * c));
     ux = gam1 * (ux + v1 * gamp);
-    a.B.x[d] = x;
-    a.B.y[d] = y;
-    a.B.ux[d] = ux;
-    a.B.uy[d] = uy;
-    a.B.uz[d] = uz;
-    a.B.id[d] = (uint64_t)(-((long long)m + a.idoff[rw]));
+    store_rec(a.B, d, Rec{x, y, ux, uy, uz, (uint64_t)(-((long long)m + a.idoff[rw]))});
   }
   if (threadIdx.x == 0 && nl > 0) {
     int* cr = a.cumcnt + (size_t)rw * (g.nx + 1);
@@ -668,7 +650,7 @@ __global__ __launch_bounds__(256) void k_energy(Grid2D g, Parts A, PartsM M, con
   for (int rw = blockIdx.x; rw < nrow; rw += gridDim.x) {
     const int s = rw / g.ny;
     const int base = rowbase[rw], n = np2[rw];
-#pragma unroll 4
+#pragma unroll 8
     for (int k = threadIdx.x; k < n; k += 256) {
       const int p = ap ? ap[base + k] : base + k;
       double ux, uy, uz;

@@ -290,16 +290,13 @@ __global__ void k_ic_weibel3(IcW3Args a) {
   const long long d = s * g.ncap + q;
   const int j = g.nys + col % g.ny, k = g.nzs + col / g.ny;
   const int np2 = (int)colen;
-  a.A.x[d] = (g.nxgs + (g.nxge - g.nxgs + 1) * (ii - 5e-1) / np2) * g.delx;
-  a.A.y[d] = (j + u01_3(rkey3(a.seed, 4, col, 0, ii))) * g.delx;
-  a.A.z[d] = (k + u01_3(rkey3(a.seed, 5, col, 0, ii))) * g.delx;
+  const double x = (g.nxgs + (g.nxge - g.nxgs + 1) * (ii - 5e-1) / np2) * g.delx;
+  const double y = (j + u01_3(rkey3(a.seed, 4, col, 0, ii))) * g.delx;
+  const double z = (k + u01_3(rkey3(a.seed, 5, col, 0, ii))) * g.delx;
   double n0, n1, n2, n3;
   normal2_3(rkey3(a.seed, 20 + 4 * s, col, 0, ii), rkey3(a.seed, 21 + 4 * s, col, 0, ii), n0, n1);
   normal2_3(rkey3(a.seed, 22 + 4 * s, col, 0, ii), rkey3(a.seed, 23 + 4 * s, col, 0, ii), n2, n3);
-  a.A.ux[d] = a.sd[s] * n0;
-  a.A.uy[d] = a.sd[s] * n1;
-  a.A.uz[d] = a.t_ani * a.sd[s] * n2;
-  a.A.id[d] = (uint64_t)(-(q + 1));
+  store_rec(a.A, d, Rec3{x, y, z, a.sd[s] * n0, a.sd[s] * n1, a.t_ani * a.sd[s] * n2, (uint64_t)(-(q + 1))});
 }
 
 hipError_t launch_ic_weibel3d(wpic_ctx3d* c, unsigned long long seed, int n0, const double* sd, double t_ani) {
