@@ -75,7 +75,7 @@ struct Carve {
 // 7.5 ms at a time.  As 119 allocations a pass took, 55x52, 20 ppc, 23 steps, 23
 // ms or, then, 75; 256x256, 16 ppc, 40 steps 70 ms or 167 to 384.  As one it
 // takes 16, and 51 or, when passes free their 5.2 GB faster than the driver
-// clears them, 155 to 163.
+// clears them, 155 to 163 (once 302).
 size_t carve_record(AdjState& a, char* base) {
   Carve m{base};
   for (auto& p : a.ck_part) m(p, PART_DOUBLES * a.N);
