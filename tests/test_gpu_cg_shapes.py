@@ -92,3 +92,33 @@ def test_field_solve_with_more_work_units_than_blocks(n):
             got = sim.download_dfield()
             assert np.abs(got - o.df).max() <= 1e-11 * np.abs(o.df).max()
             assert np.abs(sim.download_fields() - uf).max() <= 1e-11 * np.abs(uf).max()
+
+
+@pytest.mark.parametrize("n", [(4, 4), (8, 8), (5, 13), (15, 17), (16, 16), (4, 65), (37, 31), (4, 4, 4), (5, 5, 5),
+                               (4, 8, 8), (7, 9, 11)], ids=lambda n: "x".join(map(str, n)))
+def test_parity_solve_is_bit_exact(n):
+    """the parity mode's serial sums, taken 256 elements at a time: fewer than 64, whole chunks, remainders"""
+    from wumingpic_amd import MODE_PARITY
+    from wumingpic_amd.pic2d import Pic2D
+    from wumingpic_amd.pic3d import Pic3D
+    rng = np.random.default_rng(6)
+    q, r = S.weibel_consts(2)
+    if len(n) == 2:
+        p = po.make_params(*n, np_cap=8 * n[0], delt=0.5, q=q, r=r)
+        o, (up, cc, np2) = po.Oracle2D(p), S.sorted_particles(p, 2, rng)
+        uf = np.asfortranarray(S.periodic_fill_fields(p, S.random_fields(p, rng, scale=0.02)))
+    else:
+        p = po.make_params3d(*n, np_cap=8 * n[0], delt=0.5, q=q, r=r)
+        o, (up, cc, np2) = po.Oracle3D(p), S3.sorted_particles3d(p, 2, rng)
+        uf = S3.periodic_fill_fields3d(p, S3.random_fields3d(p, rng, scale=0.02))
+    gp = np.zeros_like(up, order="F")
+    o.particle_solv(gp, up, uf, cc)
+    print(n, flush=True)
+    with (Pic2D if len(n) == 2 else Pic3D)(*n, list(q), list(r), delt=0.5, mode=MODE_PARITY,
+                                           capacity=int(np2.sum())) as sim:
+        sim.upload_up(up, np2, cc)
+        sim.upload_fields(uf)
+        sim.particle_solv()
+        assert tuple(sim.field_fdtd_i()) == tuple(o.field_fdtd_i(uf, up, gp, cc))
+        assert np.array_equal(sim.download_dfield().view(np.int64), o.df.copy(order="F").view(np.int64))
+        assert np.array_equal(sim.download_fields().view(np.int64), uf.view(np.int64))
